@@ -134,6 +134,15 @@ struct FusedArgs {
     int hstride, estride;
 };
 
+// Workgroup barrier with its own wait for this wave's LDS accesses. hipcc (ROCm 7.2, gfx950)
+// leaves out the wait of a __syncthreads() that heads a loop whose back edge ends in LDS
+// stores: the wave then arrives with its last stores still under way, and another wave's
+// read-modify-write of the same word loses one of the two sums.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0), the other counters untouched
+    __syncthreads();
+}
+
 __device__ __forceinline__ int color_of(const int32_t *__restrict__ cp, int i) {
     int c = 0;
     while (cp[c + 1] <= i) ++c;
@@ -289,7 +298,7 @@ __global__ __launch_bounds__(512) void k_cd_fused(FusedArgs a) {
         const int clo = color_of(cp, base);
         const int chi = color_of(cp, min(base + B, ne) - 1);
         for (int c = clo; c <= chi; ++c) {
-            __syncthreads();
+            lds_barrier();
             if (mycol == c) {
 #pragma unroll
                 for (int q2 = 0; q2 < NEN; ++q2)

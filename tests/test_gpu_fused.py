@@ -170,3 +170,22 @@ def test_fp32_element_variant(tile_nodes):
     assert ig["elem_precision"] == 2 and rel_l2(hg, refg["U"]) < 1e-4
     with pytest.raises(Exception):
         DeviceModel(block_model(4, 4, 3, transform=rotation())[0], elem_precision=2)
+
+
+def test_color_phase_kernel_repeats_exactly():
+    """Eight 400 x 200 layers stepped by the color-phase kernel three times: bitwise the same (a
+    wave that reached a color's barrier with its last LDS store under way lost a corner force about once
+    in a million tile steps; these runs are three million)."""
+    from svl_amd import batch
+    parts = [W.realization2d(400, 200, 77 + i, nt=601, x0=408.0 * i) for i in range(8)]
+    m, node_ptr, free_ptr = batch.union([p[0] for p in parts])
+    dm = DeviceModel(m, variant=1)
+    it = batch.BatchedCentralDifference(dm, [p[1] for p in parts], node_ptr, free_ptr)
+    runs = []
+    for _ in range(3):
+        it.Initialize()
+        it.advance(1, 600)
+        runs.append(it.GetDisplacements())
+    dm.close()
+    assert np.isfinite(runs[0]).all() and np.abs(runs[0]).max() > 0.0
+    assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
