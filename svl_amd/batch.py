@@ -138,14 +138,19 @@ class BatchedCentralDifference:
                    "svlg_cd_get_state")
         return U, V, A
 
+    def _field(self, i: int, part: int | None) -> np.ndarray:
+        """One of U, V, A (the library leaves out the fields whose pointer is null)."""
+        out = np.zeros(self.mesh.nfree)
+        p = [None, None, None]
+        p[i] = capi.fptr(out)
+        capi.check(capi.lib().svlg_cd_get_state(self.mesh.h, *p), "svlg_cd_get_state")
+        return out if part is None else out[self.free_ptr[part]:self.free_ptr[part + 1]]
+
     def GetDisplacements(self, part: int | None = None) -> np.ndarray:
-        U = self._state()[0]
-        return U if part is None else U[self.free_ptr[part]:self.free_ptr[part + 1]]
+        return self._field(0, part)
 
     def GetVelocities(self, part: int | None = None) -> np.ndarray:
-        V = self._state()[1]
-        return V if part is None else V[self.free_ptr[part]:self.free_ptr[part + 1]]
+        return self._field(1, part)
 
     def GetAccelerations(self, part: int | None = None) -> np.ndarray:
-        A = self._state()[2]
-        return A if part is None else A[self.free_ptr[part]:self.free_ptr[part + 1]]
+        return self._field(2, part)

@@ -150,6 +150,7 @@ struct Model {
     DevBuf<double> kinv;              // 1 / keff (0 where keff = 0: the restrained DOFs)
     DevBuf<uint16_t> egid;            // [nelem] geometry-table entry per element (table paths)
     DevBuf<double> hist;              // recorder buffer
+    DevBuf<double> snap;              // fields in free order on their way to the caller (svlg_*_get_state)
     DevBuf<int32_t> rec;              // recorded node-DOFs
     // Independent meshes advanced together (one model whose parts share no node): each part
     // keeps its own time step.

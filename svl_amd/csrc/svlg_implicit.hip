@@ -1186,16 +1186,19 @@ int svlg_nm_get_state(svlg_model *h, double *U, double *V, double *A) {
     SVLG_CHECK(h, "null model");
     Model &m = h->m;
     SVLG_CHECK(m.nm_ready, "svlg_nm_init has not been called");
-    DevBuf<double> tmp;
-    SVLG_HIP(tmp.alloc(std::max(m.nfree, 1)));
     double *outs[3] = {U, V, A};
     const double *src[3] = {m.nU.p, m.nV.p, m.nA.p};
+    const size_t nf = std::max(m.nfree, 1);
+    if (m.snap.n < 3 * nf) {
+        SVLG_HIP(m.snap.alloc(3 * nf));
+        SVLG_HIP(hipMemsetAsync(m.snap.p, 0, sizeof(double) * m.snap.n, m.stream));
+    }
     for (int i = 0; i < 3; ++i) {
         if (!outs[i]) continue;
-        if (int rc = gather_free(m, src[i], tmp.p)) return rc;
-        SVLG_HIP(hipMemcpyAsync(outs[i], tmp.p, sizeof(double) * m.nfree, hipMemcpyDeviceToHost, m.stream));
-        SVLG_HIP(hipStreamSynchronize(m.stream));
+        if (int rc = gather_free(m, src[i], m.snap.p + i * nf)) return rc;
+        SVLG_HIP(hipMemcpyAsync(outs[i], m.snap.p + i * nf, sizeof(double) * m.nfree, hipMemcpyDeviceToHost, m.stream));
     }
+    SVLG_HIP(hipStreamSynchronize(m.stream));
     return 0;
 }
 

@@ -172,8 +172,16 @@ class PmlNewmark:
                    "svlg_pml_get_state")
         return U, V, A
 
+    def _field(self, i: int):
+        """One of U, V, A (the library leaves out the fields whose pointer is null)."""
+        out = np.zeros(self.nfree)
+        p = [None, None, None]
+        p[i] = capi.fptr(out)
+        capi.check(capi.lib().svlg_pml_get_state(self.h, *p), "svlg_pml_get_state")
+        return out
+
     def GetDisplacements(self):
-        return self.state()[0]
+        return self._field(0)
 
     def set_graph(self, on: bool):
         """Replay the MINRES iterations from a captured hipGraph (default) or launch them eagerly."""
@@ -186,10 +194,10 @@ class PmlNewmark:
         return out
 
     def GetVelocities(self):
-        return self.state()[1]
+        return self._field(1)
 
     def GetAccelerations(self):
-        return self.state()[2]
+        return self._field(2)
 
 
 def soil_column(n_reg: int, n_pml: int, load_series, E=5e7, nu=0.25, rho=2000.0, m=2.0, L=None, R=1e-5,
