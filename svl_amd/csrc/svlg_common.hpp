@@ -80,6 +80,17 @@ struct TileSet {
     DevBuf<double> lampad, mupad;
 };
 
+// Deep-halo plan of the multi-step explicit kernel (device copy of HostMulti, svlg_tiles.hpp).
+struct MultiSet {
+    int depth = 0;                           // 0: not built, one step per launch
+    int ntiles = 0, ns = 0, ne = 0, nu = 0, block = 0;
+    size_t lds_bytes = 0;
+    DevBuf<int32_t> cnt, node;
+    DevBuf<uint16_t> econn, ncor, egeo;
+    DevBuf<double> elam, emu;
+    DevBuf<double> U[3];                     // output buffers, exchanged with the state's ring
+};
+
 struct Model {
     int ndim = 0, nen = 0, nnodes = 0, nelem = 0, nfree = 0, ndofn = 0;  // ndofn = nnodes*ndim
     int device = 0;                   // HIP device current at creation (the model's memory lives there)
@@ -152,6 +163,21 @@ struct Model {
     DevBuf<double> hist;              // recorder buffer
     DevBuf<double> snap;              // fields in free order on their way to the caller (svlg_*_get_state)
     DevBuf<int32_t> rec;              // recorded node-DOFs
+    // Recording inside the step kernels: the history column of every node-DOF (-1: none) and
+    // the tiles that own a recorded DOF.
+    DevBuf<int32_t> recmap, recdup;
+    DevBuf<int32_t> rectile;
+    std::vector<int32_t> h_f2n;       // node-DOF position of every free DOF (made on first use)
+    // Multi-step plan: made by the first CentralDifference initialisation of a model that can use it.
+    MultiSet multi;
+    bool auto_variant = false;        // the kernels were chosen by the library, not by the caller
+    bool multi_tried = false;
+    bool corner_unique = false;       // every (node, corner position) pair belongs to at most one element
+    std::vector<int32_t> h_conn;      // [nelem*nen] connectivity in device numbering
+    std::vector<int32_t> h_own_ptr;   // [ntiles+1]
+    std::vector<uint8_t> h_special;   // [nnodes] device order: nodes that take the general update
+    std::vector<double> h_lam, h_mu;  // [nelem] Lame constants
+    std::vector<uint16_t> h_gid;      // [nelem] geometry-table entry
     // Independent meshes advanced together (one model whose parts share no node): each part
     // keeps its own time step.
     std::vector<double> h_dt_dof;     // [ndofn] time step of every DOF (empty: m.dt everywhere)

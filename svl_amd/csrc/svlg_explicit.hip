@@ -14,18 +14,20 @@
 // U_{k-2}) can be formed on demand with SVL's expressions.
 #include <algorithm>
 #include <cstring>
+#include <numeric>
 
 #include "svlg_common.hpp"
 #include "svlg_drm.hpp"
 #include "svlg_support.hpp"
 #include "svlg_elem.hpp"
 #include "svlg_mfma.hpp"
+#include "svlg_tiles.hpp"
 
 namespace svlg {
 
 int launch_fint_colored(Model &m, const double *U, double ftol, double *F);
 int gather_free(Model &m, const double *dnode, double *dfree);
-int record_positions(const Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos);
+int record_positions(Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos);
 int scatter_free(Model &m, const double *dfree, double *dnode);
 
 // keff = M/dt^2 + C/2dt, kforce = M/dt^2 - C/2dt per DOF (CentralDifference.cpp:64-70); dtv
@@ -109,6 +111,43 @@ __global__ void k_record(int nrec, const int32_t *__restrict__ rec, const double
     if (r < nrec) out[r] = U[rec[r]];
 }
 
+// Recording inside the step kernels (map null: none): the owner of a recorded DOF writes its new
+// value into the history row of the step. A launch of its own per step cost 3 us of latency beside
+// steps of 3 to 5 us on small models.
+struct RecRef {
+    const int32_t *map;     // [ndofn] column or -1
+    const int32_t *tile;    // [ntiles] 1: the tile owns a recorded DOF
+    double *hist;           // row of the launch's first step
+    int nrec;
+};
+
+// Data that no kernel in flight writes: constant address space, so that a uniform index is a scalar
+// load whose wait joins the tile bounds' (as ordinary memory it is a vector load with a full wait).
+using const_i32 = const __attribute__((address_space(4))) int32_t;
+
+__device__ __forceinline__ bool tile_records(const RecRef &r, int tile) {
+    return r.map && ((const_i32 *)r.tile)[tile] != 0;
+}
+
+__device__ __forceinline__ void record_dof(const RecRef &r, size_t g, int row, double u) {
+    const int c = r.map[g];
+    if (c >= 0) r.hist[size_t(row) * r.nrec + c] = u;
+}
+
+__global__ void k_rec_map(int nrec, const int32_t *__restrict__ rec, int on, int32_t *__restrict__ map) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < nrec && rec[r] >= 0) map[rec[r]] = on ? r : -1;
+}
+
+// Columns that repeat an earlier column's DOF: dup holds (column, earlier column) pairs.
+__global__ void k_rec_dup(int ndup, const int32_t *__restrict__ dup, int nsteps, int nrec,
+                          double *__restrict__ hist) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ndup * nsteps) return;
+    double *row = hist + size_t(i / ndup) * nrec;
+    row[dup[2 * (i % ndup)]] = row[dup[2 * (i % ndup) + 1]];
+}
+
 // U, V, A of the free DOFs in free order (CentralDifference::ComputeNewStep, :141-145, with U =
 // U_{k-1}, Up = U_{k-2}, dU = U_k - U_{k-1}); null outputs are left out. Bandwidth-bound: one
 // pass over the three vectors, then one copy per field that the caller asks for. The host loop
@@ -152,6 +191,7 @@ struct FusedArgs {
     const uint16_t *lcpad, *geopad;
     const double *lampad, *mupad;
     int hstride, estride;
+    RecRef rec;
 };
 
 // Workgroup barrier with its own wait for this wave's LDS accesses. hipcc (ROCm 7.2, gfx950)
@@ -334,6 +374,7 @@ __global__ __launch_bounds__(512) void k_cd_fused(FusedArgs a) {
     }
     // Owned DOFs: load U_{k-2} and keff with NB loads in flight, then update.
     const int npl = a.nplain[tile];
+    const bool has_rec = tile_records(a.rec, tile);
     const size_t g0 = size_t(o0) * DIM;
     for (int base = 0; base < nU; base += NB * B) {
         double up[NB], kd[NB];
@@ -350,11 +391,10 @@ __global__ __launch_bounds__(512) void k_cd_fused(FusedArgs a) {
             if (i >= nU) continue;
             const int sl = i / DIM;
             const double u = sU[i], fi = sF[i];
+            double un = 0.0;
             if (sl < npl) {
-                a.Unext[g0 + i] = u + ((0.0 - fi) + kd[k] * (u - up[k])) / kd[k];
-            } else if (kd[k] == 0.0) {
-                a.Unext[g0 + i] = 0.0;
-            } else {
+                un = u + ((0.0 - fi) + kd[k] * (u - up[k])) / kd[k];
+            } else if (kd[k] != 0.0) {
                 const int c = i - sl * DIM, node = o0 + sl;
                 double fe = 0.0;
                 for (int q2 = a.nl_ptr[node]; q2 < a.nl_ptr[node + 1]; ++q2) {
@@ -365,8 +405,10 @@ __global__ __launch_bounds__(512) void k_cd_fused(FusedArgs a) {
                 }
                 const int ds = drm_slot(a.drm, node);
                 if (ds >= 0) fe += drm_force(a.drm, ds, kstep, DIM, c);
-                a.Unext[g0 + i] = u + ((fe - fi) + a.kforce[g0 + i] * (u - up[k])) / kd[k];
+                un = u + ((fe - fi) + a.kforce[g0 + i] * (u - up[k])) / kd[k];
             }
+            a.Unext[g0 + i] = un;
+            if (has_rec) record_dof(a.rec, g0 + i, 0, un);
         }
     }
 }
@@ -435,6 +477,7 @@ __device__ __forceinline__ void cd_corner_body(const FusedArgs &a) {
     const int h0 = a.halo_ptr[tile], nh = a.halo_ptr[tile + 1] - h0;
     const int e0 = a.elem_ptr[tile], ne = a.elem_ptr[tile + 1] - e0;
     const int npl = a.nplain[tile];  // read with the tile bounds (one scalar round trip)
+    const bool has_rec = tile_records(a.rec, tile);
     const int MO = MOC > 0 ? MOC + 1 : a.max_own;
     double *sU = smem;
     double *sX = smem + size_t(a.max_stage) * DIM;
@@ -723,12 +766,11 @@ __device__ __forceinline__ void cd_corner_body(const FusedArgs &a) {
     for (int d = 0; d < DIM; ++d) {
         const double u = sU[tid * DIM + d];
         const size_t g = g0 + size_t(tid) * DIM + d;
+        double un = 0.0;
         if (tid < npl) {
             // Plain nodes: kforce = keff (no damping), so Feff / keff = (u - up) - fi / keff.
-            a.Unext[g] = u + ((u - up[d]) - fi[d] * kd[d]);
-        } else if (kd[d] == 0.0) {
-            a.Unext[g] = 0.0;
-        } else {
+            un = u + ((u - up[d]) - fi[d] * kd[d]);
+        } else if (kd[d] != 0.0) {
             const int node = o0 + tid;
             double fe = 0.0;
             for (int q2 = a.nl_ptr[node]; q2 < a.nl_ptr[node + 1]; ++q2) {
@@ -738,14 +780,268 @@ __device__ __forceinline__ void cd_corner_body(const FusedArgs &a) {
                 fe += a.load_factor[l] * (amp * a.load_dir[size_t(l) * DIM + d]);
             }
             if (ds >= 0) fe += drm_force(a.drm, ds, kstep, DIM, d);
-            a.Unext[g] = u + ((fe - fi[d]) + a.kforce[g] * (u - up[d])) * kd[d];
+            un = u + ((fe - fi[d]) + a.kforce[g] * (u - up[d])) * kd[d];
         }
+        a.Unext[g] = un;
+        if (has_rec) record_dof(a.rec, g, 0, un);
     }
 }
 
 template <int DIM, int PATH, int MOC = 0, bool LATE = false, int NP = 2, bool PAD = false>
 __global__ __launch_bounds__(512) void k_cd_corner(FusedArgs a) {
     cd_corner_body<DIM, PATH, MOC, LATE, NP, PAD>(a);
+}
+
+// Arguments of the multi-step kernel.
+struct MultiArgs {
+    const int32_t *cnt, *node;
+    const uint16_t *econn, *ncor, *egeo;
+    const double *elam, *emu, *geo, *X, *Ucur, *Uprev;
+    double *out0, *out1, *out2;   // U_k, U_{k-1}, U_{k-2} of the owned nodes (null: not written)
+    const double *kforce, *kinv;
+    const int32_t *nl_ptr, *nl_idx;
+    const double *load_dir, *load_factor, *load_series;
+    int load_nt, k, nsteps;
+    double th, ftol;
+    int ntiles, depth, ns, ne, nu;
+    DrmRef drm;
+    RecRef rec;
+};
+
+// nsteps CentralDifference steps k .. k + nsteps - 1 for one node tile per workgroup, from one
+// staging of the tile's nodes and nsteps rings of neighbours: step t updates the nodes of the
+// rings that the steps after it still need, so tiles recompute each other's border instead of
+// meeting at a launch boundary (nsteps <= depth, or one tile that holds the whole mesh). Ring
+// nodes are computed by several tiles, each with the same operations in the same order.
+//
+// Bound: models whose single step leaves the chip idle are bound by the launch and by the chain of
+// dependent global round trips before the first element (4.3 us for 0.3 us of data on 40,602
+// DOFs), models of many tiles by the bytes of the state; both are paid once per nsteps
+// here, and what a step keeps is its own chain of two LDS round trips and two barriers.
+// One thread is one element and one node of the tile, with the element's constants and the node's
+// u, u_prev, 1/keff in registers over all the steps. Elements write their corner forces to
+// planes indexed by the element (neighbouring lanes, neighbouring words: no bank conflicts, no
+// slots to clear, no ownership test), and a node reads its at most one element per corner
+// position through 16-bit indices, in corner order; column ne of the planes is zero.
+template <int DIM, int PATH, int MAXB, int MAXE, bool WIDE>
+__global__ __launch_bounds__(MAXB) __attribute__((amdgpu_waves_per_eu(WIDE ? 8 : 1))) void k_cd_multi(MultiArgs a) {
+    constexpr int NEN = Elem<DIM>::nen;
+    constexpr bool STAGE_X = PATH < 2;
+    constexpr int MO = MAXE + 1;  // column MAXE: no element
+    extern __shared__ double smem[];
+    const int b = blockIdx.x, xcd = b & 7, j = b >> 3;
+    const int q = a.ntiles >> 3, r8 = a.ntiles & 7;
+    const int tile = xcd * q + min(xcd, r8) + j;
+    const int tid = threadIdx.x, n = a.nsteps;
+    // Scalar loads: as ordinary memory the counts cost a vector round trip at the head of every step.
+    const_i32 *ncnt = (const_i32 *)(a.cnt + size_t(tile) * 2 * (a.depth + 1)), *ecnt = ncnt + a.depth + 1;
+    double *sF = smem;  // [NEN * DIM][MO]
+    double *sU = sF + NEN * DIM * MO;
+    double *sX = sU + size_t(a.ns) * DIM;
+    // Everything addressed by the tile index goes out first, with indices clamped into the tile's rows.
+    const int32_t nraw = a.node[size_t(tile) * a.ns + min(tid, a.ns - 1)];
+    const size_t er = size_t(tile) * a.ne + min(tid, a.ne - 1);
+    const size_t cr = size_t(tile) * a.nu + min(tid, a.nu - 1);
+    uint32_t lcw[NEN / 2], ncw[NEN / 2];
+    if constexpr (NEN == 8) {
+        const uint4 x = *reinterpret_cast<const uint4 *>(a.econn + er * 8);
+        const uint4 y = *reinterpret_cast<const uint4 *>(a.ncor + cr * 8);
+        lcw[0] = x.x, lcw[1] = x.y, lcw[2] = x.z, lcw[3] = x.w;
+        ncw[0] = y.x, ncw[1] = y.y, ncw[2] = y.z, ncw[3] = y.w;
+    } else {
+        const uint2 x = *reinterpret_cast<const uint2 *>(a.econn + er * 4);
+        const uint2 y = *reinterpret_cast<const uint2 *>(a.ncor + cr * 4);
+        lcw[0] = x.x, lcw[1] = x.y;
+        ncw[0] = y.x, ncw[1] = y.y;
+    }
+    const double lam = a.elam[er], mu = a.emu[er];
+    const int gid = PATH >= 2 ? int(a.egeo[er]) : 0;
+    const int nown = ncnt[0];
+    const bool staged = tid < ncnt[min(n, a.depth)];
+    const int node = nraw & INT32_MAX;
+    const bool special = nraw < 0;
+    const size_t g = size_t(node) * DIM;
+    double u[DIM], up[DIM], kd[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+        u[d] = staged ? a.Ucur[g + d] : 0.0;
+        up[d] = staged ? a.Uprev[g + d] : 0.0;
+        kd[d] = staged ? a.kinv[g + d] : 0.0;
+    }
+    int q0 = 0, q1 = 0, ds = -1;
+    if (staged && special) {
+        q0 = a.nl_ptr[node];
+        q1 = a.nl_ptr[node + 1];
+        ds = drm_slot(a.drm, node);
+    }
+    if (staged) {
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            sU[tid * DIM + d] = u[d];
+            if constexpr (STAGE_X) sX[tid * DIM + d] = a.X[g + d];
+        }
+    }
+    if (tid < NEN * DIM) sF[tid * MO + MAXE] = 0.0;
+    // Few tiles: the node's first load stays in registers, so that a step waits for one load of
+    // its sample, in flight during the element phase (further loads are read in the step).
+    double f0 = 0.0, d0[DIM], kf[DIM];
+    const double *ser = nullptr;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) d0[d] = 0.0;
+    if constexpr (!WIDE)
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) kf[d] = (staged && special) ? a.kforce[g + d] : 0.0;
+    if constexpr (!WIDE)
+        if (q1 > q0) {
+            const int l = a.nl_idx[q0];
+            f0 = a.load_factor[l];
+            ser = a.load_series + size_t(l) * a.load_nt;
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) d0[d] = a.load_dir[size_t(l) * DIM + d];
+            ++q0;
+        }
+    int rc[DIM];
+    if constexpr (!WIDE)
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) rc[d] = (a.rec.map && tid < nown) ? a.rec.map[g + d] : -1;
+    const bool rec = WIDE && tile_records(a.rec, tile) && tid < nown;
+    int lc[NEN];
+#pragma unroll
+    for (int c = 0; c < NEN / 2; ++c) {
+        lc[2 * c] = int(lcw[c] & 0xffffu) * DIM;
+        lc[2 * c + 1] = int(lcw[c] >> 16) * DIM;
+    }
+    double Lam[DIM][DIM];
+    if constexpr (PATH >= 2) {
+        const double *gt = a.geo + size_t(gid) * (DIM * DIM);
+#pragma unroll
+        for (int x = 0; x < DIM; ++x)
+#pragma unroll
+            for (int y = 0; y < DIM; ++y) Lam[x][y] = gt[x * DIM + y];
+    }
+    int ee = ecnt[min(n - 1, a.depth - 1)], nn = ncnt[min(n - 1, a.depth)];
+    // Every load above has arrived before the loop: a wait inside it would also wait for the
+    // sample loads and history stores of the steps.
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    lds_barrier();
+    for (int t = 0; t < n; ++t) {
+        const int left = n - 1 - t, k = a.k + t;
+        // The next step's counts, a step ahead.
+        const int nl = max(left - 1, 0), een = ecnt[min(nl, a.depth - 1)], nnn = ncnt[min(nl, a.depth)];
+        const bool live = k >= 0 && k < a.load_nt;
+        double amp = 0.0, dr[DIM];
+        if constexpr (!WIDE) {
+            if (ser && live) amp = ser[k];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) dr[d] = ds >= 0 ? drm_force(a.drm, ds, k, DIM, d) : 0.0;
+        }
+        if (tid < ee) {
+            double v[NEN][DIM], f[NEN][DIM];
+#pragma unroll
+            for (int c = 0; c < NEN; ++c) {
+                if constexpr (DIM == 2) {
+                    const double2 w = *reinterpret_cast<const double2 *>(sU + lc[c]);
+                    v[c][0] = w.x;
+                    v[c][1] = w.y;
+                } else {
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) v[c][d] = sU[lc[c] + d];
+                }
+            }
+            if constexpr (PATH >= 2) {
+                if constexpr (DIM == 3)
+                    hexa_modal_force<PATH == 3>(Lam, lam, mu, v, f);
+                else
+                    quad_modal_force<PATH == 3>(Lam, lam, mu, v, f);
+            } else {
+                double x[NEN][DIM];
+#pragma unroll
+                for (int c = 0; c < NEN; ++c)
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) x[c][d] = sX[lc[c] + d];
+                if constexpr (DIM == 3) {
+                    if constexpr (PATH == 1)
+                        hexa_affine_fint(x, v, lam, mu, f);
+                    else
+                        hexa_fint(x, v, lam, mu, f);
+                } else {
+                    if constexpr (PATH == 1)
+                        quad_affine_fint(x, v, lam, mu, a.th, f);
+                    else
+                        quad_fint(x, v, lam, mu, a.th, f);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < NEN; ++c)
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) sF[(c * DIM + d) * MO + tid] = fabs(f[c][d]) > a.ftol ? f[c][d] : 0.0;
+        }
+        lds_barrier();
+        if (tid < nn) {
+            double fi[DIM];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) fi[d] = 0.0;
+#pragma unroll
+            for (int c = 0; c < NEN; ++c) {
+                const int e = (c & 1) ? int(ncw[c / 2] >> 16) : int(ncw[c / 2] & 0xffffu);
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) fi[d] += sF[(c * DIM + d) * MO + e];
+            }
+            double un[DIM];
+            if (!special) {
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) un[d] = u[d] + ((u[d] - up[d]) - fi[d] * kd[d]);
+            } else {
+                double fe[DIM];
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) fe[d] = f0 * (amp * d0[d]);
+                for (int x = q0; x < q1; ++x) {
+                    const int l = a.nl_idx[x];
+                    const double am = live ? a.load_series[size_t(l) * a.load_nt + k] : 0.0;
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) fe[d] += a.load_factor[l] * (am * a.load_dir[size_t(l) * DIM + d]);
+                }
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) {
+                    if constexpr (WIDE) {
+                        dr[d] = ds >= 0 ? drm_force(a.drm, ds, k, DIM, d) : 0.0;
+                        kf[d] = a.kforce[g + d];
+                    }
+                    un[d] = kd[d] == 0.0
+                                ? 0.0
+                                : u[d] + ((fe[d] + dr[d] - fi[d]) + kf[d] * (u[d] - up[d])) * kd[d];
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) {
+                up[d] = u[d];
+                u[d] = un[d];
+            }
+            if constexpr (DIM == 2) {
+                *reinterpret_cast<double2 *>(sU + tid * 2) = make_double2(un[0], un[1]);
+            } else {
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) sU[tid * DIM + d] = un[d];
+            }
+            // The last steps leave their displacements as they are made (left = 2: U_{k-2}, ...).
+            double *out = left == 0 ? a.out0 : left == 1 ? a.out1 : left == 2 ? a.out2 : nullptr;
+            if (out && tid < nown)
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) out[g + d] = un[d];
+            if constexpr (WIDE) {
+                if (rec)
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) record_dof(a.rec, g + d, t, un[d]);
+            } else {
+#pragma unroll
+                for (int d = 0; d < DIM; ++d)
+                    if (rc[d] >= 0) a.rec.hist[size_t(t) * a.rec.nrec + rc[d]] = un[d];
+            }
+        }
+        ee = een;
+        nn = nnn;
+        lds_barrier();
+    }
 }
 
 template <int DIM, int PATH>
@@ -834,9 +1130,10 @@ int prepare_fused(Model &m) {
 }
 
 static int launch_fused(Model &m, int k, const double *Ucur, const double *Uprev, double *Unext,
-                        const int *kdev = nullptr) {
+                        const int *kdev = nullptr, const RecRef *rec = nullptr) {
     const TileSet &t = m.tiles;
     FusedArgs a;
+    a.rec = rec ? *rec : RecRef{nullptr, nullptr, nullptr, 0};
     a.kdev = kdev;
     a.own_ptr = t.own_ptr.p;
     a.nplain = t.nplain.p;
@@ -908,7 +1205,184 @@ static int launch_fused(Model &m, int k, const double *Ucur, const double *Uprev
     return 0;
 }
 
-static int cd_one_step(Model &m, int k) {
+// Block and element-plane sizes of the multi-step kernel: the plan takes the smallest class that
+// holds its tiles (0: none does).
+struct MultiClass {
+    int block, elems;
+};
+static constexpr MultiClass kMulti2[] = {{256, 256}, {512, 456}, {1024, 968}}, kMulti3[] = {{256, 256}, {512, 512}, {1024, 640}};
+
+template <int DIM, int MAXB, int MAXE, bool WIDE>
+static const void *multi_fn_t(int path) {
+    switch (path) {
+        case 3: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 3, MAXB, MAXE, WIDE>);
+        case 2: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 2, MAXB, MAXE, WIDE && DIM == 2>);
+        case 1: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 1, MAXB, MAXE, false>);
+        default: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 0, MAXB, MAXE, false>);
+    }
+}
+
+static const void *multi_fn(const Model &m) {
+    const bool wide = m.multi.ntiles > 1024;
+    if (m.ndim == 2) {
+        switch (m.multi.block) {
+            case 256: return wide ? multi_fn_t<2, 256, 256, true>(m.elem_path) : multi_fn_t<2, 256, 256, false>(m.elem_path);
+            case 512: return wide ? multi_fn_t<2, 512, 456, true>(m.elem_path) : multi_fn_t<2, 512, 456, false>(m.elem_path);
+            default: return wide ? multi_fn_t<2, 1024, 968, true>(m.elem_path) : multi_fn_t<2, 1024, 968, false>(m.elem_path);
+        }
+    }
+    switch (m.multi.block) {
+        case 256: return multi_fn_t<3, 256, 256, false>(m.elem_path);
+        case 512: return multi_fn_t<3, 512, 512, false>(m.elem_path);
+        default: return multi_fn_t<3, 1024, 640, false>(m.elem_path);
+    }
+}
+
+// Steps per launch of the multi-step kernel for this model's tiles (0: single-step kernels).
+// Measured, microseconds per step, single-step kernel against the multi-step kernel:
+//   one tile (231 Quad4 nodes)            4.3 -> 0.80
+//   Quad4, 5,151 nodes, 64-node tiles     5.0 -> 1.37 (depth 6)      20,301 nodes, 128-node tiles  4.4 -> 1.42 (8)
+//   Quad4, 80,601 nodes, 400-node tiles   5.4 -> 2.24 (4)            0.55M nodes, 400-node tiles  13.5 -> 9.6 (4)
+//   Quad4, 1.77M nodes, 400-node tiles   29.4 -> 31.4 (4)            0.55M nodes, 128-node tiles  13.6 -> 19.9 (4)
+//   Hexa8, 1,183 / 8,125 nodes            5.6 -> 3.3 / 5.7 -> 3.6 (2)
+//   Hexa8, 18,513 / 60,025 nodes          5.9 -> 6.3 / 7.0 -> 17 (2)
+// Below a chip full of workgroups the launch is saved and the recomputed rings are free; above
+// it they compete with the tiles: in 2D the state's bytes still pay for them while a tile is
+// large against its rings and up to about a million nodes, in 3D never. Gauss-point hexahedra
+// (2,600 operations an element) recompute nothing.
+static int multi_depth(const Model &m) {
+    const int nt = m.tiles.ntiles, own = m.nnodes / nt;
+    if (nt == 1) return 1;
+    if (m.ndim == 3) return m.elem_path >= 2 && nt <= 384 && own <= 64 ? 2 : 0;
+    if (nt > 512) return own >= 256 && m.nnodes <= 1000000 ? 4 : 0;
+    int d = 1;  // rings up to about six times the tile
+    while (d < 8 && (2.0 * (d + 1)) * (2.0 * (d + 1)) <= 2.4 * own) ++d;
+    return d;
+}
+
+// The multi-step plan of a model that steps one tile per workgroup with kernels of the library's choice.
+static int multi_setup(Model &m) {
+    if (m.multi_tried) return 0;
+    m.multi_tried = true;
+    MultiSet &t = m.multi;
+    std::vector<int32_t> conn, own;
+    std::vector<uint8_t> special;
+    std::vector<double> lam, mu;
+    std::vector<uint16_t> gid;
+    conn.swap(m.h_conn);  // used once
+    special.swap(m.h_special);
+    lam.swap(m.h_lam);
+    mu.swap(m.h_mu);
+    gid.swap(m.h_gid);
+    if (!m.auto_variant || !m.corner_unique || m.sm_ndofs > 0 || m.elem_bf16 || m.elem_fp32) return 0;
+    int depth = multi_depth(m);
+    HostMulti h;
+    MultiClass cls{0, 0};
+    size_t lds = 0;
+    for (; depth >= 1; --depth) {  // the deepest that fits a class and the LDS
+        cls = MultiClass{0, 0};
+        if (make_multi(m.nnodes, m.nelem, m.nen, conn.data(), special.data(), m.h_own_ptr, depth, 1024, h))
+            for (const MultiClass &c : m.ndim == 2 ? kMulti2 : kMulti3)
+                if (cls.block == 0 && h.ns <= c.block && h.ne <= c.elems) cls = c;
+        lds = (size_t(m.elem_path < 2 ? 2 : 1) * h.ns * m.ndim + size_t(m.nen) * m.ndim * (cls.elems + 1)) *
+              sizeof(double);
+        if (cls.block != 0 && lds <= 160 * 1024) break;
+    }
+    if (depth < 1) return 0;
+    // No element at a corner: the zero column of the class.
+    for (uint16_t &c : h.ncor)
+        if (c == h.ne) c = uint16_t(cls.elems);
+    std::vector<double> el(h.elem.size(), 0.0), em(h.elem.size(), 0.0);
+    std::vector<uint16_t> eg(h.elem.size(), 0);
+    for (size_t i = 0; i < h.elem.size(); ++i) {
+        const int e = h.elem[i];
+        if (e < 0) continue;
+        const double sc = m.elem_path >= 2 ? m.h_escale[e] : 1.0;
+        el[i] = lam[e] * sc;
+        em[i] = mu[e] * sc;
+        if (m.elem_path >= 2) eg[i] = gid[e];
+    }
+    hipStream_t s = m.stream;
+    SVLG_HIP(t.cnt.upload(h.cnt.data(), h.cnt.size(), s));
+    SVLG_HIP(t.node.upload(h.node.data(), h.node.size(), s));
+    SVLG_HIP(t.econn.upload(h.econn.data(), h.econn.size(), s));
+    SVLG_HIP(t.ncor.upload(h.ncor.data(), h.ncor.size(), s));
+    SVLG_HIP(t.egeo.upload(eg.data(), eg.size(), s));
+    SVLG_HIP(t.elam.upload(el.data(), el.size(), s));
+    SVLG_HIP(t.emu.upload(em.data(), em.size(), s));
+    for (int i = 0; i < 2; ++i) SVLG_HIP(t.U[i].alloc(m.ndofn));
+    SVLG_HIP(hipStreamSynchronize(s));
+    t.ntiles = h.ntiles;
+    t.ns = h.ns;
+    t.ne = h.ne;
+    t.nu = h.nu;
+    t.block = cls.block;
+    t.lds_bytes = lds;
+    t.depth = depth;
+    if (lds > 64 * 1024)
+        SVLG_HIP(hipFuncSetAttribute(multi_fn(m), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    return 0;
+}
+
+// n steps from k in one launch (n <= depth, or one tile); last: the caller reads the state next,
+// which takes U_{k-2} too. Tiles read U_{k0} and U_{k0-1} of their neighbours, so the results go
+// to other buffers, which then take the place of those in the ring.
+static int multi_launch(Model &m, int k, int n, bool last, const RecRef &rec) {
+    MultiSet &t = m.multi;
+    double *&cur = m.U[m.ring].p, *&prev = m.U[(m.ring + 2) % 3].p, *&old = m.U[(m.ring + 1) % 3].p;
+    MultiArgs a;
+    a.cnt = t.cnt.p;
+    a.node = t.node.p;
+    a.econn = t.econn.p;
+    a.ncor = t.ncor.p;
+    a.egeo = t.egeo.p;
+    a.elam = t.elam.p;
+    a.emu = t.emu.p;
+    a.geo = m.geo.p;
+    a.X = m.X.p;
+    a.Ucur = cur;
+    a.Uprev = prev;
+    a.out0 = n == 1 ? old : t.U[0].p;
+    a.out1 = n == 1 ? nullptr : n == 2 ? old : t.U[1].p;
+    a.out2 = n >= 3 && last ? old : nullptr;
+    a.kforce = m.kforce.p;
+    a.kinv = m.kinv.p;
+    a.nl_ptr = m.nl_ptr.p;
+    a.nl_idx = m.nl_idx.p;
+    a.load_dir = m.load_dir.p;
+    a.load_factor = m.load_factor.p;
+    a.load_series = m.load_series.p;
+    a.load_nt = m.load_nt;
+    a.k = k;
+    a.nsteps = n;
+    a.th = m.th;
+    a.ftol = m.ftol;
+    a.ntiles = t.ntiles;
+    a.depth = t.depth;
+    a.ns = t.ns;
+    a.ne = t.ne;
+    a.nu = t.nu;
+    a.drm = drm_ref(m);
+    a.rec = rec;
+    void *args[] = {&a};
+    SVLG_HIP(hipLaunchKernel(multi_fn(m), dim3(t.ntiles), dim3(t.block), args, t.lds_bytes, m.stream));
+    if (n == 1) {
+        m.ring = (m.ring + 1) % 3;
+    } else if (n == 2) {
+        double *free_buf = prev;  // U_{k0-1} is no longer part of the state
+        prev = old;
+        old = cur;
+        cur = t.U[0].p;
+        t.U[0].p = free_buf;
+    } else {
+        std::swap(cur, t.U[0].p);
+        std::swap(prev, t.U[1].p);
+    }
+    m.steps_done += n;
+    return 0;
+}
+
+static int cd_one_step(Model &m, int k, const RecRef *rec = nullptr) {
     double *Ucur = m.U[m.ring].p;
     double *Uprev = m.U[(m.ring + 2) % 3].p;
     double *Unext = m.U[(m.ring + 1) % 3].p;
@@ -916,7 +1390,7 @@ static int cd_one_step(Model &m, int k) {
     // increment); afterwards U_(k-1) returns and U_k = U_(k-1) + a_k there.
     if (int rc = sm_lag_in(m, Ucur, Uprev, nullptr)) return rc;
     if (m.variant == 1 || m.variant == 3) {
-        if (int rc = launch_fused(m, k, Ucur, Uprev, Unext)) return rc;
+        if (int rc = launch_fused(m, k, Ucur, Uprev, Unext, nullptr, rec)) return rc;
         if (int rc = sm_finish(m, 1, k, Ucur, Unext)) return rc;
         m.ring = (m.ring + 1) % 3;
         m.steps_done++;
@@ -937,6 +1411,39 @@ static int cd_one_step(Model &m, int k) {
     return 0;
 }
 
+// Whether steps go through the multi-step kernel: a plan exists, and the stream is not being
+// captured by the caller (the launches exchange buffers, which a replay would not repeat).
+static bool multi_ready(const Model &m) {
+    if (m.multi.depth == 0) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(m.stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return st == hipStreamCaptureStatusNone;
+}
+
+// nsteps steps from k0, recording into rec (map null: nothing).
+static int cd_advance(Model &m, int k0, int nsteps, const RecRef &rec) {
+    if (!multi_ready(m)) {
+        RecRef r = rec;
+        for (int s = 0; s < nsteps; ++s) {
+            if (int rc = cd_one_step(m, k0 + s, rec.map ? &r : nullptr)) return rc;
+            if (rec.map) r.hist += rec.nrec;
+        }
+        return 0;
+    }
+    const int most = m.multi.ntiles == 1 ? 2048 : m.multi.depth;
+    RecRef r = rec;
+    for (int s = 0; s < nsteps;) {
+        const int n = std::min(most, nsteps - s);
+        if (int rc = multi_launch(m, k0 + s, n, s + n == nsteps, r)) return rc;
+        if (rec.map) r.hist += size_t(n) * rec.nrec;
+        s += n;
+    }
+    return 0;
+}
+
 // CentralDifference::Initialize (CentralDifference.cpp:36-71) with the per-DOF time steps
 // dtd (device DOF order) or one dt.
 static int cd_init_impl(Model &m, double dt, const std::vector<double> *dtd, double ftol) {
@@ -947,6 +1454,7 @@ static int cd_init_impl(Model &m, double dt, const std::vector<double> *dtd, dou
     m.dt = dt;
     m.ftol = ftol;
     m.cd_ready = false;
+    if (int rc = multi_setup(m)) return rc;
     if (m.cd_graph) {
         (void)hipGraphExecDestroy(m.cd_graph);
         m.cd_graph = nullptr;
@@ -1069,8 +1577,7 @@ int svlg_cd_steps_async(svlg_model *h, int32_t k0, int32_t nsteps) {
     SVLG_CHECK(h, "null model");
     Model &m = h->m;
     SVLG_CHECK(m.cd_ready, "svlg_cd_init has not been called");
-    for (int s = 0; s < nsteps; ++s)
-        if (int rc = cd_one_step(m, k0 + s)) return rc;
+    if (int rc = cd_advance(m, k0, nsteps, RecRef{nullptr, nullptr, nullptr, 0})) return rc;
     SVLG_HIP(hipGetLastError());
     return 0;
 }
@@ -1083,6 +1590,13 @@ int svlg_cd_graph_steps(svlg_model *h, int32_t k0, int32_t nsteps, int32_t graph
     SVLG_CHECK(m.variant == 1 || m.variant == 3, "graph stepping needs the fused kernel (variant 1 or 3)");
     SVLG_CHECK(graph_steps >= 3 && graph_steps % 3 == 0 && graph_steps <= 3000,
                "graph_steps must be a multiple of 3 in [3, 3000]");
+    if (multi_ready(m)) {
+        // A launch already covers several steps, with its step index and buffers as arguments:
+        // nothing is left for a graph to save.
+        if (int rc = cd_advance(m, k0, nsteps, RecRef{nullptr, nullptr, nullptr, 0})) return rc;
+        SVLG_HIP(hipGetLastError());
+        return 0;
+    }
     int done = 0;
     if (nsteps >= graph_steps) {
         if (!m.cd_graph || m.cd_graph_steps != graph_steps || m.cd_graph_ring != m.ring)
@@ -1117,9 +1631,10 @@ int svlg_autotune_tiles(const svlg_mesh_desc *desc, const svlg_exec_opts *base, 
         if (rc == 0 && (m.variant == 1 || m.variant == 3)) {
             hipEvent_t e0 = nullptr, e1 = nullptr;
             bool ok = hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess;
-            for (int s = 0; ok && s < 3; ++s) ok = cd_one_step(m, 1 + s) == 0;
+            const RecRef none{nullptr, nullptr, nullptr, 0};
+            ok = ok && cd_advance(m, 1, 3, none) == 0;
             ok = ok && hipEventRecord(e0, m.stream) == hipSuccess;
-            for (int s = 0; ok && s < steps; ++s) ok = cd_one_step(m, 4 + s) == 0;
+            ok = ok && cd_advance(m, 4, steps, none) == 0;
             ok = ok && hipEventRecord(e1, m.stream) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
             float ms = 0.0f;
             if (ok && hipEventElapsedTime(&ms, e0, e1) == hipSuccess) {
@@ -1144,19 +1659,75 @@ int svlg_cd_steps(svlg_model *h, int32_t k0, int32_t nsteps, int32_t nrec, const
     Model &m = h->m;
     SVLG_CHECK(m.cd_ready, "svlg_cd_init has not been called");
     SVLG_CHECK(nsteps >= 0 && nrec >= 0, "negative count");
+    RecRef rec{nullptr, nullptr, nullptr, 0};
+    std::vector<int32_t> dup;
+    // The step kernels record, except where support motion moves DOFs after them or the
+    // element-colored kernels run: there a kernel per step does.
+    const bool inside = m.sm_ndofs == 0 && (m.variant == 1 || m.variant == 3);
     if (nrec > 0) {
         SVLG_CHECK(rec_dofs && hist, "recorder arrays missing");
         std::vector<int32_t> rn;
         if (int rc = record_positions(m, nrec, rec_dofs, rn)) return rc;
-        SVLG_HIP(m.rec.upload(rn.data(), rn.size(), m.stream));
-        SVLG_HIP(m.hist.alloc(size_t(nrec) * std::max(nsteps, 1)));
+        const size_t want = size_t(nrec) * std::max(nsteps, 1);
+        if (m.hist.n < want) SVLG_HIP(m.hist.alloc(want));
+        if (inside) {
+            // A DOF asked for more than once is recorded in its first column and copied.
+            std::vector<int32_t> ord(nrec);
+            std::iota(ord.begin(), ord.end(), 0);
+            std::sort(ord.begin(), ord.end(),
+                      [&](int32_t a, int32_t b) { return rn[a] < rn[b] || (rn[a] == rn[b] && a < b); });
+            std::vector<int32_t> pos = rn;
+            std::vector<int32_t> tf(m.tiles.ntiles, 0);
+            for (int i = 0, first = 0; i < nrec; ++i) {
+                if (i > 0 && rn[ord[i]] == rn[ord[first]]) {
+                    dup.push_back(ord[i]);
+                    dup.push_back(ord[first]);
+                    pos[ord[i]] = -1;
+                } else {
+                    first = i;
+                    const int node = rn[ord[i]] / m.ndim;
+                    tf[std::upper_bound(m.h_own_ptr.begin(), m.h_own_ptr.end(), node) - m.h_own_ptr.begin() - 1] = 1;
+                }
+            }
+            if (!m.recmap.p) {
+                std::vector<int32_t> none(m.ndofn, -1);
+                SVLG_HIP(m.recmap.upload(none.data(), none.size(), m.stream));
+                SVLG_HIP(hipStreamSynchronize(m.stream));
+                SVLG_HIP(m.rectile.alloc(tf.size()));
+            }
+            if (m.rec.n < pos.size()) SVLG_HIP(m.rec.alloc(pos.size()));
+            SVLG_HIP(hipMemcpyAsync(m.rec.p, pos.data(), sizeof(int32_t) * pos.size(), hipMemcpyHostToDevice, m.stream));
+            SVLG_HIP(hipMemcpyAsync(m.rectile.p, tf.data(), sizeof(int32_t) * tf.size(), hipMemcpyHostToDevice, m.stream));
+            if (!dup.empty()) SVLG_HIP(m.recdup.upload(dup.data(), dup.size(), m.stream));
+            hipLaunchKernelGGL(k_rec_map, dim3((nrec + 255) / 256), dim3(256), 0, m.stream, nrec, m.rec.p, 1,
+                               m.recmap.p);
+            SVLG_HIP(hipStreamSynchronize(m.stream));  // the host arrays above end with this block
+            rec = RecRef{m.recmap.p, m.rectile.p, m.hist.p, nrec};
+        } else {
+            if (m.rec.n < rn.size()) SVLG_HIP(m.rec.alloc(rn.size()));
+            SVLG_HIP(hipMemcpyAsync(m.rec.p, rn.data(), sizeof(int32_t) * rn.size(), hipMemcpyHostToDevice, m.stream));
+            SVLG_HIP(hipStreamSynchronize(m.stream));
+        }
     }
-    for (int s = 0; s < nsteps; ++s) {
-        if (int rc = cd_one_step(m, k0 + s)) return rc;
-        if (nrec > 0)
-            hipLaunchKernelGGL(k_record, dim3((nrec + 63) / 64), dim3(64), 0, m.stream, nrec, m.rec.p, m.U[m.ring].p,
-                               m.hist.p + size_t(s) * nrec);
+    int rc = 0;
+    if (inside || nrec == 0) {
+        rc = cd_advance(m, k0, nsteps, rec);
+    } else {
+        for (int s = 0; s < nsteps && rc == 0; ++s) {
+            rc = cd_one_step(m, k0 + s);
+            if (rc == 0)
+                hipLaunchKernelGGL(k_record, dim3((nrec + 63) / 64), dim3(64), 0, m.stream, nrec, m.rec.p,
+                                   m.U[m.ring].p, m.hist.p + size_t(s) * nrec);
+        }
     }
+    if (rec.map) {
+        const int nd = int(dup.size() / 2);
+        if (nd > 0 && nsteps > 0 && rc == 0)
+            hipLaunchKernelGGL(k_rec_dup, dim3((size_t(nd) * nsteps + 255) / 256), dim3(256), 0, m.stream, nd,
+                               m.recdup.p, nsteps, nrec, m.hist.p);
+        hipLaunchKernelGGL(k_rec_map, dim3((nrec + 255) / 256), dim3(256), 0, m.stream, nrec, m.rec.p, 0, m.recmap.p);
+    }
+    if (rc) return rc;
     SVLG_HIP(hipGetLastError());
     if (nrec > 0 && nsteps > 0)
         SVLG_HIP(hipMemcpyAsync(hist, m.hist.p, sizeof(double) * size_t(nrec) * nsteps, hipMemcpyDeviceToHost,

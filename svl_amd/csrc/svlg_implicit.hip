@@ -34,7 +34,7 @@
 namespace svlg {
 
 int gather_free(Model &m, const double *dnode, double *dfree);
-int record_positions(const Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos);
+int record_positions(Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos);
 int scatter_free(Model &m, const double *dfree, double *dnode);
 
 enum { OP_CG = 0, OP_RHS = 1 };

@@ -166,15 +166,19 @@ int scatter_free(Model &m, const double *dfree, double *dnode) {
 // Recorder positions: rec_dofs[r] >= 0 is a free DOF index, -1 - t the total DOF t = node *
 // ndim + c of a mesh node (a restrained DOF, e.g. one with support motion); pos[r] is its
 // device node-DOF position.
-int record_positions(const Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos) {
-    std::vector<int32_t> f2n(m.nfree, -1);
-    for (int i = 0; i < m.ndofn; ++i)
-        if (m.h_free[i] >= 0) f2n[m.h_free[i]] = i;
+int record_positions(Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos) {
+    std::vector<int32_t> &f2n = m.h_f2n;
+    if (f2n.empty()) {
+        f2n.assign(m.nfree, -1);
+        for (int i = 0; i < m.ndofn; ++i)
+            if (m.h_free[i] >= 0) f2n[m.h_free[i]] = i;
+    }
     pos.assign(nrec, 0);
     for (int r = 0; r < nrec; ++r) {
         const int32_t v = rec_dofs[r];
         if (v >= 0) {
             SVLG_CHECK(v < m.nfree, "recorded DOF is not a free DOF");
+            SVLG_CHECK(f2n[v] >= 0, "recorded DOF is not a free DOF");
             pos[r] = f2n[v];
         } else {
             const int64_t t = -1 - int64_t(v);
@@ -323,7 +327,7 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     m.ndofn = nn * ndim;
     m.th = d->thickness;
     m.lumped = d->lumped != 0;
-    int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : (ndim == 3 ? 160 : 448);
+    int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : default_tile_nodes(ndim, nn);
     int block = (o && o->block > 0) ? o->block : 512;
     const int req_variant = (o && o->variant > 0) ? o->variant : 0;
     if (req_variant < 0 || req_variant > 3) { set_error("variant must be 0 (auto), 1, 2 or 3"); return fail(11); }
@@ -458,9 +462,10 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     std::vector<uint16_t> gid(ne, 0);
     if (m.affine && geo_opt != -1) {
         std::map<std::vector<uint64_t>, int> classes;
+        uint64_t last[10] = {};
         bool ok = true;
         for (int e = 0; e < ne && ok; ++e) {
-            std::vector<double> lam_e(ndim * ndim);
+            double lam_e[9];
             double adet;
             if (ndim == 3) {
                 double x[8][3], L[3][3];
@@ -477,15 +482,23 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
                 for (int i = 0; i < 4; ++i) lam_e[i] = L[i / 2][i % 2];
                 escale[e] = 0.25 * adet * m.th;
             }
-            std::vector<uint64_t> key(lam_e.size() + 1);
-            std::memcpy(key.data(), lam_e.data(), sizeof(double) * lam_e.size());
-            std::memcpy(&key[lam_e.size()], &adet, sizeof(double));
+            // Neighbouring elements mostly share their geometry: the previous class first.
+            const size_t ng = size_t(ndim) * ndim;
+            uint64_t raw[10] = {};
+            std::memcpy(raw, lam_e, sizeof(double) * ng);
+            std::memcpy(raw + ng, &adet, sizeof(double));
+            if (e > 0 && std::memcmp(raw, last, sizeof(uint64_t) * (ng + 1)) == 0) {
+                gid[e] = gid[e - 1];
+                continue;
+            }
+            std::memcpy(last, raw, sizeof(raw));
+            const std::vector<uint64_t> key(raw, raw + ng + 1);
             auto it = classes.find(key);
             if (it == classes.end()) {
                 if (classes.size() >= 65535) { ok = false; break; }
                 int id = int(classes.size());
                 classes.emplace(key, id);
-                gtab.insert(gtab.end(), lam_e.begin(), lam_e.end());
+                gtab.insert(gtab.end(), lam_e, lam_e + ng);
                 gid[e] = uint16_t(id);
             } else {
                 gid[e] = uint16_t(it->second);
@@ -508,6 +521,17 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
         UP(m.egid, gid.data(), gid.size());
     }
     m.h_escale = escale;
+    m.auto_variant = req_variant == 0;
+    m.corner_unique = corner_unique;
+    m.h_own_ptr = ht.own_ptr;
+    if (m.auto_variant && corner_unique) {
+        m.h_conn = connp;
+        m.h_special.resize(nn);
+        for (int p = 0; p < nn; ++p) m.h_special[p] = special[m.perm[p]];
+        m.h_lam = lam;
+        m.h_mu = mu;
+        m.h_gid = gid;
+    }
     // Tiles.
     {
         TileSet &t = m.tiles;
@@ -754,7 +778,7 @@ int svlg_plan_tiles(const svlg_mesh_desc *d, int32_t tile_nodes, int64_t *stats)
     HostTiles t;
     try {
         make_tiles(ndim, nn, ne, nen, d->coords, d->conn, color.data(), ncolors, special.data(),
-                   tile_nodes > 0 ? tile_nodes : (ndim == 3 ? 160 : 448), t);
+                   tile_nodes > 0 ? tile_nodes : default_tile_nodes(ndim, nn), t);
     } catch (const std::exception &ex) {
         set_error(std::string("tiling failed: ") + ex.what());
         return 11;

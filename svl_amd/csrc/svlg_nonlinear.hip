@@ -25,7 +25,7 @@
 namespace svlg {
 
 int gather_free(Model &m, const double *dnode, double *dfree);
-int record_positions(const Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos);
+int record_positions(Model &m, int nrec, const int32_t *rec_dofs, std::vector<int32_t> &pos);
 int launch_nl_rhs(Model &m, int k, const double *un, const double *w, const double *dU, double *b);
 
 static constexpr int kNlGrid = 256, kNlBlock = 512;

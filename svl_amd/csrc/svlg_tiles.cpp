@@ -9,9 +9,11 @@
 // elements reach outside the tile. This layout has no counterpart in SVL, which
 // loops over a std::map of elements (RP/07-Assembler/Assembler.cpp:240-269).
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <numeric>
 #include <stdexcept>
+#include <thread>
 #include <vector>
 
 #include "svlg_tiles.hpp"
@@ -153,6 +155,116 @@ void make_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const
     }
     t.elem_ptr[t.ntiles] = int32_t(t.elem_id.size());
     t.halo_ptr[t.ntiles] = int32_t(t.halo_node.size());
+}
+
+bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8_t *special,
+                const std::vector<int32_t> &own_ptr, int depth, int max_threads, HostMulti &t) {
+    const int nt = int(own_ptr.size()) - 1;
+    std::vector<int32_t> n2e_ptr(nnodes + 1, 0), n2e(size_t(nelem) * nen);
+    for (size_t i = 0; i < size_t(nelem) * nen; ++i) n2e_ptr[conn[i] + 1]++;
+    for (int n = 0; n < nnodes; ++n) n2e_ptr[n + 1] += n2e_ptr[n];
+    {
+        std::vector<int32_t> p(n2e_ptr.begin(), n2e_ptr.end() - 1);
+        for (int e = 0; e < nelem; ++e)
+            for (int a = 0; a < nen; ++a) n2e[p[conn[size_t(e) * nen + a]]++] = e;
+    }
+    struct Tile {
+        std::vector<int32_t> node, elem, ncnt, ecnt;
+    };
+    std::vector<Tile> tiles(nt);
+    // Tiles are independent: a few host threads take them in turn (the result does not depend on
+    // which thread built a tile).
+    const int nthr = std::max(1, std::min({8, int(std::thread::hardware_concurrency()), nt / 16}));
+    std::atomic<int> next{0};
+    std::atomic<bool> fits{true};
+    auto run = [&](auto &&fn) {
+        next = 0;
+        std::vector<std::thread> th;
+        for (int i = 1; i < nthr; ++i) th.emplace_back(fn);
+        fn();
+        for (auto &x : th) x.join();
+    };
+    run([&] {
+        std::vector<int32_t> seen_n(nnodes, -1), seen_e(nelem, -1);
+        for (int ti; fits && (ti = next++) < nt;) {
+            Tile &q = tiles[ti];
+            for (int32_t n = own_ptr[ti]; n < own_ptr[ti + 1]; ++n) {
+                q.node.push_back(n);
+                seen_n[n] = ti;
+            }
+            q.ncnt.push_back(int32_t(q.node.size()));
+            size_t from = 0;
+            for (int d = 0; d < depth; ++d) {
+                const size_t end = q.node.size(), e0 = q.elem.size();
+                for (size_t i = from; i < end; ++i)
+                    for (int k = n2e_ptr[q.node[i]]; k < n2e_ptr[q.node[i] + 1]; ++k)
+                        if (seen_e[n2e[k]] != ti) {
+                            seen_e[n2e[k]] = ti;
+                            q.elem.push_back(n2e[k]);
+                        }
+                for (size_t i = e0; i < q.elem.size(); ++i)
+                    for (int a = 0; a < nen; ++a) {
+                        const int32_t n = conn[size_t(q.elem[i]) * nen + a];
+                        if (seen_n[n] != ti) {
+                            seen_n[n] = ti;
+                            q.node.push_back(n);
+                        }
+                    }
+                std::sort(q.node.begin() + end, q.node.end());
+                from = end;
+                q.ecnt.push_back(int32_t(q.elem.size()));
+                q.ncnt.push_back(int32_t(q.node.size()));
+                if (int(q.node.size()) > max_threads || int(q.elem.size()) > max_threads) {
+                    fits = false;
+                    break;
+                }
+            }
+        }
+    });
+    if (!fits) return false;
+    t.depth = depth;
+    t.ntiles = nt;
+    t.ns = t.ne = t.nu = 1;
+    for (const Tile &q : tiles) {
+        t.ns = std::max(t.ns, q.ncnt[depth]);
+        t.ne = std::max(t.ne, q.ecnt[depth - 1]);
+        t.nu = std::max(t.nu, q.ncnt[depth - 1]);
+    }
+    const int nc = 2 * (depth + 1);
+    t.cnt.assign(size_t(nt) * nc, 0);
+    t.node.assign(size_t(nt) * t.ns, 0);
+    t.elem.assign(size_t(nt) * t.ne, -1);
+    t.econn.assign(size_t(nt) * t.ne * nen, 0);
+    t.ncor.assign(size_t(nt) * t.nu * nen, uint16_t(t.ne));
+    run([&] {
+        std::vector<int32_t> slot(nnodes, -1), ord;
+        for (int ti; (ti = next++) < nt;) {
+            Tile &q = tiles[ti];
+            for (size_t i = 0; i < q.node.size(); ++i) {
+                slot[q.node[i]] = int32_t(i);
+                t.node[size_t(ti) * t.ns + i] = q.node[i] | (special[q.node[i]] ? INT32_MIN : 0);
+            }
+            for (int d = 0; d <= depth; ++d) t.cnt[size_t(ti) * nc + d] = q.ncnt[d];
+            for (int d = 0; d < depth; ++d) t.cnt[size_t(ti) * nc + depth + 1 + d] = q.ecnt[d];
+            // Inside a layer: in the order of the first corner's slot (neighbouring lanes gather
+            // neighbouring LDS words).
+            for (int d = 0; d < depth; ++d)
+                std::sort(q.elem.begin() + (d ? q.ecnt[d - 1] : 0), q.elem.begin() + q.ecnt[d],
+                          [&](int32_t a, int32_t b) {
+                              const int32_t x = slot[conn[size_t(a) * nen]], y = slot[conn[size_t(b) * nen]];
+                              return x < y || (x == y && a < b);
+                          });
+            for (size_t i = 0; i < q.elem.size(); ++i) {
+                t.elem[size_t(ti) * t.ne + i] = q.elem[i];
+                for (int a = 0; a < nen; ++a) {
+                    const int32_t sl = slot[conn[size_t(q.elem[i]) * nen + a]];
+                    t.econn[(size_t(ti) * t.ne + i) * nen + a] = uint16_t(sl);
+                    if (sl < q.ncnt[depth - 1]) t.ncor[(size_t(ti) * t.nu + sl) * nen + a] = uint16_t(i);
+                }
+            }
+        }
+    });
+    return true;
 }
 
 }  // namespace svlg

@@ -21,9 +21,43 @@ struct HostTiles {
     std::vector<int32_t> color_ptr;  // [ntiles*(ncolors+1)] offsets inside the tile's elements
 };
 
+// Node-tile size when the caller names none. 3D: 160 nodes fill the chip and recompute 0.7
+// elements per element; up to 12,000 nodes smaller tiles spread the mesh over the 256 CUs and leave
+// room for the second ring of the multi-step kernel (8,125 nodes: 36 to 48 nodes 3.6 us per
+// step, 64 nodes 3.8, 160 nodes 5.7). 2D: one tile while a workgroup holds the mesh, then tiles that
+// give about a workgroup per CU (5,151 nodes: 64 nodes 1.37 us, 128 nodes 1.43; 20,301 nodes: 128 nodes
+// 1.42, 64 nodes 1.64), 400 nodes where the rings of the multi-step kernel need the room
+// (80,601 nodes: 400 nodes 2.2 us, 128 nodes 3.2), and 192 nodes above a million, where single steps
+// of small workgroups hide their latencies best (1.77M nodes: 192 nodes 29.4 us; 448 nodes 28 us when
+// no tile touches more than 512 elements, 52 us when one does).
+inline int default_tile_nodes(int ndim, int nnodes) {
+    if (ndim == 3) return nnodes <= 160 ? 160 : nnodes <= 12000 ? 40 : 160;
+    if (nnodes <= 512) return 512;
+    return nnodes <= 8000 ? 64 : nnodes <= 36000 ? 128 : nnodes <= 1000000 ? 400 : 192;
+}
+
 // special[n] != 0 marks nodes that need the general update (restrained DOF, dashpot,
 // Rayleigh mass damping, point load).
 void make_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const int32_t *conn,
                 const int32_t *color, int ncolors, const uint8_t *special, int max_own, HostTiles &t);
+
+// Deep-halo plan of the multi-step explicit kernel over the same tiles: every tile's nodes in
+// rings around its owned nodes (ring d: reached through d layers of elements) and its elements in
+// layers (layer d: touching a node of ring d or nearer), so that a workgroup can advance its owned
+// nodes by up to `depth` steps from one staging. All arrays have fixed strides per tile.
+struct HostMulti {
+    int depth = 0, ntiles = 0;
+    int ns = 0, ne = 0, nu = 0;      // strides: staged nodes, elements, updated nodes (rings < depth)
+    std::vector<int32_t> cnt;        // [ntiles][2 (depth + 1)]: nodes up to ring 0..depth, elements up to layer 0..depth-1, 0
+    std::vector<int32_t> node;       // [ntiles][ns] device node, the sign bit set on special nodes
+    std::vector<int32_t> elem;       // [ntiles][ne] element (tag order), -1 padding
+    std::vector<uint16_t> econn;     // [ntiles][ne][nen] staged slot of each corner
+    std::vector<uint16_t> ncor;      // [ntiles][nu][nen] tile element whose corner a the node is; ne: none
+};
+
+// own_ptr, conn and special in device numbering; false if a tile needs more than max_threads
+// staged nodes or elements.
+bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8_t *special,
+                const std::vector<int32_t> &own_ptr, int depth, int max_threads, HostMulti &t);
 
 }  // namespace svlg

@@ -189,3 +189,66 @@ def test_color_phase_kernel_repeats_exactly():
     dm.close()
     assert np.isfinite(runs[0]).all() and np.abs(runs[0]).max() > 0.0
     assert np.array_equal(runs[0], runs[1]) and np.array_equal(runs[0], runs[2])
+
+
+def _multi_model(kind):
+    if kind == "quad_one_tile":
+        return W.realization2d(20, 10, 5, nt=61)[:2]
+    if kind == "quad_tiles":
+        return W.realization2d(61, 37, 6, nt=61)[:2]
+    if kind == "quad_large_tiles":
+        return W.realization2d(233, 171, 7, nt=61)[:2]
+    if kind == "hexa_one_tile":
+        return block_model(4, 4, 3)[:2]
+    if kind == "hexa_one_tile_distorted":
+        return block_model(4, 3, 4, distort=0.15, seed=3)[:2]
+    if kind == "hexa_tiles":
+        return W.halfspace3d(13, 11, 9, nt=61)[:2]
+    if kind == "hexa_tiles_rotated":
+        return block_model(11, 9, 8, transform=rotation())[:2]
+    from _meshes import drm_quad_model
+    from svl_amd.drm import attach, drm_box
+    m, box = drm_quad_model(61, 1e-3)
+    elems, nodes, cond = drm_box(m, *box)
+    sig = np.random.default_rng(8).standard_normal((nodes.size, 61, 6)) * 1e-4
+    attach(m, elems, nodes, cond, sig)
+    return m, 1e-3
+
+
+@pytest.mark.parametrize("kind", ["quad_one_tile", "quad_tiles", "quad_large_tiles", "hexa_one_tile",
+                                  "hexa_one_tile_distorted", "hexa_tiles", "hexa_tiles_rotated", "drm"])
+def test_multi_step_kernel(kind):
+    """The multi-step kernel (default options) against the single-step kernel (variant 3) over 60 steps,
+    with one node under two loads and columns recorded twice; calls of every length up to past its depth
+    equal one call bit for bit, state and history. Both add the same terms in the same corner order
+    and differ in the rounding of a few contractions only: 1e-12."""
+    m, dt = _multi_model(kind)
+    n = int(m.load_node[0])
+    m.add_point_load(n, np.ones(m.ndim), 3e4 * np.sin(0.3 * np.arange(m.load_series.shape[1])), 0.7)
+    rec = np.concatenate([np.arange(0, m.nfree, 7), [0, 14, 7, 7]]).astype(np.int32)
+    dm = DeviceModel(m)
+    cd = CentralDifference(dm, dt)
+    cd.Initialize()
+    hist = cd.advance(1, 60, rec)
+    state = [cd.GetDisplacements(), cd.GetVelocities(), cd.GetAccelerations()]
+    cd.Initialize()
+    parts, k = [], 1
+    for c in (1, 2, 3, 4, 5, 9, 11, 1, 1, 2, 21):
+        parts.append(cd.advance(k, c, rec))
+        k += c
+    again = [cd.GetDisplacements(), cd.GetVelocities(), cd.GetAccelerations()]
+    assert np.array_equal(np.concatenate(parts), hist)
+    for a, b in zip(state, again):
+        assert np.array_equal(a, b)
+    dm.close()
+    ref = DeviceModel(m, variant=3)
+    cr = CentralDifference(ref, dt)
+    cr.Initialize()
+    href = cr.advance(1, 60, rec)
+    assert rel_l2(hist, href) < 1e-12
+    assert rel_l2(state[0], cr.GetDisplacements()) < 1e-12
+    # V and A divide differences of U by dt and dt^2: their rounding grows by |U| / (dt |V|) and |U| / (dt^2 |A|).
+    for f, (a, b, h) in enumerate(((state[1], cr.GetVelocities(), dt), (state[2], cr.GetAccelerations(), dt * dt))):
+        amp = np.linalg.norm(state[0]) / (h * np.linalg.norm(b))
+        assert rel_l2(a, b) < 1e-12 * max(1.0, amp), f
+    ref.close()
