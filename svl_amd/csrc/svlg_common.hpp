@@ -85,10 +85,11 @@ struct MultiSet {
     int depth = 0;                           // 0: not built, one step per launch
     int ntiles = 0, ns = 0, ne = 0, nu = 0, block = 0;
     size_t lds_bytes = 0;
-    DevBuf<int32_t> cnt, node;
-    DevBuf<uint16_t> econn, ncor, egeo;
-    DevBuf<double> elam, emu;
-    DevBuf<double> U[3];                     // output buffers, exchanged with the state's ring
+    DevBuf<uint8_t> slab;                    // holds the arrays below
+    const int32_t *cnt = nullptr, *node = nullptr;
+    const uint16_t *econn = nullptr, *ncor = nullptr, *egeo = nullptr;
+    const double *elam = nullptr, *emu = nullptr;
+    DevBuf<double> U[2];                     // output buffers, exchanged with the state's ring
 };
 
 struct Model {

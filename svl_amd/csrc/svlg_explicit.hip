@@ -14,6 +14,7 @@
 // U_{k-2}) can be formed on demand with SVL's expressions.
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <numeric>
 
 #include "svlg_common.hpp"
@@ -1292,26 +1293,42 @@ static int multi_setup(Model &m) {
     // No element at a corner: the zero column of the class.
     for (uint16_t &c : h.ncor)
         if (c == h.ne) c = uint16_t(cls.elems);
-    std::vector<double> el(h.elem.size(), 0.0), em(h.elem.size(), 0.0);
-    std::vector<uint16_t> eg(h.elem.size(), 0);
-    for (size_t i = 0; i < h.elem.size(); ++i) {
-        const int e = h.elem[i];
-        if (e < 0) continue;
-        const double sc = m.elem_path >= 2 ? m.h_escale[e] : 1.0;
-        el[i] = lam[e] * sc;
-        em[i] = mu[e] * sc;
-        if (m.elem_path >= 2) eg[i] = gid[e];
-    }
     hipStream_t s = m.stream;
-    SVLG_HIP(t.cnt.upload(h.cnt.data(), h.cnt.size(), s));
-    SVLG_HIP(t.node.upload(h.node.data(), h.node.size(), s));
-    SVLG_HIP(t.econn.upload(h.econn.data(), h.econn.size(), s));
-    SVLG_HIP(t.ncor.upload(h.ncor.data(), h.ncor.size(), s));
-    SVLG_HIP(t.egeo.upload(eg.data(), eg.size(), s));
-    SVLG_HIP(t.elam.upload(el.data(), el.size(), s));
-    SVLG_HIP(t.emu.upload(em.data(), em.size(), s));
-    for (int i = 0; i < 2; ++i) SVLG_HIP(t.U[i].alloc(m.ndofn));
+    // One allocation and one copy for all of it (each costs tens of microseconds of set-up).
+    size_t total = 0;
+    auto room = [&](size_t bytes) {
+        const size_t at = total;
+        total += (bytes + 15) / 16 * 16;
+        return at;
+    };
+    const size_t ne = h.elem.size(), o_cnt = room(h.cnt.size() * 4), o_node = room(h.node.size() * 4),
+                 o_econn = room(h.econn.size() * 2), o_ncor = room(h.ncor.size() * 2), o_egeo = room(ne * 2),
+                 o_lam = room(ne * 8), o_mu = room(ne * 8);
+    std::unique_ptr<uint8_t[]> slab(new uint8_t[total]);
+    std::memcpy(slab.get() + o_cnt, h.cnt.data(), h.cnt.size() * 4);
+    std::memcpy(slab.get() + o_node, h.node.data(), h.node.size() * 4);
+    std::memcpy(slab.get() + o_econn, h.econn.data(), h.econn.size() * 2);
+    std::memcpy(slab.get() + o_ncor, h.ncor.data(), h.ncor.size() * 2);
+    uint16_t *eg = reinterpret_cast<uint16_t *>(slab.get() + o_egeo);
+    double *el = reinterpret_cast<double *>(slab.get() + o_lam), *em = reinterpret_cast<double *>(slab.get() + o_mu);
+    for (size_t i = 0; i < ne; ++i) {
+        const int e = h.elem[i];
+        const double sc = e >= 0 && m.elem_path >= 2 ? m.h_escale[e] : 1.0;
+        el[i] = e >= 0 ? lam[e] * sc : 0.0;
+        em[i] = e >= 0 ? mu[e] * sc : 0.0;
+        eg[i] = e >= 0 && m.elem_path >= 2 ? gid[e] : uint16_t(0);
+    }
+    SVLG_HIP(t.slab.alloc(total));
+    SVLG_HIP(hipMemcpyAsync(t.slab.p, slab.get(), total, hipMemcpyHostToDevice, s));
     SVLG_HIP(hipStreamSynchronize(s));
+    t.cnt = reinterpret_cast<const int32_t *>(t.slab.p + o_cnt);
+    t.node = reinterpret_cast<const int32_t *>(t.slab.p + o_node);
+    t.econn = reinterpret_cast<const uint16_t *>(t.slab.p + o_econn);
+    t.ncor = reinterpret_cast<const uint16_t *>(t.slab.p + o_ncor);
+    t.egeo = reinterpret_cast<const uint16_t *>(t.slab.p + o_egeo);
+    t.elam = reinterpret_cast<const double *>(t.slab.p + o_lam);
+    t.emu = reinterpret_cast<const double *>(t.slab.p + o_mu);
+    for (int i = 0; i < 2; ++i) SVLG_HIP(t.U[i].alloc(m.ndofn));
     t.ntiles = h.ntiles;
     t.ns = h.ns;
     t.ne = h.ne;
@@ -1331,13 +1348,13 @@ static int multi_launch(Model &m, int k, int n, bool last, const RecRef &rec) {
     MultiSet &t = m.multi;
     double *&cur = m.U[m.ring].p, *&prev = m.U[(m.ring + 2) % 3].p, *&old = m.U[(m.ring + 1) % 3].p;
     MultiArgs a;
-    a.cnt = t.cnt.p;
-    a.node = t.node.p;
-    a.econn = t.econn.p;
-    a.ncor = t.ncor.p;
-    a.egeo = t.egeo.p;
-    a.elam = t.elam.p;
-    a.emu = t.emu.p;
+    a.cnt = t.cnt;
+    a.node = t.node;
+    a.econn = t.econn;
+    a.ncor = t.ncor;
+    a.egeo = t.egeo;
+    a.elam = t.elam;
+    a.emu = t.emu;
     a.geo = m.geo.p;
     a.X = m.X.p;
     a.Ucur = cur;

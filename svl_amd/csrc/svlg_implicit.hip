@@ -527,7 +527,7 @@ __global__ void k_kdiag_colored(int e0, int e1, const int32_t *__restrict__ conn
             if constexpr (DIM == 2)
                 quad_fint(x, u, lam[tag], mu[tag], th, f);
             else
-                hexa_fint(x, u, lam[tag], mu[tag], f);
+                hexa_fint_points(x, u, lam[tag], mu[tag], f);
             double v = cf * f[a][d];
             if (rho) {
 #pragma unroll

@@ -327,7 +327,8 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     m.ndofn = nn * ndim;
     m.th = d->thickness;
     m.lumped = d->lumped != 0;
-    int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : default_tile_nodes(ndim, nn);
+    m.affine = all_affine(ndim, ne, nen, d->conn, d->coords);
+    int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : default_tile_nodes(ndim, nn, m.affine, any_j2);
     int block = (o && o->block > 0) ? o->block : 512;
     const int req_variant = (o && o->variant > 0) ? o->variant : 0;
     if (req_variant < 0 || req_variant > 3) { set_error("variant must be 0 (auto), 1, 2 or 3"); return fail(11); }
@@ -344,7 +345,6 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
         set_error("element coloring needs more than 64 colors");
         return fail(11);
     }
-    m.affine = all_affine(ndim, ne, nen, d->conn, d->coords);
     std::vector<double> am(ne, 0.0), ak(ne, 0.0);
     for (int e = 0; e < ne; ++e) {
         if (d->ray_am) am[e] = d->ray_am[e];
@@ -775,10 +775,15 @@ int svlg_plan_tiles(const svlg_mesh_desc *d, int32_t tile_nodes, int64_t *stats)
         SVLG_CHECK(d->drm_elem && d->drm_elem[i] >= 0 && d->drm_elem[i] < ne, "DRM element out of range");
         for (int a = 0; a < nen; ++a) special[d->conn[size_t(d->drm_elem[i]) * nen + a]] = 1;
     }
+    bool has_j2 = false;
+    for (int e = 0; d->mat_type && e < ne; ++e) has_j2 |= d->mat_type[e] == SVLG_MAT_J2;
     HostTiles t;
     try {
         make_tiles(ndim, nn, ne, nen, d->coords, d->conn, color.data(), ncolors, special.data(),
-                   tile_nodes > 0 ? tile_nodes : default_tile_nodes(ndim, nn), t);
+                   tile_nodes > 0 ? tile_nodes
+                                  : default_tile_nodes(ndim, nn, all_affine(ndim, ne, nen, d->conn, d->coords),
+                                                       has_j2),
+                   t);
     } catch (const std::exception &ex) {
         set_error(std::string("tiling failed: ") + ex.what());
         return 11;

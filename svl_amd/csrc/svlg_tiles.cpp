@@ -170,11 +170,12 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
     }
     struct Tile {
         std::vector<int32_t> node, elem, ncnt, ecnt;
+        std::vector<uint16_t> conn;
     };
     std::vector<Tile> tiles(nt);
     // Tiles are independent: a few host threads take them in turn (the result does not depend on
     // which thread built a tile).
-    const int nthr = std::max(1, std::min({8, int(std::thread::hardware_concurrency()), nt / 16}));
+    const int nthr = std::max(1, std::min({12, int(std::thread::hardware_concurrency()), nt / 16}));
     std::atomic<int> next{0};
     std::atomic<bool> fits{true};
     auto run = [&](auto &&fn) {
@@ -185,32 +186,35 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
         for (auto &x : th) x.join();
     };
     run([&] {
-        std::vector<int32_t> seen_n(nnodes, -1), seen_e(nelem, -1);
+        std::vector<int32_t> slot(nnodes, -1), seen(nelem, -1);
         for (int ti; fits && (ti = next++) < nt;) {
             Tile &q = tiles[ti];
             for (int32_t n = own_ptr[ti]; n < own_ptr[ti + 1]; ++n) {
+                slot[n] = int32_t(q.node.size());
                 q.node.push_back(n);
-                seen_n[n] = ti;
             }
             q.ncnt.push_back(int32_t(q.node.size()));
             size_t from = 0;
             for (int d = 0; d < depth; ++d) {
+                // Elements in the order of the nodes that reach them first: neighbouring lanes gather
+                // neighbouring LDS words.
                 const size_t end = q.node.size(), e0 = q.elem.size();
                 for (size_t i = from; i < end; ++i)
                     for (int k = n2e_ptr[q.node[i]]; k < n2e_ptr[q.node[i] + 1]; ++k)
-                        if (seen_e[n2e[k]] != ti) {
-                            seen_e[n2e[k]] = ti;
+                        if (seen[n2e[k]] != ti) {
+                            seen[n2e[k]] = ti;
                             q.elem.push_back(n2e[k]);
                         }
                 for (size_t i = e0; i < q.elem.size(); ++i)
                     for (int a = 0; a < nen; ++a) {
                         const int32_t n = conn[size_t(q.elem[i]) * nen + a];
-                        if (seen_n[n] != ti) {
-                            seen_n[n] = ti;
+                        if (slot[n] < 0) {
+                            slot[n] = 0;
                             q.node.push_back(n);
                         }
                     }
                 std::sort(q.node.begin() + end, q.node.end());
+                for (size_t i = end; i < q.node.size(); ++i) slot[q.node[i]] = int32_t(i);
                 from = end;
                 q.ecnt.push_back(int32_t(q.elem.size()));
                 q.ncnt.push_back(int32_t(q.node.size()));
@@ -219,6 +223,11 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
                     break;
                 }
             }
+            q.conn.resize(q.elem.size() * nen);
+            for (size_t i = 0; i < q.elem.size(); ++i)
+                for (int a = 0; a < nen; ++a)
+                    q.conn[i * nen + a] = uint16_t(slot[conn[size_t(q.elem[i]) * nen + a]]);
+            for (int32_t n : q.node) slot[n] = -1;
         }
     });
     if (!fits) return false;
@@ -237,31 +246,19 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
     t.econn.assign(size_t(nt) * t.ne * nen, 0);
     t.ncor.assign(size_t(nt) * t.nu * nen, uint16_t(t.ne));
     run([&] {
-        std::vector<int32_t> slot(nnodes, -1), ord;
         for (int ti; (ti = next++) < nt;) {
-            Tile &q = tiles[ti];
-            for (size_t i = 0; i < q.node.size(); ++i) {
-                slot[q.node[i]] = int32_t(i);
+            const Tile &q = tiles[ti];
+            for (size_t i = 0; i < q.node.size(); ++i)
                 t.node[size_t(ti) * t.ns + i] = q.node[i] | (special[q.node[i]] ? INT32_MIN : 0);
-            }
             for (int d = 0; d <= depth; ++d) t.cnt[size_t(ti) * nc + d] = q.ncnt[d];
             for (int d = 0; d < depth; ++d) t.cnt[size_t(ti) * nc + depth + 1 + d] = q.ecnt[d];
-            // Inside a layer: in the order of the first corner's slot (neighbouring lanes gather
-            // neighbouring LDS words).
-            for (int d = 0; d < depth; ++d)
-                std::sort(q.elem.begin() + (d ? q.ecnt[d - 1] : 0), q.elem.begin() + q.ecnt[d],
-                          [&](int32_t a, int32_t b) {
-                              const int32_t x = slot[conn[size_t(a) * nen]], y = slot[conn[size_t(b) * nen]];
-                              return x < y || (x == y && a < b);
-                          });
-            for (size_t i = 0; i < q.elem.size(); ++i) {
-                t.elem[size_t(ti) * t.ne + i] = q.elem[i];
+            std::copy(q.elem.begin(), q.elem.end(), t.elem.begin() + size_t(ti) * t.ne);
+            std::copy(q.conn.begin(), q.conn.end(), t.econn.begin() + size_t(ti) * t.ne * nen);
+            for (size_t i = 0; i < q.elem.size(); ++i)
                 for (int a = 0; a < nen; ++a) {
-                    const int32_t sl = slot[conn[size_t(q.elem[i]) * nen + a]];
-                    t.econn[(size_t(ti) * t.ne + i) * nen + a] = uint16_t(sl);
+                    const int sl = q.conn[i * nen + a];
                     if (sl < q.ncnt[depth - 1]) t.ncor[(size_t(ti) * t.nu + sl) * nen + a] = uint16_t(i);
                 }
-            }
         }
     });
     return true;

@@ -21,7 +21,7 @@ struct HostTiles {
     std::vector<int32_t> color_ptr;  // [ntiles*(ncolors+1)] offsets inside the tile's elements
 };
 
-// Node-tile size when the caller names none. 3D: 160 nodes fill the chip and recompute 0.7
+// Node-tile size when the caller names none (bricks: the elements are parallelepipeds). 3D: 160 nodes fill the chip and recompute 0.7
 // elements per element; up to 12,000 nodes smaller tiles spread the mesh over the 256 CUs and leave
 // room for the second ring of the multi-step kernel (8,125 nodes: 36 to 48 nodes 3.6 us per
 // step, 64 nodes 3.8, 160 nodes 5.7). 2D: one tile while a workgroup holds the mesh, then tiles that
@@ -30,8 +30,14 @@ struct HostTiles {
 // (80,601 nodes: 400 nodes 2.2 us, 128 nodes 3.2), and 192 nodes above a million, where single steps
 // of small workgroups hide their latencies best (1.77M nodes: 192 nodes 29.4 us; 448 nodes 28 us when
 // no tile touches more than 512 elements, 52 us when one does).
-inline int default_tile_nodes(int ndim, int nnodes) {
-    if (ndim == 3) return nnodes <= 160 ? 160 : nnodes <= 12000 ? 40 : 160;
+// Gauss-point hexahedra (256 registers, one wave per SIMD) take 96 nodes, whose elements are three
+// waves: 16,128 nodes 9.5 us per step against 12.9 with 160 and 12.2 with 64 nodes, 62,279 nodes 18.0
+// against 23.3 and 24.1.
+// Models with J2 elements keep one size: the tiles set the order of the solver's dot products, and
+// a yielding point's elastic or plastic branch can follow their last bits.
+inline int default_tile_nodes(int ndim, int nnodes, bool bricks, bool j2) {
+    if (j2) return ndim == 3 ? 160 : 448;
+    if (ndim == 3) return nnodes <= 160 ? 160 : nnodes <= 12000 ? 40 : bricks ? 160 : 96;
     if (nnodes <= 512) return 512;
     return nnodes <= 8000 ? 64 : nnodes <= 36000 ? 128 : nnodes <= 1000000 ? 400 : 192;
 }
