@@ -75,6 +75,7 @@ struct TileSet {
     // Built when the element path needs no staged coordinates and one staging pass covers
     // every tile; hstride = 0 otherwise.
     int hstride = 0, estride = 0;
+    bool one_pass = false;  // two strides of the block cover every tile's owned DOFs and halo (variant 3)
     DevBuf<int32_t> hpad;
     DevBuf<uint16_t> lcpad, geopad;
     DevBuf<double> lampad, mupad;
@@ -189,8 +190,7 @@ struct Model {
     int cd_graph_steps = 0, cd_graph_ring = -1;
     DevBuf<int> kdev;
     // Captured runs of CG iterations (2 or 8, starting at an even iteration) for the solution
-    // buffers the integrators reuse, keyed by (x, flexible, operator kernel, count); the
-    // iteration base lives in jdev.
+    // buffers the integrators reuse, keyed by (x, flexible, operator kernel, count).
     struct CgGraph {
         hipGraphExec_t exec;
         const double *x;
@@ -199,7 +199,6 @@ struct Model {
         int count;
     };
     std::vector<CgGraph> cg_graphs;
-    DevBuf<int> jdev;
     void drop_cg_graphs() {
         for (auto &g : cg_graphs) (void)hipGraphExecDestroy(g.exec);
         cg_graphs.clear();
@@ -224,6 +223,7 @@ struct Model {
     DevBuf<double> scal;              // device scalars of the solver
     int cg_last_iters[2] = {0, 0};    // iterations of the last solve (Jacobi, flexible)
     double *scal_host = nullptr;      // pinned host copy of the solver scalars (convergence polls)
+    double poll_seq = 0.0;            // number of the last poll
     std::vector<int32_t> tile_elem_id;   // tag index of every tile element (host)
     DevBuf<int32_t> tile_eid;         // the same on the device
 

@@ -76,7 +76,6 @@ struct GcnArgs {
     double *z, *scal;
     CgParts cg;
     int iter, normalize;
-    const int *jdev;           // non-null: the iteration is *jdev + iter (graph replays)
     int test;                  // first layer in the solver: CG's stopping test on r_iter first
     const float *elamf, *emuf, *dgnf;  // FP32 copies of elam, emu, dgn (one-channel kernel)
     const float *jacf;                 // D^-1 in FP32 (one-channel kernel)
@@ -146,10 +145,10 @@ __global__ __launch_bounds__(512) void k_gcn_layer(GcnArgs a) {
     __shared__ double red[3 * 17];
     if constexpr (MODE != G_BWD) {
         if (a.scal && a.scal[SC_DONE] != 0.0) return;
-        if (a.test && cg_stop_test(a.cg, a.jdev, a.iter, a.scal, red)) return;
+        if (a.test && cg_stop_test(a.cg, a.iter, a.scal, red)) return;
     }
     double sig = 1.0;
-    if constexpr (MODE == G_OUT) sig = gcn_sigma(a.cg, iter_of(a.jdev, a.iter), a.normalize, a.ndofn, red);
+    if constexpr (MODE == G_OUT) sig = gcn_sigma(a.cg, a.iter, a.normalize, a.ndofn, red);
     const int nt = a.ntiles;
     const int bI = blockIdx.x, xcd = bI & 7, j = bI >> 3;
     const int q = nt >> 3, r = nt & 7;
@@ -263,7 +262,7 @@ __global__ __launch_bounds__(512) void k_gcn_layer(GcnArgs a) {
         acc0 = block_sum(acc0, red);
         acc1 = block_sum(acc1, red);
         if (tid == 0) {
-            double *t = a.cg.tp + size_t(iter_of(a.jdev, a.iter) & 1) * 3 * nt;
+            double *t = a.cg.tp + size_t(a.iter & 1) * 3 * nt;
             t[3 * tile] = acc0;
             t[3 * tile + 1] = acc1;
             t[3 * tile + 2] = 0.0;
@@ -304,7 +303,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MOC > 0 ? 8
     // First layer in the solver: the stopping test on r_iter (with the DONE flag) before the
     // prefetch, whose registers would be held across the test's barriers.
     if constexpr (TEST)
-        if (cg_stop_test(a.cg, a.jdev, a.iter, a.scal, red)) return;
+        if (cg_stop_test(a.cg, a.iter, a.scal, red)) return;
     int hn[2];
     uint4 pk[MAXR];
     if constexpr (PAD) {
@@ -320,7 +319,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MOC > 0 ? 8
     if constexpr (!TEST)
         if (a.scal && a.scal[SC_DONE] != 0.0) return;
     double sig = 1.0;
-    if constexpr (OUT) sig = gcn_sigma(a.cg, iter_of(a.jdev, a.iter), a.normalize, a.ndofn, red);
+    if constexpr (OUT) sig = gcn_sigma(a.cg, a.iter, a.normalize, a.ndofn, red);
     const int o0 = a.own_ptr[tile], nown = a.own_ptr[tile + 1] - o0;
     const int h0 = a.halo_ptr[tile], nh = a.halo_ptr[tile + 1] - h0;
     const int e0 = a.elem_ptr[tile], ne = a.elem_ptr[tile + 1] - e0;
@@ -452,7 +451,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(MOC > 0 ? 8
         acc0 = block_sum(acc0, red);
         acc1 = block_sum(acc1, red);
         if (tid == 0) {
-            double *t = a.cg.tp + size_t(iter_of(a.jdev, a.iter) & 1) * 3 * nt;
+            double *t = a.cg.tp + size_t(a.iter & 1) * 3 * nt;
             t[3 * tile] = acc0;
             t[3 * tile + 1] = acc1;
             t[3 * tile + 2] = 0.0;
@@ -485,11 +484,10 @@ __global__ void k_gcn_kimg(const float *__restrict__ kmat, uint4 *__restrict__ i
 __global__ __launch_bounds__(512) void k_gcn_first(int n, int C, int normalize, CgParts cg, int j,
                                                    const double *__restrict__ r, const double *__restrict__ s,
                                                    const float *__restrict__ c1, const double *scal,
-                                                   float *__restrict__ x0, float *__restrict__ h1,
-                                                   const int *jdev) {
+                                                   float *__restrict__ x0, float *__restrict__ h1) {
     __shared__ double red[3 * 17];
     if (normalize && scal[SC_DONE] != 0.0) return;
-    const double sig = gcn_sigma(cg, iter_of(jdev, j), normalize, n, red);
+    const double sig = gcn_sigma(cg, j, normalize, n, red);
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const float xv = float(s[i] * r[i] / sig);
         x0[i] = xv;
@@ -773,11 +771,11 @@ static bool gcn_scaled_states(const Model &m) { return m.gcn_mfma && m.gcn_C == 
 static const double *gcn_input_scale(const Model &m) { return gcn_scaled_states(m) ? m.jac.p : m.gcn_s.p; }
 
 static int gcn_run(Model &m, const CgParts &cg, int j, const double *r, const double *q, double *z, int normalize,
-                   const int *jdev = nullptr, bool first = true, bool test = false) {
+                   bool first = true, bool test = false) {
     const int n = m.ndofn, C = m.gcn_C, L = m.gcn_L;
     if (first)
         hipLaunchKernelGGL(k_gcn_first, dim3(kVecGrid), dim3(kVecBlock), 0, m.stream, n, C, normalize, cg, j, r,
-                           gcn_input_scale(m), theta_c(m, 1), m.scal.p, m.gcn_x0.p, m.gcn_h[0].p, jdev);
+                           gcn_input_scale(m), theta_c(m, 1), m.scal.p, m.gcn_x0.p, m.gcn_h[0].p);
     GcnArgs a = gcn_args(m);
     int cur = 0;
     for (int l = 2; l <= L; ++l) {
@@ -793,7 +791,6 @@ static int gcn_run(Model &m, const CgParts &cg, int j, const double *r, const do
         if (a.test || mode == G_OUT) {
             a.cg = cg;
             a.iter = j;
-            a.jdev = jdev;
         }
         if (mode == G_OUT) {
             a.w = theta_w(m);
@@ -802,7 +799,6 @@ static int gcn_run(Model &m, const CgParts &cg, int j, const double *r, const do
             a.z = z;
             a.cg = cg;
             a.iter = j;
-            a.jdev = jdev;
             a.normalize = normalize;
         }
         if (gcn_scaled_states(m)) {
@@ -820,8 +816,8 @@ static int gcn_run(Model &m, const CgParts &cg, int j, const double *r, const do
 
 // In the solver the network runs unnormalised (it is linear in r, and FP32 / BF16 cover the
 // residual's range), so its input layer comes from the CG vector kernel with no global norm.
-int gcn_precond(Model &m, const CgParts &c, int j, const double *r, const double *q, double *z, const int *jdev) {
-    return gcn_run(m, c, j, r, q, z, 0, jdev, false, true);
+int gcn_precond(Model &m, const CgParts &c, int j, const double *r, const double *q, double *z) {
+    return gcn_run(m, c, j, r, q, z, 0, false, true);
 }
 
 GcnInput gcn_input_args(Model &m) {
@@ -841,7 +837,7 @@ static int gcn_loss_grad(Model &m, int np, const double *const *R, const double 
     for (int p = 0; p < np; ++p) {
         // Forward with stored states: H^l at gcn_H + l * plane (l = 1..L), Ehat H^(l-1) at gcn_Y + l * plane.
         hipLaunchKernelGGL(k_gcn_first, dim3(kVecGrid), dim3(kVecBlock), 0, s, n, C, 0, CgParts{}, 0, R[p],
-                           m.gcn_s.p, theta_c(m, 1), m.scal.p, m.gcn_x0.p, m.gcn_H.p + plane, nullptr);
+                           m.gcn_s.p, theta_c(m, 1), m.scal.p, m.gcn_x0.p, m.gcn_H.p + plane);
         GcnArgs a = gcn_args(m);
         for (int l = 2; l <= L; ++l) {
             a.in = m.gcn_H.p + size_t(l - 1) * plane;

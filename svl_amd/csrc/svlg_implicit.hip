@@ -20,6 +20,8 @@
 // touching its nodes and sums the corner slots of each owned node in a fixed order, so a
 // solve is bitwise reproducible.
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -74,7 +76,6 @@ struct OpArgs {
     const double *state;   // [nelem * ngp * kJ2State]
     const int32_t *plastic;  // [nelem] elastoplastic tangent somewhere in the element
     const double *Vm, *dUn;
-    const int *jdev;       // non-null: the iteration is *jdev + iter (graph replays)
     int nelem;             // elements (the Gauss-point state stride)
     DrmRef drm;            // OP_RHS: domain reduction forces of every step (F null: none)
     // Consistent mass (kernels with CM): per tile element the mass scale (OP_CG: times
@@ -100,7 +101,13 @@ struct OpArgs {
 // w = 4/dt V + A (Newton: 4/dt V + A - 4/dt^2 dU) and subtracts M_e (w_e + am V_e) from its
 // slot, so that the node sum gives Feff = Fext - sum_e [K_e (U - ak V) - M_e (w + am V)]_e
 // + C_dash V.
-template <int DIM, int PATH, int MODE, bool NL, int MOC = 0, bool CM = false>
+// PRE (OP_CG, tiles whose owned DOFs and halo take two strides of the block at most): every load that
+// does not depend on beta (tile bounds, element data, z and p_old of owned and halo nodes) is
+// issued before the sums behind beta, whose own three dependent round trips and barriers they
+// overlap: the kernel is that chain, not its bytes (2,196 Quad4 nodes 6.9 -> 6.1 us, 64^3 block with 2,188
+// tiles under the learned preconditioner 47 -> 32 us; the partials of J2 tangents as before).
+// The arithmetic and its order stay.
+template <int DIM, int PATH, int MODE, bool NL, int MOC = 0, bool CM = false, bool PRE = false>
 __global__ __launch_bounds__(512) void k_nm_op(OpArgs a) {
     constexpr int NEN = Elem<DIM>::nen;
     // J2 Gauss-point loops need the coordinates, except on axis-aligned Hexa8 bricks (the
@@ -111,46 +118,9 @@ __global__ __launch_bounds__(512) void k_nm_op(OpArgs a) {
     constexpr int NPRE = RHS ? (CM ? 3 : 2) : 1;  // staged state arrays before the coordinates
     extern __shared__ double smem[];
     __shared__ double red[3 * 17];
-    double beta = 0.0;
-    if constexpr (!RHS) {
-        if (a.reduce) {
-            // The DONE flag and *jdev are loaded together.
-            const double flag = a.scal[SC_DONE];
-            const int j = iter_of(a.jdev, a.iter);
-            if (flag != 0.0) return;
-            // Stopping test and beta of iteration j from the partials of the previous kernels;
-            // scal holds r.z and p.q of iteration j-1 (left by the vector kernel). The flexible
-            // solve's test on r_j was applied by the first layer of its preconditioner
-            // (cg_stop_test, the same sums), which set DONE if it held: only beta remains.
-            double v[3] = {0.0, 0.0, 0.0};
-            bool done = false;
-            if (!a.cg.flexible) {
-                cg_vec(a.cg, j, red, v);
-                done = v[1] <= a.scal[SC_TOL2] * v[2] || v[2] == 0.0;
-            }
-            if (j > 0) {
-                if (a.cg.flexible) {
-                    double zz[2];
-                    cg_pre(a.cg, j, red, zz);
-                    const double pq = a.scal[SC_PQ];
-                    beta = pq != 0.0 ? -zz[1] / pq : 0.0;
-                } else {
-                    const double rz0 = a.scal[SC_RHO];
-                    beta = rz0 != 0.0 ? v[0] / rz0 : 0.0;
-                }
-            }
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                if (!a.cg.flexible) {
-                    a.scal[SC_RR] = v[1];
-                    a.scal[SC_BB] = v[2];
-                }
-                a.scal[SC_ITERS] = double(j);
-                a.scal[SC_BETA] = beta;
-                if (done) a.scal[SC_DONE] = 1.0;
-            }
-            if (done) return;
-        }
-    }
+    double flag = 0.0;
+    if constexpr (!RHS)
+        if (a.reduce) flag = a.scal[SC_DONE];
     const int nt = a.ntiles;
     // XCD-aware mapping: consecutive workgroups go to different XCDs, each XCD walks a
     // contiguous range of tiles.
@@ -190,36 +160,115 @@ __global__ __launch_bounds__(512) void k_nm_op(OpArgs a) {
 #pragma unroll
         for (int c = 0; c < NEN; ++c) lc[c] = 0;
     }
-    for (int i = tid; i < nown * DIM; i += B) {
-        const size_t g = g0 + i;
-        if constexpr (RHS) {
-            sU[i] = a.U[g];
-            sV[i] = a.V[g];
-            if constexpr (CM)
-                sW[i] = a.Vm ? 4.0 / a.dt * a.Vm[g] + a.A[g] - 4.0 / a.dt / a.dt * a.dUn[g]
-                             : 4.0 / a.dt * a.V[g] + a.A[g];
-        } else {
-            const double v = a.z[g] + beta * a.p_old[g];
-            sU[i] = v;
-            a.p_new[g] = v;
-        }
-        if constexpr (STAGE_X) sX[i] = a.X[g];
-    }
-    for (int sl = tid; sl < nh; sl += B) {
-        const size_t n = size_t(a.halo_node[h0 + sl]) * DIM;
+    constexpr int NS = 2;
+    double zo[NS], po[NS], zh[NS][DIM], ph[NS][DIM];
+    if constexpr (PRE) {
+        int hn[NS];
 #pragma unroll
-        for (int c = 0; c < DIM; ++c) {
-            const int i = (nown + sl) * DIM + c;
-            if constexpr (RHS) {
-                sU[i] = a.U[n + c];
-                sV[i] = a.V[n + c];
-                if constexpr (CM)
-                    sW[i] = a.Vm ? 4.0 / a.dt * a.Vm[n + c] + a.A[n + c] - 4.0 / a.dt / a.dt * a.dUn[n + c]
-                                 : 4.0 / a.dt * a.V[n + c] + a.A[n + c];
-            } else {
-                sU[i] = a.z[n + c] + beta * a.p_old[n + c];
+        for (int k = 0; k < NS; ++k) hn[k] = k * B + tid < nh ? a.halo_node[h0 + k * B + tid] : 0;
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            const int i = k * B + tid;
+            zo[k] = i < nown * DIM ? a.z[g0 + i] : 0.0;
+            po[k] = i < nown * DIM ? a.p_old[g0 + i] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+#pragma unroll
+            for (int c = 0; c < DIM; ++c) {
+                const bool in = k * B + tid < nh;
+                zh[k][c] = in ? a.z[size_t(hn[k]) * DIM + c] : 0.0;
+                ph[k][c] = in ? a.p_old[size_t(hn[k]) * DIM + c] : 0.0;
             }
-            if constexpr (STAGE_X) sX[i] = a.X[n + c];
+    }
+    double beta = 0.0;
+    if constexpr (!RHS) {
+        if (a.reduce) {
+            if (flag != 0.0) return;
+            const int j = a.iter;
+            // Stopping test and beta of iteration j from the partials of the previous kernels;
+            // scal holds r.z and p.q of iteration j-1 (left by the vector kernel). The flexible
+            // solve's test on r_j was applied by the first layer of its preconditioner
+            // (cg_stop_test, the same sums), which set DONE if it held: only beta remains.
+            double v[3] = {0.0, 0.0, 0.0};
+            bool done = false;
+            if (!a.cg.flexible) {
+                cg_vec(a.cg, j, red, v);
+                done = v[1] <= a.scal[SC_TOL2] * v[2] || v[2] == 0.0;
+            }
+            // (In the first iteration both scalars are the reset's zeros, and beta is 0.)
+            if (a.cg.flexible) {
+                double zz[2];
+                cg_pre(a.cg, j, red, zz);
+                const double pq = a.scal[SC_PQ];
+                beta = pq != 0.0 ? -zz[1] / pq : 0.0;
+            } else {
+                const double rz0 = a.scal[SC_RHO];
+                beta = rz0 != 0.0 ? v[0] / rz0 : 0.0;
+            }
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+                if (!a.cg.flexible) {
+                    a.scal[SC_RR] = v[1];
+                    a.scal[SC_BB] = v[2];
+                }
+                const double cnt = a.scal[SC_CNT];
+                a.scal[SC_ITERS] = cnt;
+                if (!done) a.scal[SC_CNT] = cnt + 1.0;
+                a.scal[SC_BETA] = beta;
+                if (done) a.scal[SC_DONE] = 1.0;
+            }
+            if (done) return;
+        }
+    }
+    if constexpr (PRE) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+            const int i = k * B + tid;
+            if (i < nown * DIM) {
+                const double v = zo[k] + beta * po[k];
+                sU[i] = v;
+                a.p_new[g0 + i] = v;
+                if constexpr (STAGE_X) sX[i] = a.X[g0 + i];
+            }
+            if (i < nh)
+#pragma unroll
+                for (int c = 0; c < DIM; ++c) {
+                    sU[(nown + i) * DIM + c] = zh[k][c] + beta * ph[k][c];
+                    if constexpr (STAGE_X) sX[(nown + i) * DIM + c] = a.X[size_t(a.halo_node[h0 + i]) * DIM + c];
+                }
+        }
+    } else {
+        for (int i = tid; i < nown * DIM; i += B) {
+            const size_t g = g0 + i;
+            if constexpr (RHS) {
+                sU[i] = a.U[g];
+                sV[i] = a.V[g];
+                if constexpr (CM)
+                    sW[i] = a.Vm ? 4.0 / a.dt * a.Vm[g] + a.A[g] - 4.0 / a.dt / a.dt * a.dUn[g]
+                                 : 4.0 / a.dt * a.V[g] + a.A[g];
+            } else {
+                const double v = a.z[g] + beta * a.p_old[g];
+                sU[i] = v;
+                a.p_new[g] = v;
+            }
+            if constexpr (STAGE_X) sX[i] = a.X[g];
+        }
+        for (int sl = tid; sl < nh; sl += B) {
+            const size_t n = size_t(a.halo_node[h0 + sl]) * DIM;
+#pragma unroll
+            for (int c = 0; c < DIM; ++c) {
+                const int i = (nown + sl) * DIM + c;
+                if constexpr (RHS) {
+                    sU[i] = a.U[n + c];
+                    sV[i] = a.V[n + c];
+                    if constexpr (CM)
+                        sW[i] = a.Vm ? 4.0 / a.dt * a.Vm[n + c] + a.A[n + c] - 4.0 / a.dt / a.dt * a.dUn[n + c]
+                                     : 4.0 / a.dt * a.V[n + c] + a.A[n + c];
+                } else {
+                    sU[i] = a.z[n + c] + beta * a.p_old[n + c];
+                }
+                if constexpr (STAGE_X) sX[i] = a.X[n + c];
+            }
         }
     }
     for (int i = tid; i < NEN * DIM * MO; i += B) sIn[i] = 0.0;
@@ -339,7 +388,7 @@ __global__ __launch_bounds__(512) void k_nm_op(OpArgs a) {
     if constexpr (!RHS) {
         if (!a.reduce) return;
         const double sp = block_sum(acc, red);
-        if (tid == 0) a.cg.pq[size_t(iter_of(a.jdev, a.iter) & 1) * nt + tile] = sp;
+        if (tid == 0) a.cg.pq[size_t(a.iter & 1) * nt + tile] = sp;
     }
 }
 
@@ -382,41 +431,25 @@ __global__ __launch_bounds__(512) void k_cg_init(int n, CgParts c, const double 
     }
 }
 
-// Iteration j: alpha_j = r_j.z_j / p_j.q_j; x += alpha p; r -= alpha q; for Jacobi also
-// z = jac r. Partials (r.z (Jacobi), r.r, b.b) of iteration j+1 into vp[(j+1)&1]; the first
+// Iteration j (given by its parity): alpha_j = r_j.z_j / p_j.q_j; x += alpha p; r -= alpha q; for
+// Jacobi also z = jac r. Partials (r.z (Jacobi), r.r, b.b) of iteration j+1 into vp[(j+1)&1]; the first
 // workgroup leaves r_j.z_j and p_j.q_j in scal for the next operator kernel.
-__global__ __launch_bounds__(512) void k_cg_update(int n, int j0, CgParts c, double *scal, double *__restrict__ x,
+// The vectors of the first four strides are loaded before the sums behind alpha, and both sums go
+// through one reduction (the order of each is that of a reduction of its own): the kernel is
+// otherwise a chain of three round trips and four barriers (4,392 DOFs: 6.1 -> 4.5 us, 140,000 DOFs 6.9 -> 5.5).
+__global__ __launch_bounds__(512) void k_cg_update(int n, int j, CgParts c, double *scal, double *__restrict__ x,
                                                    const double *__restrict__ p, const double *__restrict__ q,
                                                    double *__restrict__ r, double *__restrict__ z,
-                                                   const double *__restrict__ jac, const int *jdev, GcnInput g) {
+                                                   const double *__restrict__ jac, GcnInput g) {
     __shared__ double red[3 * 17];
     const double flag = scal[SC_DONE];
-    const int j = iter_of(jdev, j0);
-    if (flag != 0.0) return;
-    const double pq = cg_pq(c, j, red);
-    double rzj;
-    if (c.flexible) {
-        double zz[2];
-        cg_pre(c, j, red, zz);
-        rzj = zz[0];
-    } else {
-        double v[3];
-        cg_vec(c, j, red, v);
-        rzj = v[0];
-    }
-    const double alpha = pq != 0.0 ? rzj / pq : 0.0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        scal[SC_RHO] = rzj;
-        scal[SC_PQ] = pq;
-        scal[SC_ALPHA] = alpha;
-    }
-    double rz = 0.0, rr = 0.0;
     // Grid-stride loop, four strides per pass with every load issued first (the per-thread
     // summation order is that of the plain grid-stride loop).
     constexpr int NB = 4;
     const int S = gridDim.x * blockDim.x;
-    for (int base = blockIdx.x * blockDim.x + threadIdx.x; base < n; base += NB * S) {
-        double xv[NB], pv[NB], qv[NB], rv[NB], jv[NB];
+    int base = blockIdx.x * blockDim.x + threadIdx.x;
+    double xv[NB], pv[NB], qv[NB], rv[NB], jv[NB];
+    auto load = [&] {
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
             const int i = base + k * S;
@@ -427,6 +460,29 @@ __global__ __launch_bounds__(512) void k_cg_update(int n, int j0, CgParts c, dou
             rv[k] = in ? r[i] : 0.0;
             jv[k] = (in && !c.flexible) ? jac[i] : 0.0;
         }
+    };
+    load();
+    // p_j.q_j over the operator's tiles; r_j.z_j over the vector partials (Jacobi) or the
+    // preconditioner's tiles.
+    double v[2] = {0.0, 0.0}, tot[2];
+    {
+        const double *pq = c.pq + size_t(j & 1) * c.ntiles;
+        for (int i = threadIdx.x; i < c.ntiles; i += blockDim.x) v[0] += pq[i];
+        const double *rz = c.flexible ? c.tp + size_t(j & 1) * 3 * c.ntiles : c.vp + size_t(j & 1) * 3 * c.nvb;
+        const int cnt = c.flexible ? c.ntiles : c.nvb;
+        for (int i = threadIdx.x; i < cnt; i += blockDim.x) v[1] += rz[size_t(i) * 3];
+    }
+    if (flag != 0.0) return;
+    reduce_records<2>(v, red, tot);
+    const double pq = tot[0], rzj = tot[1];
+    const double alpha = pq != 0.0 ? rzj / pq : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        scal[SC_RHO] = rzj;
+        scal[SC_PQ] = pq;
+        scal[SC_ALPHA] = alpha;
+    }
+    double acc[2] = {0.0, 0.0};  // r.z, r.r
+    for (; base < n; base += NB * S) {
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
             const int i = base + k * S;
@@ -437,21 +493,35 @@ __global__ __launch_bounds__(512) void k_cg_update(int n, int j0, CgParts c, dou
             if (!c.flexible) {
                 const double zi = jv[k] * ri;
                 z[i] = zi;
-                rz += ri * zi;
+                acc[0] += ri * zi;
             } else {
                 gcn_input(g, n, i, ri);
             }
-            rr += ri * ri;
+            acc[1] += ri * ri;
+        }
+        if (base + NB * S < n) {
+            base += NB * S;
+            load();
+            base -= NB * S;
         }
     }
-    rz = block_sum(rz, red);
-    rr = block_sum(rr, red);
+    double rs[2];
+    reduce_records<2>(acc, red, rs);
     if (threadIdx.x == 0) {
-        double *v = c.vp + size_t((j + 1) & 1) * 3 * c.nvb;
-        v[3 * blockIdx.x + 0] = rz;
-        v[3 * blockIdx.x + 1] = rr;
-        v[3 * blockIdx.x + 2] = c.ip[blockIdx.x];
+        double *o = c.vp + size_t((j + 1) & 1) * 3 * c.nvb;
+        o[3 * blockIdx.x + 0] = rs[0];
+        o[3 * blockIdx.x + 1] = rs[1];
+        o[3 * blockIdx.x + 2] = c.ip[blockIdx.x];
     }
+}
+
+// The scalars into pinned host memory, then the poll's number for the host that waits for it.
+__global__ void k_cg_poll(const double *__restrict__ scal, double seq, double *host) {
+    const int i = threadIdx.x;
+    if (i < SC_COUNT && i != SC_SEQ) host[i] = scal[i];
+    __threadfence_system();
+    __syncthreads();
+    if (i == 0) *reinterpret_cast<volatile double *>(host + SC_SEQ) = seq;
 }
 
 // After `niter` iterations without convergence: the stopping test on r_niter.
@@ -622,7 +692,14 @@ static size_t op_lds(const Model &m, int mode) {
 }
 
 template <int DIM, int MODE, bool NL, bool CM>
-static const void *op_fn_p(int path) {
+static const void *op_fn_p(int path, bool pre) {
+    if constexpr (MODE == OP_CG)
+        if (pre) switch (path) {
+                case 3: return reinterpret_cast<const void *>(&k_nm_op<DIM, 3, MODE, NL, 0, CM, true>);
+                case 2: return reinterpret_cast<const void *>(&k_nm_op<DIM, 2, MODE, NL, 0, CM, true>);
+                case 1: return reinterpret_cast<const void *>(&k_nm_op<DIM, 1, MODE, NL, 0, CM, true>);
+                default: return reinterpret_cast<const void *>(&k_nm_op<DIM, 0, MODE, NL, 0, CM, true>);
+            }
     switch (path) {
         case 3: return reinterpret_cast<const void *>(&k_nm_op<DIM, 3, MODE, NL, 0, CM>);
         case 2: return reinterpret_cast<const void *>(&k_nm_op<DIM, 2, MODE, NL, 0, CM>);
@@ -632,12 +709,22 @@ static const void *op_fn_p(int path) {
 }
 
 template <int DIM, int MODE>
-static const void *op_fn_t(int path, bool nl, bool cm) {
-    if (nl) return cm ? op_fn_p<DIM, MODE, true, true>(path) : op_fn_p<DIM, MODE, true, false>(path);
-    return cm ? op_fn_p<DIM, MODE, false, true>(path) : op_fn_p<DIM, MODE, false, false>(path);
+static const void *op_fn_t(int path, bool nl, bool cm, bool pre) {
+    if (nl) return cm ? op_fn_p<DIM, MODE, true, true>(path, pre) : op_fn_p<DIM, MODE, true, false>(path, pre);
+    return cm ? op_fn_p<DIM, MODE, false, true>(path, pre) : op_fn_p<DIM, MODE, false, false>(path, pre);
 }
 
 static const void *op_fn_sel(const Model &m, int mode, bool nl) {
+    const bool pre = m.tiles.one_pass;
+    if (pre && mode == OP_CG) switch (op_moc(m, mode)) {
+            case 168:
+                return nl ? reinterpret_cast<const void *>(&k_nm_op<3, 3, OP_CG, true, 168, false, true>)
+                          : reinterpret_cast<const void *>(&k_nm_op<3, 3, OP_CG, false, 168, false, true>);
+            case 336:
+                return nl ? reinterpret_cast<const void *>(&k_nm_op<3, 3, OP_CG, true, 336, false, true>)
+                          : reinterpret_cast<const void *>(&k_nm_op<3, 3, OP_CG, false, 336, false, true>);
+            default: break;
+        }
     switch (op_moc(m, mode) * (mode == OP_CG ? 1 : -1)) {
         case 168:
             return nl ? reinterpret_cast<const void *>(&k_nm_op<3, 3, OP_CG, true, 168>)
@@ -655,8 +742,10 @@ static const void *op_fn_sel(const Model &m, int mode, bool nl) {
     }
     const bool cm = !m.lumped;
     if (m.ndim == 3)
-        return mode == OP_CG ? op_fn_t<3, OP_CG>(m.elem_path, nl, cm) : op_fn_t<3, OP_RHS>(m.elem_path, nl, cm);
-    return mode == OP_CG ? op_fn_t<2, OP_CG>(m.elem_path, nl, cm) : op_fn_t<2, OP_RHS>(m.elem_path, nl, cm);
+        return mode == OP_CG ? op_fn_t<3, OP_CG>(m.elem_path, nl, cm, pre)
+                               : op_fn_t<3, OP_RHS>(m.elem_path, nl, cm, false);
+    return mode == OP_CG ? op_fn_t<2, OP_CG>(m.elem_path, nl, cm, pre)
+                           : op_fn_t<2, OP_RHS>(m.elem_path, nl, cm, false);
 }
 
 static const void *op_fn(const Model &m, int mode) {
@@ -726,45 +815,33 @@ static size_t cg_parts_size(const Model &m) { return 8 * size_t(m.tiles.ntiles) 
 // preconditioner (SVLG_PRECOND_LEARNED; beta = -z.q / p.q, Notay's FCG(1)). Per iteration:
 // one operator launch, one vector launch (plus the preconditioner's); the host polls the
 // done flag every 16 iterations.
-__global__ void k_iter_set(int *jdev, int j) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *jdev = j;
-}
-
-__global__ void k_iter_advance(int *jdev, int by) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *jdev += by;
-}
-
-// Launches of CG iteration j (jdev null: j is the iteration; else *jdev + j is, with j the
-// parity-fixed position inside a captured pair). p ping-pongs: even iterations stage
+// Launches of CG iteration j, of which the kernels use the parity (so a captured run of iterations
+// that starts at an even one is replayed for any). p ping-pongs: even iterations stage
 // p = z + beta cg_p[1] into cg_p[0], odd ones the reverse.
-static int cg_iteration(Model &m, const CgParts &c, OpArgs &a, double *x, int j, const int *jdev) {
+static int cg_iteration(Model &m, const CgParts &c, OpArgs &a, double *x, int j) {
     const int cur = (j & 1) ? 0 : 1;
     a.iter = j;
-    a.jdev = jdev;
     a.p_old = m.cg_p[cur].p;
     a.p_new = m.cg_p[1 - cur].p;
     if (int rc = launch_op(m, OP_CG, a)) return rc;
     hipLaunchKernelGGL(k_cg_update, dim3(kVecGrid), dim3(kVecBlock), 0, m.stream, m.ndofn, j, c, m.scal.p, x,
-                       m.cg_p[1 - cur].p, m.cg_q.p, m.cg_r.p, m.cg_z.p, m.jac.p, jdev,
+                       m.cg_p[1 - cur].p, m.cg_q.p, m.cg_r.p, m.cg_z.p, m.jac.p,
                        c.flexible ? gcn_input_args(m) : GcnInput{});
     if (c.flexible)
-        if (int rc = gcn_precond(m, c, j + 1, m.cg_r.p, m.cg_q.p, m.cg_z.p, jdev)) return rc;
+        if (int rc = gcn_precond(m, c, j + 1, m.cg_r.p, m.cg_q.p, m.cg_z.p)) return rc;
     return 0;
 }
 
-// The executable graph of `count` iterations *jdev .. *jdev + count - 1 (starting at an even
-// iteration) followed by *jdev += count, captured on first use for (x, flexible, operator
-// kernel, count).
+// The executable graph of `count` iterations starting at an even one, captured on first use for
+// (x, flexible, operator kernel, count).
 static hipGraphExec_t cg_run_graph(Model &m, const CgParts &c, const OpArgs &a0, double *x, int count) {
     const void *op = op_fn(m, OP_CG);
     for (auto &g : m.cg_graphs)
         if (g.x == x && g.flexible == c.flexible && g.op == op && g.count == count) return g.exec;
-    if (!m.jdev.p && m.jdev.alloc(1) != hipSuccess) return nullptr;
     if (hipStreamBeginCapture(m.stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
     OpArgs a = a0;
     int rc = 0;
-    for (int j = 0; j < count && rc == 0; ++j) rc = cg_iteration(m, c, a, x, j, m.jdev.p);
-    hipLaunchKernelGGL(k_iter_advance, dim3(1), dim3(64), 0, m.stream, m.jdev.p, count);
+    for (int j = 0; j < count && rc == 0; ++j) rc = cg_iteration(m, c, a, x, j);
     hipGraph_t g = nullptr;
     const hipError_t ec = hipStreamEndCapture(m.stream, &g);
     if (ec != hipSuccess || rc != 0 || !g) {
@@ -781,6 +858,28 @@ static hipGraphExec_t cg_run_graph(Model &m, const CgParts &c, const OpArgs &a0,
     }
     m.cg_graphs.push_back({exec, x, c.flexible, op, count});
     return exec;
+}
+
+// Reads the solver scalars back: a one-wave kernel writes them into pinned memory and the host
+// watches the poll's number there (a copy and a stream synchronisation took 25 us, and the
+// solve's follow-up launches wait for it). After 2 ms of watching the host sleeps in the
+// synchronisation instead, which also returns the stream's errors.
+static int cg_poll(Model &m) {
+    hipStream_t s = m.stream;
+    m.poll_seq += 1.0;
+    hipLaunchKernelGGL(k_cg_poll, dim3(1), dim3(64), 0, s, m.scal.p, m.poll_seq, m.scal_host);
+    SVLG_HIP(hipGetLastError());
+    const volatile double *seq = m.scal_host + SC_SEQ;
+    const auto t0 = std::chrono::steady_clock::now();
+    while (*seq != m.poll_seq) {
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+            SVLG_HIP(hipStreamSynchronize(s));
+            SVLG_CHECK(*seq == m.poll_seq, "the solver's scalars did not arrive");
+            break;
+        }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return 0;
 }
 
 int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int precond, int *iters, double *relres,
@@ -809,13 +908,13 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
     hipGraphExec_t pair = graph && maxit >= 2 ? cg_run_graph(m, c, a, x, 2) : nullptr;
     hipGraphExec_t run8 = pair && maxit >= 8 ? cg_run_graph(m, c, a, x, 8) : nullptr;
     hipGraphExec_t one = pair ? cg_run_graph(m, c, a, x, 1) : nullptr;
-    if (pair) hipLaunchKernelGGL(k_iter_set, dim3(1), dim3(64), 0, s, m.jdev.p, 0);
     // The polls copy the scalars into pinned host memory (a direct copy, no staging).
     if (!m.scal_host && hipHostMalloc((void **)&m.scal_host, sizeof(double) * SC_COUNT) != hipSuccess) {
         m.scal_host = nullptr;
         set_error("hipHostMalloc failed");
         return 10;
     }
+    if (m.poll_seq == 0.0) m.scal_host[SC_SEQ] = 0.0;
     double *hs = m.scal_host;
     int launched = 0;  // iterations 0 .. launched-1 are queued
     bool done = false;
@@ -834,7 +933,7 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
         // expected to see DONE: that iteration goes alone.
         const bool tail = det > 0 && launched == det - 1;
         if (pair && launched + 2 <= maxit && !tail) {
-            // The graphs start at even iterations: *jdev tracks `launched`. Runs of eight while
+            // The graphs start at even iterations. Runs of eight while
             // they stay within the prediction (every graph launch costs a few microseconds of
             // dispatch), then the rest of the prediction as one graph (captured on first use
             // for its count; after an odd count further iterations are launched eagerly), then
@@ -861,12 +960,11 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
             pair = nullptr;
         } else {
             if (pair) pair = nullptr;  // odd remainder: eager from here on
-            if (int rc = cg_iteration(m, c, a, x, launched, nullptr)) return rc;
+            if (int rc = cg_iteration(m, c, a, x, launched)) return rc;
             launched += 1;
         }
         if ((det > 0 && launched >= det) || (before >> 4) != (launched >> 4) || launched >= maxit) {
-            SVLG_HIP(hipMemcpyAsync(hs, m.scal.p, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost, s));
-            SVLG_HIP(hipStreamSynchronize(s));
+            if (int rc = cg_poll(m)) return rc;
             done = hs[SC_DONE] != 0.0;
         }
     }
@@ -874,8 +972,7 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
         // The stopping test on r_maxit, then the scalars.
         hipLaunchKernelGGL(k_cg_final, dim3(1), dim3(256), 0, s, launched, c, m.scal.p);
         SVLG_HIP(hipGetLastError());
-        SVLG_HIP(hipMemcpyAsync(hs, m.scal.p, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost, s));
-        SVLG_HIP(hipStreamSynchronize(s));
+        if (int rc = cg_poll(m)) return rc;
     }
     // The poll that saw DONE holds the final scalars (written with the flag); the work
     // queued after this call needs no further synchronisation.

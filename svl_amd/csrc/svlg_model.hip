@@ -609,9 +609,10 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
         UP(t.elem_lam, el.data(), el.size());
         UP(t.elem_mu, em.data(), em.size());
         UP(t.color_ptr, ht.color_ptr.data(), ht.color_ptr.size());
+        int hmax = 0;
+        for (int ti = 0; ti < ht.ntiles; ++ti) hmax = std::max(hmax, ht.halo_ptr[ti + 1] - ht.halo_ptr[ti]);
+        t.one_pass = m.variant == 3 && std::max(ht.max_own * ndim, hmax) <= 2 * t.block;
         if (m.variant == 3 && m.elem_path >= 2) {
-            int hmax = 0;
-            for (int ti = 0; ti < ht.ntiles; ++ti) hmax = std::max(hmax, ht.halo_ptr[ti + 1] - ht.halo_ptr[ti]);
             const int emax = ht.max_elem;
             // One staging pass of two block strides must cover the owned DOFs and the halo.
             if (std::max(ht.max_own * ndim, hmax) <= 2 * t.block && emax <= t.block && hmax > 0) {

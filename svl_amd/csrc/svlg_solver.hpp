@@ -20,6 +20,8 @@ enum {
     SC_ITERS,
     SC_TOL2,     // rtol^2
     SC_MAXIT,
+    SC_CNT,      // operator launches of the solve so far: the iteration index (kernels know its parity)
+    SC_SEQ,      // host copy only: the poll's number
     SC_COUNT = 16
 };
 
@@ -87,10 +89,6 @@ __device__ __forceinline__ void sum_records(const double *part, int count, int s
     reduce_records<K>(v, buf, out);
 }
 
-// Iteration index of a kernel launch: the launch's own index, plus the device-resident base
-// *jdev when the launch belongs to a replayed graph of iterations (jdev non-null).
-__device__ __forceinline__ int iter_of(const int *jdev, int j) { return jdev ? *jdev + j : j; }
-
 // Partial sums of one solve. Iteration j works on r_j, z_j, p_j, q_j = Keff p_j. Every kernel
 // writes its per-workgroup partials into the half of a ping-pong pair picked by the parity of
 // the iteration it produces, and the kernels that need a total re-sum the partials in
@@ -127,15 +125,14 @@ __device__ __forceinline__ void gcn_input(const GcnInput &g, int n, int i, doubl
 __device__ __forceinline__ void cg_vec(const CgParts &c, int j, double *buf, double (&o)[3]) {
     sum_records<3>(c.vp + size_t(j & 1) * 3 * c.nvb, c.nvb, 3, buf, o);
 }
-// CG's stopping test on r_j, j = iter_of(jdev, j0) (r.r <= rtol^2 b.b, or b = 0), from the
+// CG's stopping test on r_j, the iteration given by its parity (r.r <= rtol^2 b.b, or b = 0), from the
 // vector partials as the Jacobi solve's operator kernel applies it: the r.r and b.b sums are
 // bitwise cg_vec's components 1 and 2 (per-thread order and reduction tree of sum_records),
 // so every workgroup reaches the same answer. In the flexible solve this is the only test
 // (the operator kernel relies on it). Returns true (and the first workgroup records the scalars and DONE) if the
 // solve has converged, or if DONE was already set.
-__device__ __forceinline__ bool cg_stop_test(const CgParts &c, const int *jdev, int j0, double *scal, double *buf) {
+__device__ __forceinline__ bool cg_stop_test(const CgParts &c, int j, double *scal, double *buf) {
     const double flag = scal[SC_DONE];
-    const int j = iter_of(jdev, j0);
     if (flag != 0.0) return true;
     double v[2];
     sum_records<2>(c.vp + size_t(j & 1) * 3 * c.nvb + 1, c.nvb, 3, buf, v);
@@ -143,7 +140,7 @@ __device__ __forceinline__ bool cg_stop_test(const CgParts &c, const int *jdev, 
     if (done && blockIdx.x == 0 && threadIdx.x == 0) {
         scal[SC_RR] = v[0];
         scal[SC_BB] = v[1];
-        scal[SC_ITERS] = double(j);
+        scal[SC_ITERS] = scal[SC_CNT];
         scal[SC_DONE] = 1.0;
     }
     return done;
@@ -158,12 +155,11 @@ __device__ __forceinline__ void cg_pre(const CgParts &c, int j, double *buf, dou
 
 // Preconditioner hook of the flexible CG loop (svlg_gcn.hip): z = P(r) on the node-DOF
 // layout for iteration j (z = z_j; r = r_j; q = q_(j-1)) from the input layer the vector
-// kernel already formed (GcnInput); writes the tp[j&1] partials (z.r, z.q per tile). With
-// jdev the iteration is *jdev + j (graph replays). Its first layer applies the stopping test
+// kernel already formed (GcnInput); writes the tp[j&1] partials (z.r, z.q per tile). Of j the
+// kernels use the parity. Its first layer applies the stopping test
 // on r_j (cg_stop_test), so that a converged residual is not preconditioned: DONE is then set
 // one launch after the vector kernel of iteration j - 1.
-int gcn_precond(Model &m, const CgParts &c, int j, const double *r, const double *q, double *z,
-                const int *jdev = nullptr);
+int gcn_precond(Model &m, const CgParts &c, int j, const double *r, const double *q, double *z);
 // The input layer of the solver's preconditioner (x0, H^1 buffers and c_1).
 GcnInput gcn_input_args(Model &m);
 
