@@ -8,7 +8,7 @@
 // entry side by side); the free-space matrices T^T A T are summed per nonzero in
 // element order from a host-built contribution list (pure index work), and Keff is scaled
 // symmetrically by |diag|^-1/2. A step is one fused right-hand-side pass over the three
-// matrices, a MINRES solve of the scaled system (three kernels per iteration, the scalar
+// matrices, a MINRES solve of the scaled system (two kernels per iteration, the scalar
 // recurrence carried in device memory, convergence polled every few iterations) and the
 // Newmark update. Keff is indefinite (the stress blocks are negative definite), so CG does
 // not apply; SVL factorises it with Eigen (11-Solvers/EigenSolver.cpp).
@@ -24,12 +24,17 @@ namespace {
 constexpr int VB = 256;             // block of the vector and row kernels
 constexpr int MAXB = 1024;          // blocks of a reduction (partials per pass)
 constexpr int POLL = 8;             // MINRES iterations between convergence checks
-constexpr int LPR = 8;              // lanes per matrix row in the row kernels
+constexpr int RUN = 32;             // iterations of a replayed run while the prediction lasts
+constexpr int LPR = 8;              // lanes per matrix row in the right-hand-side kernel
+constexpr int LONG_ROW = 40;        // nonzeros per row from which the product takes 16 lanes
 constexpr double GA = 0.577350269189626;  // two-point Gauss abscissa (GaussQuadrature.cpp:303-316)
 
+// After the vector kernel of iteration j: the Lanczos coefficients alpha_j and beta_j, the two last
+// rotations and the residual estimate up to iteration j - 1 (beta_{j+1} is the norm of the vector
+// that the kernel made, whose partial sums the next one adds up).
 struct MrState {
-    double beta, cp, sp, c, s, eta, beta1;
-    int32_t done, iters, fail, pad;
+    double alpha, beta, cp, sp, c, s, eta, beta1;
+    int32_t done, iters, fail, started;
 };
 
 __host__ __device__ inline int class_nun(int cls) { return cls == 0 ? 2 : cls == 1 ? 5 : cls == 2 ? 3 : 9; }
@@ -293,33 +298,32 @@ __global__ void __launch_bounds__(VB) k_pml_scaled(int n, const int32_t *rowptr,
         for (int z = rowptr[i]; z < rowptr[i + 1]; ++z) vA[z] = S[i] * vE[z] * S[col[z]];
 }
 
-// Block sum of v into part[blockIdx.x] (deterministic tree).
-__device__ inline void block_sum(double v, double *part) {
-    __shared__ double sh[VB];
-    sh[threadIdx.x] = v;
+// Sums over a block: a shuffle tree inside each wave, then the waves in order (two barriers).
+template <int K>
+__device__ inline void block_sums(double (&v)[K]) {
+    __shared__ double sh[VB / 64][K];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_down(v[k], o, 64);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int k = 0; k < K; ++k) sh[threadIdx.x >> 6][k] = v[k];
     __syncthreads();
-    for (int o = VB / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-        __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        v[k] = sh[0][k];
+#pragma unroll
+        for (int w = 1; w < VB / 64; ++w) v[k] += sh[w][k];
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+    __syncthreads();
 }
 
-// Sum of the nb partials, the same value and order in every block.
-__device__ inline double reduce_parts(const double *part, int nb) {
-    __shared__ double sh[VB];
-    __shared__ double res;
-    double v = 0.0;
-    for (int t = threadIdx.x; t < nb; t += VB) v += part[t];
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = VB / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) res = sh[0];
-    __syncthreads();
-    return res;
+// Block sum of v into part[blockIdx.x] (deterministic order).
+__device__ inline void block_sum(double v, double *part) {
+    double a[1] = {v};
+    block_sums(a);
+    if (threadIdx.x == 0) part[blockIdx.x] = a[0];
 }
 
 struct RhsArgs {
@@ -358,107 +362,155 @@ __global__ void __launch_bounds__(VB) k_pml_rhs(RhsArgs a) {
     block_sum(acc, a.part);
 }
 
-__global__ void __launch_bounds__(VB) k_mr_init(int n, int nb, const double *part, const double *r, double *v,
-                                                double *vprev, double *w, double *wprev, double *x, double rtol,
-                                                MrState *st) {
-    const double beta1 = sqrt(reduce_parts(part, nb));
-    const double inv = beta1 > 0.0 ? 1.0 / beta1 : 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        v[i] = r[i] * inv;
-        vprev[i] = 0.0;
-        w[i] = 0.0;
-        wprev[i] = 0.0;
-        x[i] = 0.0;
-    }
+// u_1 = r (in place), the other vectors zero; the first vector kernel finds beta_1^2 in its sums.
+__global__ void __launch_bounds__(VB) k_mr_init(int n, int nbr, int nb, const double *part, double *vprev, double *w,
+                                                double *wprev, double *x, double *part2, MrState *st) {
+    double a[1] = {0.0};
+    for (int t = threadIdx.x; t < nbr; t += VB) a[0] += part[t];
+    block_sums(a);
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        vprev[i] = w[i] = wprev[i] = x[i] = 0.0;
+    if (threadIdx.x == 0) part2[blockIdx.x] = blockIdx.x == 0 ? a[0] : 0.0;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const double beta1 = sqrt(a[0]);
         MrState s{};
-        s.beta = 0.0; s.cp = 1.0; s.sp = 0.0; s.c = 1.0; s.s = 0.0; s.eta = beta1; s.beta1 = beta1;
+        s.cp = 1.0; s.c = 1.0; s.eta = beta1; s.beta1 = beta1;
         s.done = beta1 == 0.0 ? 1 : 0;
-        s.iters = 0;
-        s.fail = 0;
         st[0] = s;
         st[1] = s;
     }
 }
 
-// MINRES (Paige-Saunders) iteration, part 1: Av = A v and the partials of v.Av; LPR lanes
-// per row stride through its nonzeros and combine by shuffles.
-
+// MINRES (Paige-Saunders), iteration j, in two kernels on Lanczos vectors that are normalised where they
+// are used: u_j with beta_j = |u_j|, v_j = u_j / beta_j. The product kernel needs no scalar (t = A
+// u_j and the partials of u_j.t = alpha_j beta_j^2), and everything elementwise fits one
+// kernel: the next Lanczos vector, and the rotation, direction and iterate of iteration
+// j - 1, whose beta_j has just become known. Three kernels (product, Lanczos vector, rotation) took
+// 13.6 us per iteration on 28,073 unknowns (2D) and 27.1 on 41,586 (3D), most of it launches,
+// partial sums and dependent loads; these take 8.5 and 15.6 (9.2 and 20.0 with one nonzero of a lane
+// in flight).
+// Product: LANES lanes per row stride through its nonzeros and combine by shuffles.
+template <int LANES>
 __global__ void __launch_bounds__(VB) k_mr_spmv(int n, const int32_t *rowptr, const int32_t *col, const double *vA,
-                                                const double *v, double *Av, double *part, const MrState *st) {
-    if (st->done) return;
+                                                const double *u, double *t, double *part, const MrState *st) {
+    constexpr int NF = 4;  // in flight per lane (6 are no faster)
     double acc = 0.0;
-    const int lane = threadIdx.x % LPR;
-    const int64_t nthr = (int64_t)n * LPR;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t - lane < nthr;
-         t += (int64_t)gridDim.x * blockDim.x) {
-        const int i = (int)(t / LPR);
+    const int lane = threadIdx.x % LANES;
+    const int64_t nthr = (int64_t)n * LANES, step = (int64_t)gridDim.x * blockDim.x;
+    int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // The first row's bounds are loaded beside the done flag, and a lane's nonzeros NF at a time
+    // (entries past the row: factor 0 on the row's own column), so that a row is three
+    // dependent round trips, not two for every nonzero of a lane.
+    int z0 = 0, z1 = 0;
+    if (k < nthr) {
+        z0 = rowptr[k / LANES];
+        z1 = rowptr[k / LANES + 1];
+    }
+    if (st->done) return;
+    for (; k - lane < nthr; k += step) {
+        const int i = (int)(k / LANES);
         double s = 0.0;
-        if (i < n)
-            for (int z = rowptr[i] + lane; z < rowptr[i + 1]; z += LPR) s += vA[z] * v[col[z]];
-        for (int o = LPR / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LPR);
-        if (lane == 0 && i < n) {
-            Av[i] = s;
-            acc += v[i] * s;
+        for (int z = z0 + lane; z < z1; z += NF * LANES) {
+            int c[NF];
+            double f[NF];
+#pragma unroll
+            for (int m = 0; m < NF; ++m) {
+                const int y = z + m * LANES;
+                c[m] = y < z1 ? col[y] : i;
+                f[m] = y < z1 ? vA[y] : 0.0;
+            }
+#pragma unroll
+            for (int m = 0; m < NF; ++m) s += f[m] * u[c[m]];
+        }
+        if (k + step < nthr) {
+            z0 = rowptr[(k + step) / LANES];
+            z1 = rowptr[(k + step) / LANES + 1];
+        }
+#pragma unroll
+        for (int o = LANES / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, LANES);
+        if (lane == 0) {
+            t[i] = s;
+            acc += u[i] * s;
         }
     }
     block_sum(acc, part);
 }
 
-// Part 2: the Lanczos vector Av - alpha v - beta vprev (in Av) and the partials of its square.
-__global__ void __launch_bounds__(VB) k_mr_lanczos(int n, int nbs, const double *part1, const double *v,
-                                                   const double *vprev, double *Av, double *part2, const MrState *st) {
-    if (st->done) return;
-    const double alpha = reduce_parts(part1, nbs), beta = st->beta;
-    double acc = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double u = Av[i] - alpha * v[i] - beta * vprev[i];
-        Av[i] = u;
-        acc += u * u;
-    }
-    block_sum(acc, part2);
-}
-
-// Part 3: the Givens rotations, the new search direction (into wprev's buffer), the iterate,
-// and the normalised Lanczos vector (into vprev's buffer); the host then swaps the pairs.
-// Block 0 writes the scalar state of the next iteration into the other slot.
-__global__ void __launch_bounds__(VB) k_mr_update(int n, int nbs, int nb, const double *part1, const double *part2,
-                                                  const double *v, double *vprev, const double *Av, const double *w,
-                                                  double *wprev, double *x, double rtol, const MrState *st,
-                                                  MrState *nxt) {
+// Vector kernel of iteration j: beta_j from part2 (nb partials), alpha_j from part1 (nbs), then per
+// entry x and the direction of iteration j - 1 (into wprev's buffer; the host swaps the pair),
+// v_j (into v_{j-1}'s place) and u_{j+1} (into u_j's place) with its partials in part2n. Block 0
+// writes the next state.
+__global__ void __launch_bounds__(VB) k_mr_vec(int n, int nbs, int nb, const double *part1, const double *part2,
+                                               double *part2n, double *u, const double *t, double *v,
+                                               const double *w, double *wprev, double *x, double rtol,
+                                               const MrState *st, MrState *nxt) {
+    // The first entry's loads go out before the sums.
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    double ui = 0, ti = 0, vi = 0, wi = 0, pi = 0, xi = 0;
+    auto load = [&] {
+        ui = u[i];
+        ti = t[i];
+        vi = v[i];
+        wi = w[i];
+        pi = wprev[i];
+        xi = x[i];
+    };
+    if (i < n) load();
+    double a[2] = {0.0, 0.0};
+    for (int k = threadIdx.x; k < nbs; k += VB) a[0] += part1[k];
+    for (int k = threadIdx.x; k < nb; k += VB) a[1] += part2[k];
     const MrState s = *st;
     if (s.done) {
         if (blockIdx.x == 0 && threadIdx.x == 0) *nxt = s;
         return;
     }
-    const double alpha = reduce_parts(part1, nbs), bn = sqrt(reduce_parts(part2, nb));
-    const double eps = s.sp * s.beta, dtmp = s.cp * s.beta;
-    const double delta = s.c * dtmp + s.s * alpha, gt = -s.s * dtmp + s.c * alpha;
-    const double gam = hypot(gt, bn);
-    if (gam == 0.0) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            MrState f = s;
-            f.done = 1;
-            f.fail = 1;
-            *nxt = f;
+    block_sums(a);
+    MrState q = s;
+    const double beta = sqrt(a[1]), ib = beta > 0.0 ? 1.0 / beta : 0.0, alpha = a[0] * ib * ib;
+    // Iteration j - 1: rotations and step.
+    double delta = 0.0, eps = 0.0, ig = 0.0, step = 0.0;
+    if (s.started) {
+        eps = s.sp * s.beta;
+        const double dtmp = s.cp * s.beta;
+        delta = s.c * dtmp + s.s * s.alpha;
+        const double gt = -s.s * dtmp + s.c * s.alpha, gam = hypot(gt, beta);
+        if (gam == 0.0) {
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+                q.done = 1;
+                q.fail = 1;
+                *nxt = q;
+            }
+            return;
         }
-        return;
+        ig = 1.0 / gam;
+        q.cp = s.c;
+        q.sp = s.s;
+        q.c = gt / gam;
+        q.s = beta / gam;
+        step = q.c * s.eta;
+        q.eta = -q.s * s.eta;
+        q.iters = s.iters + 1;
+        q.done = (fabs(q.eta) <= rtol * s.beta1 || beta == 0.0) ? 1 : 0;
     }
-    const double cn = gt / gam, sn = bn / gam, step = cn * s.eta, ig = 1.0 / gam;
-    const double ib = bn > 0.0 ? 1.0 / bn : 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const double wn = (v[i] - delta * w[i] - eps * wprev[i]) * ig;
-        x[i] += step * wn;
-        wprev[i] = wn;
-        vprev[i] = Av[i] * ib;
+    q.alpha = alpha;
+    q.beta = beta;
+    q.started = 1;
+    double acc = 0.0;
+    while (i < n) {
+        if (s.started) {
+            const double wn = (vi - delta * wi - eps * pi) * ig;
+            x[i] = xi + step * wn;
+            wprev[i] = wn;
+        }
+        const double vn = ui * ib, un = ti * ib - alpha * vn - beta * vi;
+        v[i] = vn;
+        u[i] = un;
+        acc += un * un;
+        i += gridDim.x * blockDim.x;
+        if (i < n) load();
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        MrState t = s;
-        t.beta = bn; t.cp = s.c; t.sp = s.s; t.c = cn; t.s = sn; t.eta = -sn * s.eta;
-        t.iters = s.iters + 1;
-        t.done = (fabs(t.eta) <= rtol * s.beta1 || bn == 0.0) ? 1 : 0;
-        *nxt = t;
-    }
+    block_sum(acc, part2n);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *nxt = q;
 }
 
 // dU = S x, then ExtendedNewmarkBeta's update (ExtendedNewmarkBeta.cpp:123-154):
@@ -516,59 +568,63 @@ using namespace svlg;
 
 struct svlg_pml {
     hipStream_t stream = nullptr;
-    int nfree = 0, ntot = 0, nnodes = 0, nelem = 0, nb = 1, nbs = 1, nt = 0, maxit = 0;
+    int nfree = 0, ntot = 0, nnodes = 0, nelem = 0, nb = 1, nbs = 1, nbr = 1, nt = 0, maxit = 0;
     int64_t nnz = 0, ncontrib = 0;
     double dt = 0, rtol = 0, c0 = 0, c1 = 0, c2 = 0, c3 = 0;
     bool has_g = false;  // a PML3DHexa8 element: history matrix G and Ubar
     DevBuf<int32_t> rowptr, col, lptr, lrow, dfree;
     DevBuf<double> dfac, lfac, series;
-    DevBuf<double> vM, vC, vK, vG, vA, S, U, V, A, Ub, r, x, Av, vb0, vb1, wb0, wb1, part0, part1, part2;
+    DevBuf<double> vM, vC, vK, vG, vA, S, U, V, A, Ub, r, x, t, v, wb0, wb1, part0, part1, part2;
+    int lanes = 8;                   // lanes per row of the product
     DevBuf<MrState> st;
     MrState *hst = nullptr;  // pinned copy of the polled state
     int last_iters = 0;              // MINRES iterations of the previous solve
     bool use_graph = true;           // replay the batches from a captured graph (else eager)
     hipGraphExec_t batch = nullptr;  // POLL iterations, captured once (the buffer pairs swap
                                      // every iteration, so an even batch ends where it began)
+    hipGraphExec_t run = nullptr;    // RUN iterations
     ~svlg_pml() {
         if (batch) (void)hipGraphExecDestroy(batch);
+        if (run) (void)hipGraphExecDestroy(run);
         if (hst) (void)hipHostFree(hst);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
 
-static_assert(POLL % 2 == 0, "a batch must end with the buffer pairs where it began");
+static_assert(POLL % 2 == 0 && RUN % 2 == 0, "a batch must end with the buffer pairs where it began");
 
-// POLL MINRES iterations starting from slot 0 and the buffer pairs (vb0, vb1), (wb0, wb1).
-static void launch_batch(svlg_pml *p, hipStream_t s) {
+// `count` (even) MINRES iterations starting from state slot 0, the first half of part2 and (wb0, wb1).
+static void launch_batch(svlg_pml *p, hipStream_t s, int count) {
     const int n = p->nfree, nb = p->nb, nbs = p->nbs;
-    double *v = p->vb0.p, *vp = p->vb1.p, *w = p->wb0.p, *wp = p->wb1.p;
-    for (int j = 0; j < POLL; ++j) {
+    double *w = p->wb0.p, *wp = p->wb1.p;
+    for (int j = 0; j < count; ++j) {
         const MrState *cur = p->st.p + (j & 1);
         MrState *nxt = p->st.p + ((j + 1) & 1);
-        hipLaunchKernelGGL(k_mr_spmv, dim3(nbs), dim3(VB), 0, s, n, p->rowptr.p, p->col.p, p->vA.p, v, p->Av.p,
-                           p->part1.p, cur);
-        hipLaunchKernelGGL(k_mr_lanczos, dim3(nb), dim3(VB), 0, s, n, nbs, p->part1.p, v, vp, p->Av.p, p->part2.p,
-                           cur);
-        hipLaunchKernelGGL(k_mr_update, dim3(nb), dim3(VB), 0, s, n, nbs, nb, p->part1.p, p->part2.p, v, vp, p->Av.p,
-                           w, wp, p->x.p, p->rtol, cur, nxt);
-        std::swap(v, vp);
+        double *p2 = p->part2.p + (j & 1) * MAXB, *p2n = p->part2.p + ((j + 1) & 1) * MAXB;
+        if (p->lanes == 16)
+            hipLaunchKernelGGL(k_mr_spmv<16>, dim3(nbs), dim3(VB), 0, s, n, p->rowptr.p, p->col.p, p->vA.p, p->r.p,
+                               p->t.p, p->part1.p, cur);
+        else
+            hipLaunchKernelGGL(k_mr_spmv<8>, dim3(nbs), dim3(VB), 0, s, n, p->rowptr.p, p->col.p, p->vA.p, p->r.p,
+                               p->t.p, p->part1.p, cur);
+        hipLaunchKernelGGL(k_mr_vec, dim3(nb), dim3(VB), 0, s, n, nbs, nb, p->part1.p, p2, p2n, p->r.p, p->t.p,
+                           p->v.p, w, wp, p->x.p, p->rtol, cur, nxt);
         std::swap(w, wp);
     }
 }
 
 // Host-side checks of what launch_batch bakes into its launches (and a captured graph keeps):
-// grids within [1, MAXB] blocks of VB threads, static LDS only (block_sum / reduce_parts: VB
-// doubles plus one), and every pointer a live allocation of this handle of the sizes the
-// kernels index (vectors nfree, partials MAXB, two scalar slots, the CSR arrays).
+// grids within [1, MAXB] blocks of VB threads, static LDS only (block_sums: a few
+// doubles per wave), and every pointer a live allocation of this handle of the sizes the
+// kernels index (vectors nfree, partials MAXB and twice MAXB, two scalar slots, the CSR arrays).
 static int check_batch(const svlg_pml *p) {
     SVLG_CHECK(p->nb >= 1 && p->nb <= MAXB && p->nbs >= 1 && p->nbs <= MAXB, "MINRES grid out of range");
-    SVLG_CHECK((int64_t)p->nbs * VB >= std::min<int64_t>((int64_t)p->nfree * LPR, (int64_t)MAXB * VB) &&
+    SVLG_CHECK((int64_t)p->nbs * VB >= std::min<int64_t>((int64_t)p->nfree * p->lanes, (int64_t)MAXB * VB) &&
                    (int64_t)p->nb * VB >= std::min<int64_t>(p->nfree, (int64_t)MAXB * VB),
                "MINRES grid does not cover the rows");
-    const DevBuf<double> *vec[] = {&p->vb0, &p->vb1, &p->wb0, &p->wb1, &p->x, &p->Av};
+    const DevBuf<double> *vec[] = {&p->r, &p->t, &p->v, &p->wb0, &p->wb1, &p->x};
     for (const DevBuf<double> *b : vec) SVLG_CHECK(b->p && b->n == (size_t)p->nfree, "MINRES vector not allocated");
-    SVLG_CHECK(p->part1.p && p->part1.n >= (size_t)std::max(p->nb, p->nbs) && p->part2.p &&
-                   p->part2.n >= (size_t)std::max(p->nb, p->nbs),
+    SVLG_CHECK(p->part1.p && p->part1.n >= (size_t)p->nbs && p->part2.p && p->part2.n == (size_t)2 * MAXB,
                "MINRES partials not allocated");
     SVLG_CHECK(p->st.p && p->st.n == 2, "MINRES state slots not allocated");
     SVLG_CHECK(p->rowptr.p && p->rowptr.n == (size_t)p->nfree + 1 && p->col.p && p->col.n == (size_t)p->nnz &&
@@ -577,20 +633,22 @@ static int check_batch(const svlg_pml *p) {
     return 0;
 }
 
-// Captures launch_batch into a graph; on any capture error the caller launches eagerly.
-static void capture_batch(svlg_pml *p) {
+// Captures `count` iterations into a graph; on any capture error the caller launches eagerly.
+static hipGraphExec_t capture_batch(svlg_pml *p, int count) {
     hipGraph_t g = nullptr;
-    if (hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return;
-    launch_batch(p, p->stream);
+    hipGraphExec_t exec = nullptr;
+    if (hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
+    launch_batch(p, p->stream, count);
     const hipError_t ec = hipStreamEndCapture(p->stream, &g);
     if (ec != hipSuccess || !g) {
         if (g) (void)hipGraphDestroy(g);
         (void)hipGetLastError();
-        return;
+        return nullptr;
     }
-    if (hipGraphInstantiate(&p->batch, g, nullptr, nullptr, 0) != hipSuccess) p->batch = nullptr;
+    if (hipGraphInstantiate(&exec, g, nullptr, nullptr, 0) != hipSuccess) exec = nullptr;
     (void)hipGraphDestroy(g);
     (void)hipGetLastError();
+    return exec;
 }
 
 extern "C" {
@@ -711,7 +769,9 @@ int svlg_pml_create(const svlg_mixed_desc *d, double dt, double rtol, int32_t ma
     p->c0 = 4.0 / (dt * dt); p->c1 = 2.0 / dt; p->c2 = 4.0 / dt; p->c3 = dt / 3.0;
     p->has_g = has_g;
     p->nb = blocks_for(nfree);
-    p->nbs = blocks_for((int64_t)nfree * LPR);
+    p->lanes = p->nnz >= (int64_t)LONG_ROW * nfree ? 16 : 8;
+    p->nbs = blocks_for((int64_t)nfree * p->lanes);
+    p->nbr = blocks_for((int64_t)nfree * LPR);
     p->nt = d->nload ? d->load_nt : 0;
     if (hipStreamCreate(&p->stream) != hipSuccess) { set_error("hipStreamCreate failed"); return fail(10); }
     if (hipHostMalloc((void **)&p->hst, sizeof(MrState)) != hipSuccess) { set_error("hipHostMalloc failed"); return fail(10); }
@@ -748,7 +808,7 @@ int svlg_pml_create(const svlg_mixed_desc *d, double dt, double rtol, int32_t ma
     if (p->nt) UP(p->series, d->load_series, (size_t)d->nload * p->nt);
 #undef UP
     int32_t zero = 0;
-    DevBuf<double> *vecs[] = {&p->S, &p->U, &p->V, &p->A, &p->r, &p->x, &p->Av, &p->vb0, &p->vb1, &p->wb0, &p->wb1};
+    DevBuf<double> *vecs[] = {&p->S, &p->U, &p->V, &p->A, &p->r, &p->x, &p->t, &p->v, &p->wb0, &p->wb1};
     for (DevBuf<double> *b : vecs)
         if (b->alloc(nfree) != hipSuccess) { set_error("device allocation failed"); return fail(10); }
     DevBuf<double> *mats[] = {&p->vM, &p->vC, &p->vK, &p->vA};
@@ -760,7 +820,7 @@ int svlg_pml_create(const svlg_mixed_desc *d, double dt, double rtol, int32_t ma
     }
     const int64_t nent = eoff[ne];
     if (p->part0.alloc(MAXB) != hipSuccess || p->part1.alloc(MAXB) != hipSuccess ||
-        p->part2.alloc(MAXB) != hipSuccess || p->st.alloc(2) != hipSuccess || emat.alloc((size_t)4 * nent) != hipSuccess ||
+        p->part2.alloc(2 * MAXB) != hipSuccess || p->st.alloc(2) != hipSuccess || emat.alloc((size_t)4 * nent) != hipSuccess ||
         bad.upload(&zero, 1, s) != hipSuccess) {
         set_error("device allocation failed");
         return fail(10);
@@ -825,26 +885,36 @@ int svlg_pml_steps(svlg_pml *p, int32_t k0, int32_t nsteps, int32_t nrec, const 
         SVLG_HIP(hist.alloc(3 * hsz));
     }
     if (int rc = check_batch(p)) return rc;
-    if (p->use_graph && !p->batch) capture_batch(p);
+    if (p->use_graph && !p->batch) p->batch = capture_batch(p, POLL);
     RhsArgs ra{n, 0, p->nt, p->rowptr.p, p->col.p, p->lptr.p, p->lrow.p, p->vM.p, p->vC.p, p->vK.p,
                p->has_g ? p->vG.p : nullptr, p->lfac.p, p->series.p, p->S.p, p->U.p, p->V.p, p->A.p,
                p->has_g ? p->Ub.p : nullptr, p->c2, p->dt, p->r.p, p->part0.p};
     for (int st = 0; st < nsteps; ++st) {
         ra.k = k0 + st;
-        hipLaunchKernelGGL(k_pml_rhs, dim3(p->nbs), dim3(VB), 0, s, ra);
-        hipLaunchKernelGGL(k_mr_init, dim3(nb), dim3(VB), 0, s, n, p->nbs, p->part0.p, p->r.p, p->vb0.p, p->vb1.p,
-                           p->wb0.p, p->wb1.p, p->x.p, p->rtol, p->st.p);
+        hipLaunchKernelGGL(k_pml_rhs, dim3(p->nbr), dim3(VB), 0, s, ra);
+        hipLaunchKernelGGL(k_mr_init, dim3(nb), dim3(VB), 0, s, n, p->nbr, nb, p->part0.p, p->v.p, p->wb0.p,
+                           p->wb1.p, p->x.p, p->part2.p, p->st.p);
         // Batches of POLL iterations; once converged the remaining launches of a batch return
-        // at once. A batch ends in slot 0 with the buffer pairs back in place.
+        // at once. A batch ends in slot 0 with the buffer pairs back in place. (Convergence in
+        // iteration j shows in the vector kernel of iteration j + 1.)
         // The batches the previous solve needed, less one, go out before the first poll
-        // (steps of a linear analysis converge in nearly the same number of iterations).
-        for (int b = 1; b < p->last_iters / POLL; ++b) {
+        // (steps of a linear analysis converge in nearly the same number of iterations), RUN
+        // iterations to a graph while they last (a replay costs some microseconds of its own).
+        int ahead = std::max(0, (p->last_iters + 1) / POLL - 1) * POLL;
+        if (p->use_graph && p->batch && !p->run && ahead >= RUN) p->run = capture_batch(p, RUN);
+        while (ahead > 0) {
+            if (p->run && p->batch && ahead >= RUN) {
+                SVLG_HIP(hipGraphLaunch(p->run, s));
+                ahead -= RUN;
+                continue;
+            }
             if (p->batch) SVLG_HIP(hipGraphLaunch(p->batch, s));
-            else launch_batch(p, s);
+            else launch_batch(p, s, POLL);
+            ahead -= POLL;
         }
         for (;;) {
             if (p->batch) SVLG_HIP(hipGraphLaunch(p->batch, s));
-            else launch_batch(p, s);
+            else launch_batch(p, s, POLL);
             SVLG_HIP(hipGetLastError());
             SVLG_HIP(hipMemcpyAsync(p->hst, p->st.p, sizeof(MrState), hipMemcpyDeviceToHost, s));
             SVLG_HIP(hipStreamSynchronize(s));
@@ -878,6 +948,10 @@ int svlg_pml_set_graph(svlg_pml *p, int32_t on) {
     if (!on && p->batch) {
         SVLG_HIP(hipGraphExecDestroy(p->batch));
         p->batch = nullptr;
+    }
+    if (!on && p->run) {
+        SVLG_HIP(hipGraphExecDestroy(p->run));
+        p->run = nullptr;
     }
     p->use_graph = on != 0;
     return 0;
