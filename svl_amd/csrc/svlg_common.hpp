@@ -219,6 +219,7 @@ struct Model {
     // the operator, rs alone and am for the right-hand side.
     DevBuf<double> cmass_keff, cmass_rhs, cmass_am;
     DevBuf<double> cg_r, cg_z, cg_q, cg_b, cg_p[2];
+    DevBuf<double> cg_s[2];           // one-kernel iterations: Keff p (empty for J2 models)
     DevBuf<double> part;              // partial sums of a solve (CgParts)
     DevBuf<double> scal;              // device scalars of the solver
     int cg_last_iters[2] = {0, 0};    // iterations of the last solve (Jacobi, flexible)

@@ -392,6 +392,192 @@ __global__ __launch_bounds__(512) void k_nm_op(OpArgs a) {
     }
 }
 
+// Operands of the one-kernel iteration: r, w = Keff z and s = Keff p go from one half of their pairs to
+// the other (neighbours read the old ones while the owners write), p and x stay in place.
+struct OneArgs {
+    const double *r0, *w0, *s0;
+    double *r1, *w1, *s1, *p, *x;
+    double *tp;   // [2][ntiles][3] partials (r.z, w.z, r.r) by parity
+    int start;    // 1: w = Keff (jac r0) and its partials; p and s are cleared (beta_0 = 0 multiplies them)
+};
+
+// One Jacobi-PCG iteration in one kernel (Chronopoulos and Gear's arrangement: with w = Keff z,
+//   beta = g / g_old, alpha = g / (w.z - beta g / alpha_old), g = r.z,
+//   p = z + beta p, s = w + beta s, x += alpha p, r -= alpha s, z = jac r, w = Keff z),
+// so that all of an iteration's sums are behind one kernel boundary. The tile forms z of its halo
+// itself from the neighbours' old r, w and s (jac is a read more), which are in flight, like
+// every owned operand, while the sums arrive. The two-kernel iteration (operator, then vectors) is
+// bound by its two launches and two chains of sums, not by bytes (the vectors moved are about the
+// same): 41x37x29 block 16.8 -> 14.0 us per iteration, Quad4 60x35 12.5 -> 8.8. J2 models keep
+// two kernels: their branches follow the last bits of a solve.
+// Tiles whose owned DOFs and halo take two strides of the block at most.
+template <int DIM, int PATH, int MOC, bool CM>
+__global__ __launch_bounds__(512) void k_cg_one(OpArgs a, OneArgs o) {
+    constexpr int NEN = Elem<DIM>::nen, NS = 2;
+    constexpr bool STAGE_X = PATH < 2;
+    extern __shared__ double smem[];
+    __shared__ double red[3 * 17];
+    const int nt = a.ntiles, j = a.iter;
+    const int bI = blockIdx.x, xcd = bI & 7, jb = bI >> 3;
+    const int q = nt >> 3, r8 = nt & 7;
+    const int tile = xcd * q + min(xcd, r8) + jb;
+    const int o0 = a.own_ptr[tile], nown = a.own_ptr[tile + 1] - o0;
+    const int h0 = a.halo_ptr[tile], nh = a.halo_ptr[tile + 1] - h0;
+    const int e0 = a.elem_ptr[tile], ne = a.elem_ptr[tile + 1] - e0;
+    const int MS = a.max_stage, MO = MOC > 0 ? MOC + 1 : a.max_own;
+    double *sU = smem, *sX = smem + size_t(MS) * DIM, *sIn = smem + size_t((STAGE_X ? 2 : 1) * MS) * DIM;
+    const int tid = threadIdx.x, B = blockDim.x;
+    const size_t g0 = size_t(o0) * DIM;
+    const double flag = a.scal[SC_DONE], tol2 = a.scal[SC_TOL2], bb = a.scal[SC_BB];
+    const double g_old = a.scal[SC_ONE + 2 * ((j + 1) & 1)], al_old = a.scal[SC_ONE + 2 * ((j + 1) & 1) + 1];
+    const bool has_elem = tid < ne;
+    int lc[NEN];
+    double lam = 0.0, mu = 0.0;
+    int gid = 0;
+    if (has_elem) {
+        const uint16_t *l = a.lconn + size_t(e0 + tid) * NEN;
+#pragma unroll
+        for (int c = 0; c < NEN; ++c) lc[c] = l[c];
+        const double cf = a.coef[e0 + tid];
+        lam = a.elam[e0 + tid] * cf;
+        mu = a.emu[e0 + tid] * cf;
+        if constexpr (PATH >= 2) gid = a.egeo[e0 + tid];
+    } else {
+#pragma unroll
+        for (int c = 0; c < NEN; ++c) lc[c] = 0;
+    }
+    int hn[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) hn[k] = k * B + tid < nh ? a.halo_node[h0 + k * B + tid] : 0;
+    double ro[NS], wo[NS], so[NS], po[NS], xo[NS], jo[NS];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const int i = k * B + tid;
+        const bool in = i < nown * DIM;
+        ro[k] = in ? o.r0[g0 + i] : 0.0;
+        jo[k] = in ? a.jac[g0 + i] : 0.0;
+        wo[k] = in && !o.start ? o.w0[g0 + i] : 0.0;
+        so[k] = in && !o.start ? o.s0[g0 + i] : 0.0;
+        po[k] = in && !o.start ? o.p[g0 + i] : 0.0;
+        xo[k] = in && !o.start ? o.x[g0 + i] : 0.0;
+    }
+    double rh[NS][DIM], wh[NS][DIM], sh[NS][DIM], jh[NS][DIM];
+#pragma unroll
+    for (int k = 0; k < NS; ++k)
+#pragma unroll
+        for (int c = 0; c < DIM; ++c) {
+            const bool in = k * B + tid < nh;
+            const size_t g = size_t(hn[k]) * DIM + c;
+            rh[k][c] = in ? o.r0[g] : 0.0;
+            jh[k][c] = in ? a.jac[g] : 0.0;
+            wh[k][c] = in && !o.start ? o.w0[g] : 0.0;
+            sh[k][c] = in && !o.start ? o.s0[g] : 0.0;
+        }
+    double alpha = 0.0, beta = 0.0;
+    if (!o.start) {
+        double v[3];
+        sum_records<3>(o.tp + size_t(j & 1) * 3 * nt, nt, 3, red, v);
+        if (flag != 0.0) return;
+        const bool done = v[2] <= tol2 * bb || bb == 0.0;
+        beta = g_old != 0.0 ? v[0] / g_old : 0.0;
+        const double den = al_old != 0.0 ? v[1] - beta * v[0] / al_old : v[1];
+        alpha = den != 0.0 ? v[0] / den : 0.0;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            a.scal[SC_RR] = v[2];
+            const double cnt = a.scal[SC_CNT];
+            a.scal[SC_ITERS] = cnt;
+            if (!done) a.scal[SC_CNT] = cnt + 1.0;
+            a.scal[SC_ONE + 2 * (j & 1)] = v[0];
+            a.scal[SC_ONE + 2 * (j & 1) + 1] = alpha;
+            if (done) a.scal[SC_DONE] = 1.0;
+        }
+        if (done) return;
+    }
+    double acc[3] = {0.0, 0.0, 0.0};  // r.z, w.z, r.r
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const int i = k * B + tid;
+        if (i < nown * DIM) {
+            const size_t g = g0 + i;
+            double r = ro[k];
+            if (!o.start) {
+                const double p = jo[k] * ro[k] + beta * po[k], s = wo[k] + beta * so[k];
+                r = ro[k] - alpha * s;
+                o.p[g] = p;
+                o.s1[g] = s;
+                o.x[g] = xo[k] + alpha * p;
+                o.r1[g] = r;
+            } else {
+                o.p[g] = 0.0;
+                o.s1[g] = 0.0;
+            }
+            const double z = jo[k] * r;
+            sU[i] = z;
+            acc[0] += r * z;
+            acc[2] += r * r;
+            if constexpr (STAGE_X) sX[i] = a.X[g];
+        }
+        if (i < nh)
+#pragma unroll
+            for (int c = 0; c < DIM; ++c) {
+                const double s = wh[k][c] + beta * sh[k][c];
+                sU[(nown + i) * DIM + c] = jh[k][c] * (rh[k][c] - alpha * s);
+                if constexpr (STAGE_X) sX[(nown + i) * DIM + c] = a.X[size_t(hn[k]) * DIM + c];
+            }
+    }
+    for (int i = tid; i < NEN * DIM * MO; i += B) sIn[i] = 0.0;
+    __syncthreads();
+    if (has_elem) {
+        double u[NEN][DIM], f[NEN][DIM];
+#pragma unroll
+        for (int c = 0; c < NEN; ++c)
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) u[c][d] = sU[lc[c] * DIM + d];
+        tile_elem_force<DIM, PATH>(a.geo, a.th, lc, sX, lam, mu, gid, u, f);
+        if constexpr (CM) tile_elem_mass<DIM, PATH>(lc, sX, a.cmass[e0 + tid], u, f);
+#pragma unroll
+        for (int c = 0; c < NEN; ++c) {
+            if constexpr (MOC > 0) {
+                const int col = lc[c] < nown ? lc[c] : MOC;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) sIn[(c * DIM + d) * MO + col] = f[c][d];
+            } else if (lc[c] < nown) {
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) sIn[(c * DIM + d) * MO + lc[c]] = f[c][d];
+            }
+        }
+    }
+    __syncthreads();
+    if (tid < nown) {
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+            double fi = 0.0;
+#pragma unroll
+            for (int c = 0; c < NEN; ++c) fi += sIn[(c * DIM + d) * MO + tid];
+            const size_t g = g0 + size_t(tid) * DIM + d;
+            const double z = sU[tid * DIM + d];
+            const double w = a.jac[g] != 0.0 ? fi + a.dgn[g] * z : 0.0;
+            o.w1[g] = w;
+            acc[1] += w * z;
+        }
+    }
+    double tot[3];
+    reduce_records<3>(acc, red, tot);
+    if (tid == 0) {
+        double *t = o.tp + size_t(o.start ? j & 1 : (j + 1) & 1) * 3 * nt + 3 * tile;
+        t[0] = tot[0];
+        t[1] = tot[1];
+        t[2] = tot[2];
+    }
+}
+
+// b.b of a solve from the init kernel's partials, for the one-kernel iterations.
+__global__ __launch_bounds__(256) void k_cg_bb(CgParts c, double *scal) {
+    __shared__ double red[17];
+    const double bb = sum_partials(c.ip, c.nvb, 1, red);
+    if (threadIdx.x == 0) scal[SC_BB] = bb;
+}
+
 __global__ void k_solver_reset(double *scal, double tol2, double maxit) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         for (int i = 0; i < SC_COUNT; ++i) scal[i] = 0.0;
@@ -525,11 +711,17 @@ __global__ void k_cg_poll(const double *__restrict__ scal, double seq, double *h
 }
 
 // After `niter` iterations without convergence: the stopping test on r_niter.
-__global__ __launch_bounds__(256) void k_cg_final(int niter, CgParts c, double *scal) {
+__global__ __launch_bounds__(256) void k_cg_final(int niter, CgParts c, int one, double *scal) {
     __shared__ double red[3 * 17];
     if (scal[SC_DONE] != 0.0) return;
     double v[3];
-    cg_vec(c, niter, red, v);
+    if (one) {
+        sum_records<3>(c.tp + size_t(niter & 1) * 3 * c.ntiles, c.ntiles, 3, red, v);
+        v[1] = v[2];
+        v[2] = scal[SC_BB];
+    } else {
+        cg_vec(c, niter, red, v);
+    }
     if (threadIdx.x == 0) {
         scal[SC_RR] = v[1];
         scal[SC_BB] = v[2];
@@ -756,6 +948,47 @@ static const void *op_fn(const Model &m, int mode) {
     return op_fn_sel(m, mode, nl);
 }
 
+template <int DIM, bool CM>
+static const void *one_fn_t(int path) {
+    switch (path) {
+        case 3: return reinterpret_cast<const void *>(&k_cg_one<DIM, 3, 0, CM>);
+        case 2: return reinterpret_cast<const void *>(&k_cg_one<DIM, 2, 0, CM>);
+        case 1: return reinterpret_cast<const void *>(&k_cg_one<DIM, 1, 0, CM>);
+        default: return reinterpret_cast<const void *>(&k_cg_one<DIM, 0, 0, CM>);
+    }
+}
+
+static const void *one_fn(const Model &m) {
+    switch (op_moc(m, OP_CG)) {
+        case 168: return reinterpret_cast<const void *>(&k_cg_one<3, 3, 168, false>);
+        case 336: return reinterpret_cast<const void *>(&k_cg_one<3, 3, 336, false>);
+        default: break;
+    }
+    const bool cm = !m.lumped;
+    if (m.ndim == 3) return cm ? one_fn_t<3, true>(m.elem_path) : one_fn_t<3, false>(m.elem_path);
+    return cm ? one_fn_t<2, true>(m.elem_path) : one_fn_t<2, false>(m.elem_path);
+}
+
+// Whether Jacobi solves of the model take the one-kernel iteration. Every tile adds up every tile's
+// three partials, so the line is at the tiles where that costs what the second launch does
+// (microseconds per iteration, two kernels against one: 43 tiles 12.5 -> 8.8, 384 tiles 16.8 ->
+// 14.0, 1,021 tiles 40.2 both, 2,188 tiles 48.9 -> 69.8).
+static bool use_one(const Model &m) { return !m.has_j2 && m.tiles.one_pass && m.tiles.ntiles <= 768; }
+
+// One-kernel iteration j (start: the product and sums of z_0 alone, into the halves that iteration 0
+// reads). r, w, s: buffers 0 to 1 on even iterations and back on odd ones.
+static int launch_one(Model &m, const OpArgs &a0, const CgParts &c, double *x, int j, bool start) {
+    OpArgs a = a0;
+    a.iter = j;
+    if (!m.lumped) a.cmass = m.cmass_keff.p;
+    const int in = j & 1, out = start ? in : 1 - in;
+    double *r[2] = {m.cg_r.p, m.cg_z.p}, *w[2] = {m.cg_q.p, m.cg_p[1].p}, *sv[2] = {m.cg_s[0].p, m.cg_s[1].p};
+    OneArgs o{r[in], w[in], sv[in], r[out], w[out], sv[out], m.cg_p[0].p, x, c.tp, start ? 1 : 0};
+    void *args[] = {&a, &o};
+    SVLG_HIP(hipLaunchKernel(one_fn(m), dim3(m.tiles.ntiles), dim3(m.tiles.block), args, op_lds(m, OP_CG), m.stream));
+    return 0;
+}
+
 static int launch_op(Model &m, int mode, const OpArgs &a0) {
     OpArgs a = a0;
     if (!m.lumped) {
@@ -819,6 +1052,7 @@ static size_t cg_parts_size(const Model &m) { return 8 * size_t(m.tiles.ntiles) 
 // that starts at an even one is replayed for any). p ping-pongs: even iterations stage
 // p = z + beta cg_p[1] into cg_p[0], odd ones the reverse.
 static int cg_iteration(Model &m, const CgParts &c, OpArgs &a, double *x, int j) {
+    if (!c.flexible && use_one(m)) return launch_one(m, a, c, x, j, false);
     const int cur = (j & 1) ? 0 : 1;
     a.iter = j;
     a.p_old = m.cg_p[cur].p;
@@ -835,7 +1069,7 @@ static int cg_iteration(Model &m, const CgParts &c, OpArgs &a, double *x, int j)
 // The executable graph of `count` iterations starting at an even one, captured on first use for
 // (x, flexible, operator kernel, count).
 static hipGraphExec_t cg_run_graph(Model &m, const CgParts &c, const OpArgs &a0, double *x, int count) {
-    const void *op = op_fn(m, OP_CG);
+    const void *op = !c.flexible && use_one(m) ? one_fn(m) : op_fn(m, OP_CG);
     for (auto &g : m.cg_graphs)
         if (g.x == x && g.flexible == c.flexible && g.op == op && g.count == count) return g.exec;
     if (hipStreamBeginCapture(m.stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
@@ -905,6 +1139,11 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
         if (int rc = gcn_precond(m, c, 0, m.cg_r.p, m.cg_q.p, m.cg_z.p)) return rc;
     a.z = m.cg_z.p;
     a.reduce = 1;
+    const bool one_kernel = !flexible && use_one(m);
+    if (one_kernel) {
+        hipLaunchKernelGGL(k_cg_bb, dim3(1), dim3(256), 0, s, c, m.scal.p);
+        if (int rc = launch_one(m, a, c, x, 0, true)) return rc;
+    }
     hipGraphExec_t pair = graph && maxit >= 2 ? cg_run_graph(m, c, a, x, 2) : nullptr;
     hipGraphExec_t run8 = pair && maxit >= 8 ? cg_run_graph(m, c, a, x, 8) : nullptr;
     hipGraphExec_t one = pair ? cg_run_graph(m, c, a, x, 1) : nullptr;
@@ -970,7 +1209,7 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
     }
     if (!done) {
         // The stopping test on r_maxit, then the scalars.
-        hipLaunchKernelGGL(k_cg_final, dim3(1), dim3(256), 0, s, launched, c, m.scal.p);
+        hipLaunchKernelGGL(k_cg_final, dim3(1), dim3(256), 0, s, launched, c, one_kernel ? 1 : 0, m.scal.p);
         SVLG_HIP(hipGetLastError());
         if (int rc = cg_poll(m)) return rc;
     }
@@ -1045,6 +1284,15 @@ int svlg_nm_init(svlg_model *h, double dt, double rtol, int32_t maxit, int32_t p
                               &m.cg_p[0], &m.cg_p[1]}) {
         SVLG_HIP(b->alloc(n));
         SVLG_HIP(hipMemsetAsync(b->p, 0, sizeof(double) * n, s));
+    }
+    if (use_one(m)) {
+        for (DevBuf<double> &b : m.cg_s) {
+            SVLG_HIP(b.alloc(n));
+            SVLG_HIP(hipMemsetAsync(b.p, 0, sizeof(double) * n, s));
+        }
+        if (op_lds(m, OP_CG) > 64 * 1024)
+            SVLG_HIP(hipFuncSetAttribute(one_fn(m), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         int(op_lds(m, OP_CG))));
     }
     if (m.sm_ndofs > 0) {
         for (DevBuf<double> *b : {&m.sm_vec, &m.sm_y}) {

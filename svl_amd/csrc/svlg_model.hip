@@ -328,7 +328,7 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     m.th = d->thickness;
     m.lumped = d->lumped != 0;
     m.affine = all_affine(ndim, ne, nen, d->conn, d->coords);
-    int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : default_tile_nodes(ndim, nn, m.affine, any_j2);
+    int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : 0;  // 0: chosen below
     int block = (o && o->block > 0) ? o->block : 512;
     const int req_variant = (o && o->variant > 0) ? o->variant : 0;
     if (req_variant < 0 || req_variant > 3) { set_error("variant must be 0 (auto), 1, 2 or 3"); return fail(11); }
@@ -351,6 +351,8 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
         if (d->ray_ak) ak[e] = d->ray_ak[e];
         if (ak[e] != 0.0) m.has_ak = true;
     }
+    const bool auto_tiles = tile_nodes == 0;
+    if (auto_tiles) tile_nodes = default_tile_nodes(ndim, nn, m.affine, any_j2, m.has_ak && m.lumped);
     // Nodes that need the general update.
     std::vector<uint8_t> special(nn, 0);
     for (int n = 0; n < nn; ++n)
@@ -378,6 +380,13 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     HostTiles ht;
     try {
         make_tiles(ndim, nn, ne, nen, d->coords, d->conn, m.h_color.data(), m.ncolors, special.data(), tile_nodes, ht);
+        // Sizes of the library's choice must leave the corner-slot kernels possible where the
+        // smaller tiles did (512 elements a tile; flat or long tiles touch more).
+        const int safe = ndim == 3 ? 160 : 192;
+        if (auto_tiles && !any_j2 && tile_nodes > safe && ht.ntiles > 1 && std::max(ht.max_elem, ht.max_own) > 512) {
+            ht = HostTiles();
+            make_tiles(ndim, nn, ne, nen, d->coords, d->conn, m.h_color.data(), m.ncolors, special.data(), safe, ht);
+        }
     } catch (const std::exception &ex) {
         set_error(std::string("tiling failed: ") + ex.what());
         return fail(11);
@@ -778,12 +787,14 @@ int svlg_plan_tiles(const svlg_mesh_desc *d, int32_t tile_nodes, int64_t *stats)
     }
     bool has_j2 = false;
     for (int e = 0; d->mat_type && e < ne; ++e) has_j2 |= d->mat_type[e] == SVLG_MAT_J2;
+    bool has_ak = false;
+    for (int e = 0; d->ray_ak && e < ne; ++e) has_ak |= d->ray_ak[e] != 0.0;
     HostTiles t;
     try {
         make_tiles(ndim, nn, ne, nen, d->coords, d->conn, color.data(), ncolors, special.data(),
                    tile_nodes > 0 ? tile_nodes
                                   : default_tile_nodes(ndim, nn, all_affine(ndim, ne, nen, d->conn, d->coords),
-                                                       has_j2),
+                                                       has_j2, has_ak && d->lumped != 0),
                    t);
     } catch (const std::exception &ex) {
         set_error(std::string("tiling failed: ") + ex.what());

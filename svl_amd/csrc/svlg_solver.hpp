@@ -22,7 +22,8 @@ enum {
     SC_MAXIT,
     SC_CNT,      // operator launches of the solve so far: the iteration index (kernels know its parity)
     SC_SEQ,      // host copy only: the poll's number
-    SC_COUNT = 16
+    SC_ONE,      // one-kernel iterations: r.z and alpha of the even and of the odd iteration before
+    SC_COUNT = SC_ONE + 4
 };
 
 // Deterministic sum over a workgroup (blockDim a multiple of 64, at most 1024): a fixed

@@ -164,3 +164,42 @@ def test_newmark_rejects_unsupported_models():
     with pytest.raises(SvlgError):
         newmark(dm, 1e-3)
     dm.close()
+
+
+@pytest.mark.parametrize("kind,tile_nodes", [("quad", 448), ("quad", 16), ("quad_consistent", 40), ("hexa", 0),
+                                             ("hexa", 16), ("hexa_consistent", 0), ("distorted", 40),
+                                             ("many_tiles", 16), ("many_tiles", 24)])
+def test_cg_iteration_kernels(kind, tile_nodes):
+    """Jacobi solves of the one-kernel iteration (up to 768 tiles) and of the two-kernel one (`many_tiles`
+    with 16 nodes: above): the true residual, recomputed by Keff apply, meets the tolerance up to the
+    recurrence's round-off (iterations x eps x the norms' ratio, far below 1e-12 here), a zero right-hand
+    side gives zero, and a second solve is bitwise the first."""
+    from svl_amd.integrators import LinearSystem
+    if kind.startswith("quad"):
+        m, dt, nt = W.realization2d(33, 19, 4, nt=11)
+        am, ak = W.rayleigh(0.05, 1.0, 10.0)
+        m.ray_am, m.ray_ak = np.full(m.nelem, am), np.full(m.nelem, ak)
+    elif kind == "distorted":
+        from _meshes import block_model
+        m = block_model(9, 8, 7, distort=0.15, seed=2)[0]
+    elif kind == "many_tiles":
+        m, dt, nt = W.block3d_implicit(26, 22, 20, nt=11)
+    else:
+        m, dt, nt = W.block3d_implicit(9, 7, 8, nt=11)
+    m.massform_lumped = not kind.endswith("consistent")
+    dm = DeviceModel(m, tile_nodes=tile_nodes)
+    if kind == "many_tiles":
+        assert (dm.info()["ntiles"] > 768) == (tile_nodes == 16)
+    nm = ExtendedNewmarkBeta(dm, 2e-3, rtol=1e-11, maxit=2000)
+    nm.Initialize()
+    ls = LinearSystem(nm)
+    b = np.random.default_rng(5).standard_normal(m.nfree)
+    ls.SetVector(b)
+    assert not ls.SolveSystem()
+    x = ls.GetSolution().copy()
+    assert ls.iters > 0 and ls.relres <= 1e-11
+    assert np.linalg.norm(b - ls.Apply(x)) / np.linalg.norm(b) < 1.1e-11
+    assert not ls.SolveSystem() and np.array_equal(ls.GetSolution(), x)
+    ls.SetVector(np.zeros(m.nfree))
+    assert not ls.SolveSystem() and not ls.GetSolution().any() and ls.iters == 0
+    dm.close()
