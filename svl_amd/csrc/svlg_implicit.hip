@@ -59,6 +59,8 @@ struct OpArgs {
     double *scal;
     CgParts cg;
     int reduce;           // OP_CG: 1 = iteration `iter` of a solve (beta, stopping test, p.q partials)
+    int reset;            // OP_CG, reduce 0: 1 = first launch of a solve, set the solver's scalars
+    double tol2, maxit;   // their values
     int iter;
     // OP_RHS
     const double *U, *V, *A, *mdiag, *cdiag;
@@ -183,6 +185,8 @@ __global__ __launch_bounds__(512) void k_nm_op(OpArgs a) {
     }
     double beta = 0.0;
     if constexpr (!RHS) {
+        if (a.reset && blockIdx.x == 0 && tid < SC_COUNT)
+            a.scal[tid] = tid == SC_TOL2 ? a.tol2 : tid == SC_MAXIT ? a.maxit : 0.0;
         if (a.reduce) {
             if (flag != 0.0) return;
             const int j = a.iter;
@@ -398,6 +402,8 @@ struct OneArgs {
     const double *r0, *w0, *s0;
     double *r1, *w1, *s1, *p, *x;
     double *tp;   // [2][ntiles][3] partials (r.z, w.z, r.r) by parity
+    const double *ip;  // [nvb] b.b partials (start: the first workgroup leaves their sum in scal)
+    int nvb;
     int start;    // 1: w = Keff (jac r0) and its partials; p and s are cleared (beta_0 = 0 multiplies them)
 };
 
@@ -563,19 +569,16 @@ __global__ __launch_bounds__(512) void k_cg_one(OpArgs a, OneArgs o) {
     }
     double tot[3];
     reduce_records<3>(acc, red, tot);
+    if (o.start && blockIdx.x == 0) {
+        const double b2 = sum_partials(o.ip, o.nvb, 1, red);
+        if (tid == 0) a.scal[SC_BB] = b2;
+    }
     if (tid == 0) {
         double *t = o.tp + size_t(o.start ? j & 1 : (j + 1) & 1) * 3 * nt + 3 * tile;
         t[0] = tot[0];
         t[1] = tot[1];
         t[2] = tot[2];
     }
-}
-
-// b.b of a solve from the init kernel's partials, for the one-kernel iterations.
-__global__ __launch_bounds__(256) void k_cg_bb(CgParts c, double *scal) {
-    __shared__ double red[17];
-    const double bb = sum_partials(c.ip, c.nvb, 1, red);
-    if (threadIdx.x == 0) scal[SC_BB] = bb;
 }
 
 __global__ void k_solver_reset(double *scal, double tol2, double maxit) {
@@ -983,7 +986,7 @@ static int launch_one(Model &m, const OpArgs &a0, const CgParts &c, double *x, i
     if (!m.lumped) a.cmass = m.cmass_keff.p;
     const int in = j & 1, out = start ? in : 1 - in;
     double *r[2] = {m.cg_r.p, m.cg_z.p}, *w[2] = {m.cg_q.p, m.cg_p[1].p}, *sv[2] = {m.cg_s[0].p, m.cg_s[1].p};
-    OneArgs o{r[in], w[in], sv[in], r[out], w[out], sv[out], m.cg_p[0].p, x, c.tp, start ? 1 : 0};
+    OneArgs o{r[in], w[in], sv[in], r[out], w[out], sv[out], m.cg_p[0].p, x, c.tp, c.ip, c.nvb, start ? 1 : 0};
     void *args[] = {&a, &o};
     SVLG_HIP(hipLaunchKernel(one_fn(m), dim3(m.tiles.ntiles), dim3(m.tiles.block), args, op_lds(m, OP_CG), m.stream));
     return 0;
@@ -1122,7 +1125,6 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
     const int n = m.ndofn;
     const int flexible = precond == SVLG_PRECOND_LEARNED ? 1 : 0;
     const CgParts c = cg_parts(m, flexible);
-    hipLaunchKernelGGL(k_solver_reset, dim3(1), dim3(64), 0, s, m.scal.p, rtol * rtol, double(maxit));
     OpArgs a = op_args(m);
     a.coef = m.coef_keff.p;
     a.cg = c;
@@ -1132,7 +1134,11 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
     a.p_old = x;
     a.p_new = m.cg_p[1].p;
     a.reduce = 0;
+    a.reset = 1;
+    a.tol2 = rtol * rtol;
+    a.maxit = double(maxit);
     if (int rc = launch_op(m, OP_CG, a)) return rc;
+    a.reset = 0;
     hipLaunchKernelGGL(k_cg_init, dim3(kVecGrid), dim3(kVecBlock), 0, s, n, c, b, m.cg_q.p, m.jac.p, m.cg_r.p,
                        m.cg_z.p, flexible ? gcn_input_args(m) : GcnInput{});
     if (flexible)
@@ -1141,7 +1147,6 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
     a.reduce = 1;
     const bool one_kernel = !flexible && use_one(m);
     if (one_kernel) {
-        hipLaunchKernelGGL(k_cg_bb, dim3(1), dim3(256), 0, s, c, m.scal.p);
         if (int rc = launch_one(m, a, c, x, 0, true)) return rc;
     }
     hipGraphExec_t pair = graph && maxit >= 2 ? cg_run_graph(m, c, a, x, 2) : nullptr;
