@@ -166,8 +166,8 @@ def layer2d_bench(args):
     from svl_amd.integrators import CentralDifference, DeviceModel
     steps = args.layer_steps
     m, dt, nt = W.layer2d(200, 100, nt=steps + args.warmup + 2)
-    # 20,301 nodes: the default 448-node tiles give 51 workgroups for 256 CUs, so the tile
-    # size is picked by the autotuner (timed fused steps per candidate).
+    # 20,301 nodes: the tile size sets the workgroups (256 CUs) and the borders that they recompute;
+    # it is picked by the autotuner (timed steps per candidate).
     tile, tune = B.autotune_tile_nodes(m, [0, m.nnodes], [dt], candidates=(24, 32, 48, 64, 96, 128, 192, 448),
                                        steps=50)
     dm = DeviceModel(m, tile_nodes=tile)

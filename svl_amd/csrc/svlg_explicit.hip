@@ -1060,8 +1060,8 @@ static int cd_passes(const Model &m) {
 }
 
 // Owned-node bound of the compile-time slot stride of the corner-slot step on axis-aligned
-// meshes (0: the stride read from the tile set): 160 (the default 3D tile size) for Hexa8,
-// 192 and 448 (the batched and the default 2D tile sizes) for Quad4.
+// meshes (0: the stride read from the tile set): 160 (the large default 3D tiles) for Hexa8, for Quad4
+// 192 (the default above a million nodes) and 448 (covers the 400-node default).
 static int use_moc(const Model &m) {
     if (m.variant != 3 || m.elem_bf16 || m.elem_path != 3) return 0;
     if (m.elem_fp32) return m.tiles.max_own <= 160 ? 160 : 0;
@@ -1250,7 +1250,7 @@ static const void *multi_fn(const Model &m) {
 // Below a chip full of workgroups the launch is saved and the recomputed rings are free; above
 // it they compete with the tiles: in 2D the state's bytes still pay for them while a tile is
 // large against its rings and up to about a million nodes, in 3D never. Gauss-point hexahedra
-// (2,600 operations an element) recompute nothing.
+// (1,300 operations an element) recompute nothing.
 static int multi_depth(const Model &m) {
     const int nt = m.tiles.ntiles, own = m.nnodes / nt;
     if (nt == 1) return 1;

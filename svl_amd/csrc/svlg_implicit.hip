@@ -414,7 +414,7 @@ struct OneArgs {
 // itself from the neighbours' old r, w and s (jac is a read more), which are in flight, like
 // every owned operand, while the sums arrive. The two-kernel iteration (operator, then vectors) is
 // bound by its two launches and two chains of sums, not by bytes (the vectors moved are about the
-// same): 41x37x29 block 16.8 -> 14.0 us per iteration, Quad4 60x35 12.5 -> 8.8. J2 models keep
+// same): 41x37x29 block 16.8 -> 13.8 us per iteration, Quad4 60x35 12.5 -> 8.2. J2 models keep
 // two kernels: their branches follow the last bits of a solve.
 // Tiles whose owned DOFs and halo take two strides of the block at most.
 template <int DIM, int PATH, int MOC, bool CM>
@@ -974,8 +974,8 @@ static const void *one_fn(const Model &m) {
 
 // Whether Jacobi solves of the model take the one-kernel iteration. Every tile adds up every tile's
 // three partials, so the line is at the tiles where that costs what the second launch does
-// (microseconds per iteration, two kernels against one: 43 tiles 12.5 -> 8.8, 384 tiles 16.8 ->
-// 14.0, 1,021 tiles 40.2 both, 2,188 tiles 48.9 -> 69.8).
+// (microseconds per iteration, two kernels against one: 43 tiles 12.5 -> 8.2, 384 tiles 16.8 ->
+// 13.8, 1,021 tiles 40.2 both, 2,188 tiles 48.9 -> 69.8).
 static bool use_one(const Model &m) { return !m.has_j2 && m.tiles.one_pass && m.tiles.ntiles <= 768; }
 
 // One-kernel iteration j (start: the product and sums of z_0 alone, into the halves that iteration 0
