@@ -34,11 +34,19 @@ template <class T>
 struct DevBuf {
     T *p = nullptr;
     size_t n = 0;
+    // After a refused allocation the buffer is empty (n = 0), so that a caller who keeps buffers and
+    // grows them by n never launches on a null pointer.
     hipError_t alloc(size_t count) {
         release();
-        n = count;
         if (count == 0) return hipSuccess;
-        return hipMalloc((void **)&p, count * sizeof(T));
+        const hipError_t e = hipMalloc((void **)&p, count * sizeof(T));
+        if (e == hipSuccess) {
+            n = count;
+        } else {
+            p = nullptr;
+            (void)hipGetLastError();  // reported here, not by the next call's launch check
+        }
+        return e;
     }
     hipError_t upload(const T *h, size_t count, hipStream_t s) {
         hipError_t e = alloc(count);

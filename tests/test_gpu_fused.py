@@ -252,3 +252,21 @@ def test_multi_step_kernel(kind):
         amp = np.linalg.norm(state[0]) / (h * np.linalg.norm(b))
         assert rel_l2(a, b) < 1e-12 * max(1.0, amp), f
     ref.close()
+
+
+def test_recording_after_a_refused_history():
+    """A history larger than the card (400 GB; the caller's array is not reached) is refused, and the
+    next recording of the model starts from an allocation of its own: the same history as a fresh model's."""
+    from svl_amd import _capi as capi
+    m, dt = _multi_model("quad_one_tile")
+    rec = np.arange(0, m.nfree, 5, dtype=np.int32)
+    dm = DeviceModel(m)
+    cd = CentralDifference(dm, dt)
+    cd.Initialize()
+    want = cd.advance(1, 40, rec)
+    cd.Initialize()
+    many = np.resize(rec, 50000).astype(np.int32)
+    hist = np.zeros(1)
+    assert capi.lib().svlg_cd_steps(dm.h, 1, 1000000, many.size, capi.iptr(many), capi.fptr(hist)) != 0
+    assert np.array_equal(cd.advance(1, 40, rec), want)
+    dm.close()
