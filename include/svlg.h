@@ -179,7 +179,9 @@ int svlg_cd_init(svlg_model *m, double dt, double ftol);
 int svlg_cd_steps(svlg_model *m, int32_t k0, int32_t nsteps, int32_t nrec,
                   const int32_t *rec_dofs, double *hist);
 /* Same as svlg_cd_steps but leaves results on the device and returns immediately
- * after enqueueing (no recording, no host synchronisation). */
+ * after enqueueing (no recording, no host synchronisation). A caller may capture it into a
+ * graph of its own (a multiple of 3 steps, the period of the U ring): replays and eager steps, the
+ * latter again in multiples of 3, then advance the same state until the next svlg_cd_init. */
 int svlg_cd_steps_async(svlg_model *m, int32_t k0, int32_t nsteps);
 /* Current U, V, A in free DOFs (CentralDifference::GetDisplacements/Velocities/
  * Accelerations). Any pointer may be NULL. */

@@ -182,6 +182,7 @@ struct Model {
     MultiSet multi;
     bool auto_variant = false;        // the kernels were chosen by the library, not by the caller
     bool multi_tried = false;
+    bool captured = false;            // the caller has captured explicit steps since svlg_cd_init
     bool corner_unique = false;       // every (node, corner position) pair belongs to at most one element
     std::vector<int32_t> h_conn;      // [nelem*nen] connectivity in device numbering
     std::vector<int32_t> h_own_ptr;   // [ntiles+1]

@@ -1428,16 +1428,19 @@ static int cd_one_step(Model &m, int k, const RecRef *rec = nullptr) {
     return 0;
 }
 
-// Whether steps go through the multi-step kernel: a plan exists, and the stream is not being
-// captured by the caller (the launches exchange buffers, which a replay would not repeat).
-static bool multi_ready(const Model &m) {
-    if (m.multi.depth == 0) return false;
+// Whether steps go through the multi-step kernel: a plan exists, and the caller has not captured steps
+// since the last initialisation. Its launches exchange buffers with the state's ring, which a
+// replay would not repeat, and a graph captured before would go on in buffers that are no longer the state:
+// from the first capture on, every step is a single step inside the ring's three buffers.
+static bool multi_ready(Model &m) {
+    if (m.multi.depth == 0 || m.captured) return false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(m.stream, &st) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
-    return st == hipStreamCaptureStatusNone;
+    m.captured = st != hipStreamCaptureStatusNone;
+    return !m.captured;
 }
 
 // nsteps steps from k0, recording into rec (map null: nothing).
@@ -1471,6 +1474,7 @@ static int cd_init_impl(Model &m, double dt, const std::vector<double> *dtd, dou
     m.dt = dt;
     m.ftol = ftol;
     m.cd_ready = false;
+    m.captured = false;  // the state's buffers are new: graphs of the caller end here
     if (int rc = multi_setup(m)) return rc;
     if (m.cd_graph) {
         (void)hipGraphExecDestroy(m.cd_graph);

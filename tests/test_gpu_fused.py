@@ -270,3 +270,42 @@ def test_recording_after_a_refused_history():
     assert capi.lib().svlg_cd_steps(dm.h, 1, 1000000, many.size, capi.iptr(many), capi.fptr(hist)) != 0
     assert np.array_equal(cd.advance(1, 40, rec), want)
     dm.close()
+
+
+def test_caller_captured_steps_and_eager_steps():
+    """Three steps captured by the caller (past the end of the load series, so that every replay is the
+    same work), replayed between eager steps of both kernels' lengths: the state is that of as many
+    eager steps (the captured and the later steps are single steps: 1e-12, as test_multi_step_kernel)."""
+    import torch
+    m, dt = _multi_model("quad_tiles")
+    nt = m.load_series.shape[1]
+    ref = DeviceModel(m)
+    cr = CentralDifference(ref, dt)
+    cr.Initialize()
+    cr.advance(1, nt - 1 + 30)
+    want = [cr.GetDisplacements(), cr.GetVelocities(), cr.GetAccelerations()]
+    ref.close()
+    dm = DeviceModel(m)
+    stream = torch.cuda.Stream()
+    dm.set_stream(stream.cuda_stream)
+    cd = CentralDifference(dm, dt)
+    cd.Initialize()
+    cd.advance(1, nt - 1)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        cd.advance_async(nt, 3)
+    stream.synchronize()
+    for eager in (6, 3, 9):
+        with torch.cuda.stream(stream):
+            graph.replay()
+        cd.advance_async(nt, eager)
+    with torch.cuda.stream(stream):
+        graph.replay()
+    dm.sync()
+    got = [cd.GetDisplacements(), cd.GetVelocities(), cd.GetAccelerations()]
+    for f, (a, b, h) in enumerate(zip(got, want, (1.0, dt, dt * dt))):
+        amp = np.linalg.norm(want[0]) / (h * np.linalg.norm(b))
+        assert rel_l2(a, b) < 1e-12 * max(1.0, amp), f
+    dm.set_stream(None)
+    dm.close()
+    del graph
