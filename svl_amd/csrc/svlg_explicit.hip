@@ -1262,9 +1262,7 @@ static int multi_depth(const Model &m) {
 }
 
 // The multi-step plan of a model that steps one tile per workgroup with kernels of the library's choice.
-static int multi_setup(Model &m) {
-    if (m.multi_tried) return 0;
-    m.multi_tried = true;
+static int multi_build(Model &m) {
     MultiSet &t = m.multi;
     std::vector<int32_t> conn, own;
     std::vector<uint8_t> special;
@@ -1318,7 +1316,13 @@ static int multi_setup(Model &m) {
         em[i] = e >= 0 ? mu[e] * sc : 0.0;
         eg[i] = e >= 0 && m.elem_path >= 2 ? gid[e] : uint16_t(0);
     }
-    SVLG_HIP(t.slab.alloc(total));
+    if (t.slab.alloc(total) != hipSuccess || t.U[0].alloc(m.ndofn) != hipSuccess ||
+        t.U[1].alloc(m.ndofn) != hipSuccess) {
+        t.slab.release();
+        t.U[0].release();
+        t.U[1].release();
+        return 0;
+    }
     SVLG_HIP(hipMemcpyAsync(t.slab.p, slab.get(), total, hipMemcpyHostToDevice, s));
     SVLG_HIP(hipStreamSynchronize(s));
     t.cnt = reinterpret_cast<const int32_t *>(t.slab.p + o_cnt);
@@ -1328,17 +1332,27 @@ static int multi_setup(Model &m) {
     t.egeo = reinterpret_cast<const uint16_t *>(t.slab.p + o_egeo);
     t.elam = reinterpret_cast<const double *>(t.slab.p + o_lam);
     t.emu = reinterpret_cast<const double *>(t.slab.p + o_mu);
-    for (int i = 0; i < 2; ++i) SVLG_HIP(t.U[i].alloc(m.ndofn));
     t.ntiles = h.ntiles;
     t.ns = h.ns;
     t.ne = h.ne;
     t.nu = h.nu;
     t.block = cls.block;
     t.lds_bytes = lds;
-    t.depth = depth;
     if (lds > 64 * 1024)
         SVLG_HIP(hipFuncSetAttribute(multi_fn(m), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+    t.depth = depth;
     return 0;
+}
+
+// The plan saves time only: where host or device memory does not hold it, the model steps singly.
+static int multi_setup(Model &m) {
+    if (m.multi_tried) return 0;
+    m.multi_tried = true;
+    try {
+        return multi_build(m);
+    } catch (const std::bad_alloc &) {
+        return 0;
+    }
 }
 
 // n steps from k in one launch (n <= depth, or one tile); last: the caller reads the state next,

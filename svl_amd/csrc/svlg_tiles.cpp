@@ -11,6 +11,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
+#include <exception>
+#include <new>
 #include <numeric>
 #include <stdexcept>
 #include <thread>
@@ -174,15 +176,27 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
     };
     std::vector<Tile> tiles(nt);
     // Tiles are independent: a few host threads take them in turn (the result does not depend on
-    // which thread built a tile).
+    // which thread built a tile). Threads that the system refuses are done without; an allocation
+    // refused inside a worker ends the plan, not the process.
     const int nthr = std::max(1, std::min({12, int(std::thread::hardware_concurrency()), nt / 16}));
     std::atomic<int> next{0};
     std::atomic<bool> fits{true};
     auto run = [&](auto &&fn) {
         next = 0;
+        auto work = [&] {
+            try {
+                fn();
+            } catch (const std::bad_alloc &) {
+                fits = false;
+            }
+        };
         std::vector<std::thread> th;
-        for (int i = 1; i < nthr; ++i) th.emplace_back(fn);
-        fn();
+        try {
+            th.reserve(nthr);
+            for (int i = 1; i < nthr; ++i) th.emplace_back(work);
+        } catch (const std::exception &) {
+        }
+        work();
         for (auto &x : th) x.join();
     };
     run([&] {
@@ -246,7 +260,7 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
     t.econn.assign(size_t(nt) * t.ne * nen, 0);
     t.ncor.assign(size_t(nt) * t.nu * nen, uint16_t(t.ne));
     run([&] {
-        for (int ti; (ti = next++) < nt;) {
+        for (int ti; fits && (ti = next++) < nt;) {
             const Tile &q = tiles[ti];
             for (size_t i = 0; i < q.node.size(); ++i)
                 t.node[size_t(ti) * t.ns + i] = q.node[i] | (special[q.node[i]] ? INT32_MIN : 0);
@@ -261,7 +275,7 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
                 }
         }
     });
-    return true;
+    return fits;
 }
 
 }  // namespace svlg

@@ -67,7 +67,7 @@ struct HostMulti {
 };
 
 // own_ptr, conn and special in device numbering; false if a tile needs more than max_threads
-// staged nodes or elements.
+// staged nodes or elements, or if memory ran out in a worker (in the caller's thread: std::bad_alloc).
 bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8_t *special,
                 const std::vector<int32_t> &own_ptr, int depth, int max_threads, HostMulti &t);
 
