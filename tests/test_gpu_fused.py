@@ -276,7 +276,9 @@ def test_caller_captured_steps_and_eager_steps():
     """Three steps captured by the caller (past the end of the load series, so that every replay is the
     same work), replayed between eager steps of both kernels' lengths: the state is that of as many
     eager steps (the captured and the later steps are single steps: 1e-12, as test_multi_step_kernel)."""
-    import torch
+    import ctypes as C
+
+    from svl_amd import _capi as capi
     m, dt = _multi_model("quad_tiles")
     nt = m.load_series.shape[1]
     ref = DeviceModel(m)
@@ -286,26 +288,22 @@ def test_caller_captured_steps_and_eager_steps():
     want = [cr.GetDisplacements(), cr.GetVelocities(), cr.GetAccelerations()]
     ref.close()
     dm = DeviceModel(m)
-    stream = torch.cuda.Stream()
-    dm.set_stream(stream.cuda_stream)
     cd = CentralDifference(dm, dt)
     cd.Initialize()
     cd.advance(1, nt - 1)
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph, stream=stream):
-        cd.advance_async(nt, 3)
-    stream.synchronize()
-    for eager in (6, 3, 9):
-        with torch.cuda.stream(stream):
-            graph.replay()
+    hip, stream = capi.lib(), C.c_void_p(dm.stream())  # the runtime that the library is linked with
+    graph, run = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # thread-local
+    cd.advance_async(nt, 3)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for eager in (6, 3, 9, 0):
+        assert hip.hipGraphLaunch(run, stream) == 0
         cd.advance_async(nt, eager)
-    with torch.cuda.stream(stream):
-        graph.replay()
     dm.sync()
     got = [cd.GetDisplacements(), cd.GetVelocities(), cd.GetAccelerations()]
     for f, (a, b, h) in enumerate(zip(got, want, (1.0, dt, dt * dt))):
         amp = np.linalg.norm(want[0]) / (h * np.linalg.norm(b))
         assert rel_l2(a, b) < 1e-12 * max(1.0, amp), f
-    dm.set_stream(None)
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     dm.close()
-    del graph
