@@ -240,6 +240,30 @@ static bool all_affine(int dim, int nelem, int nen, const int32_t *conn, const d
     return true;
 }
 
+// Nodes that need the general update, and what the default tile size depends on.
+static TileTraits tile_inputs(const svlg_mesh_desc *d, std::vector<uint8_t> &special) {
+    const int ndim = d->ndim, nen = ndim == 2 ? 4 : 8, nn = d->nnodes, ne = d->nelem;
+    TileTraits q;
+    q.bricks = all_affine(ndim, ne, nen, d->conn, d->coords);
+    special.assign(nn, 0);
+    for (int n = 0; n < nn; ++n)
+        for (int c = 0; c < ndim; ++c)
+            if (d->free_dof[size_t(n) * ndim + c] < 0) special[n] = 1;
+    for (int i = 0; i < d->ndash; ++i) special[d->dash_node[i]] = 1;
+    for (int l = 0; l < d->nload; ++l) special[d->load_node[l]] = 1;
+    for (int i = 0; i < std::max(d->ndrm_elem, 0); ++i)
+        for (int a = 0; a < nen; ++a) special[d->conn[size_t(d->drm_elem[i]) * nen + a]] = 1;
+    bool ak = false;
+    for (int e = 0; e < ne; ++e) {
+        if (d->mat_type && d->mat_type[e] == SVLG_MAT_J2) q.j2 = true;
+        if (d->ray_ak && d->ray_ak[e] != 0.0) ak = true;
+        if (d->ray_am && d->ray_am[e] != 0.0)
+            for (int a = 0; a < nen; ++a) special[d->conn[size_t(e) * nen + a]] = 1;
+    }
+    q.implicit_lumped = ak && d->lumped != 0;
+    return q;
+}
+
 }  // namespace svlg
 
 using namespace svlg;
@@ -327,8 +351,10 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     m.ndofn = nn * ndim;
     m.th = d->thickness;
     m.lumped = d->lumped != 0;
-    m.affine = all_affine(ndim, ne, nen, d->conn, d->coords);
-    int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : 0;  // 0: chosen below
+    std::vector<uint8_t> special;
+    const TileTraits traits = tile_inputs(d, special);
+    m.affine = traits.bricks;
+    const int tile_nodes = (o && o->tile_nodes > 0) ? o->tile_nodes : 0;  // 0: the default size
     int block = (o && o->block > 0) ? o->block : 512;
     const int req_variant = (o && o->variant > 0) ? o->variant : 0;
     if (req_variant < 0 || req_variant > 3) { set_error("variant must be 0 (auto), 1, 2 or 3"); return fail(11); }
@@ -351,21 +377,6 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
         if (d->ray_ak) ak[e] = d->ray_ak[e];
         if (ak[e] != 0.0) m.has_ak = true;
     }
-    const bool auto_tiles = tile_nodes == 0;
-    if (auto_tiles) tile_nodes = default_tile_nodes(ndim, nn, m.affine, any_j2, m.has_ak && m.lumped);
-    // Nodes that need the general update.
-    std::vector<uint8_t> special(nn, 0);
-    for (int n = 0; n < nn; ++n)
-        for (int c = 0; c < ndim; ++c)
-            if (d->free_dof[size_t(n) * ndim + c] < 0) special[n] = 1;
-    for (int i = 0; i < d->ndash; ++i) special[d->dash_node[i]] = 1;
-    for (int l = 0; l < d->nload; ++l) special[d->load_node[l]] = 1;
-    for (int i = 0; i < std::max(d->ndrm_elem, 0); ++i)
-        for (int a = 0; a < nen; ++a) special[d->conn[size_t(d->drm_elem[i]) * nen + a]] = 1;
-    for (int e = 0; e < ne; ++e)
-        if (am[e] != 0.0)
-            for (int a = 0; a < nen; ++a) special[d->conn[size_t(e) * nen + a]] = 1;
-
     // Corner-slot scatter needs every (node, corner position) pair to occur at most once.
     bool corner_unique = true;
     {
@@ -379,14 +390,8 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     }
     HostTiles ht;
     try {
-        make_tiles(ndim, nn, ne, nen, d->coords, d->conn, m.h_color.data(), m.ncolors, special.data(), tile_nodes, ht);
-        // Sizes of the library's choice must leave the corner-slot kernels possible where the
-        // smaller tiles did (512 elements a tile; flat or long tiles touch more).
-        const int safe = ndim == 3 ? 160 : 192;
-        if (auto_tiles && !any_j2 && tile_nodes > safe && ht.ntiles > 1 && std::max(ht.max_elem, ht.max_own) > 512) {
-            ht = HostTiles();
-            make_tiles(ndim, nn, ne, nen, d->coords, d->conn, m.h_color.data(), m.ncolors, special.data(), safe, ht);
-        }
+        plan_tiles(ndim, nn, ne, nen, d->coords, d->conn, m.h_color.data(), m.ncolors, special.data(), tile_nodes,
+                   traits, ht);
     } catch (const std::exception &ex) {
         set_error(std::string("tiling failed: ") + ex.what());
         return fail(11);
@@ -775,27 +780,13 @@ int svlg_plan_tiles(const svlg_mesh_desc *d, int32_t tile_nodes, int64_t *stats)
     std::vector<int32_t> color;
     int ncolors = 0;
     SVLG_CHECK(color_elements(ne, nen, nn, d->conn, color, ncolors) == 0, "coloring failed");
-    std::vector<uint8_t> special(nn, 0);
-    for (int n = 0; n < nn; ++n)
-        for (int c = 0; c < ndim; ++c)
-            if (d->free_dof[size_t(n) * ndim + c] < 0) special[n] = 1;
-    for (int i = 0; i < d->ndash; ++i) special[d->dash_node[i]] = 1;
-    for (int l = 0; l < d->nload; ++l) special[d->load_node[l]] = 1;
-    for (int i = 0; i < std::max(d->ndrm_elem, 0); ++i) {
+    for (int i = 0; i < std::max(d->ndrm_elem, 0); ++i)
         SVLG_CHECK(d->drm_elem && d->drm_elem[i] >= 0 && d->drm_elem[i] < ne, "DRM element out of range");
-        for (int a = 0; a < nen; ++a) special[d->conn[size_t(d->drm_elem[i]) * nen + a]] = 1;
-    }
-    bool has_j2 = false;
-    for (int e = 0; d->mat_type && e < ne; ++e) has_j2 |= d->mat_type[e] == SVLG_MAT_J2;
-    bool has_ak = false;
-    for (int e = 0; d->ray_ak && e < ne; ++e) has_ak |= d->ray_ak[e] != 0.0;
+    std::vector<uint8_t> special;
+    const TileTraits traits = tile_inputs(d, special);
     HostTiles t;
     try {
-        make_tiles(ndim, nn, ne, nen, d->coords, d->conn, color.data(), ncolors, special.data(),
-                   tile_nodes > 0 ? tile_nodes
-                                  : default_tile_nodes(ndim, nn, all_affine(ndim, ne, nen, d->conn, d->coords),
-                                                       has_j2, has_ak && d->lumped != 0),
-                   t);
+        plan_tiles(ndim, nn, ne, nen, d->coords, d->conn, color.data(), ncolors, special.data(), tile_nodes, traits, t);
     } catch (const std::exception &ex) {
         set_error(std::string("tiling failed: ") + ex.what());
         return 11;

@@ -159,6 +159,26 @@ void make_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const
     t.halo_ptr[t.ntiles] = int32_t(t.halo_node.size());
 }
 
+int default_tile_nodes(int ndim, int nnodes, const TileTraits &q) {
+    if (q.j2) return ndim == 3 ? 160 : 448;
+    if (ndim == 3 && q.bricks && q.implicit_lumped && nnodes >= 330 * 512) return 330;
+    if (ndim == 3) return nnodes <= 160 ? 160 : nnodes <= 12000 ? 40 : q.bricks ? 160 : 96;
+    if (nnodes <= 512) return 512;
+    return nnodes <= 8000 ? 64 : nnodes <= 36000 ? 128 : nnodes <= 1000000 ? 400 : 192;
+}
+
+void plan_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const int32_t *conn, const int32_t *color,
+                int ncolors, const uint8_t *special, int tile_nodes, const TileTraits &q, HostTiles &t) {
+    const bool named = tile_nodes > 0;
+    if (!named) tile_nodes = default_tile_nodes(ndim, nnodes, q);
+    make_tiles(ndim, nnodes, nelem, nen, X, conn, color, ncolors, special, tile_nodes, t);
+    const int safe = ndim == 3 ? 160 : 192;
+    if (!named && !q.j2 && tile_nodes > safe && t.ntiles > 1 && std::max(t.max_elem, t.max_own) > 512) {
+        t = HostTiles();
+        make_tiles(ndim, nnodes, nelem, nen, X, conn, color, ncolors, special, safe, t);
+    }
+}
+
 bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8_t *special,
                 const std::vector<int32_t> &own_ptr, int depth, int max_threads, HostMulti &t) {
     const int nt = int(own_ptr.size()) - 1;

@@ -21,7 +21,14 @@ struct HostTiles {
     std::vector<int32_t> color_ptr;  // [ntiles*(ncolors+1)] offsets inside the tile's elements
 };
 
-// Node-tile size when the caller names none (bricks: the elements are parallelepipeds). 3D: 160 nodes fill the chip and recompute 0.7
+// What the default tile size depends on beside the counts.
+struct TileTraits {
+    bool bricks = false;           // the elements are parallelepipeds
+    bool j2 = false;               // a J2 element
+    bool implicit_lumped = false;  // stiffness-proportional damping and a lumped mass: implicit integrators only
+};
+
+// Node-tile size when the caller names none. 3D: 160 nodes fill the chip and recompute 0.7
 // elements per element; up to 12,000 nodes smaller tiles spread the mesh over the 256 CUs and leave
 // room for the second ring of the multi-step kernel (8,125 nodes: 36 to 48 nodes 3.6 us per
 // step, 64 nodes 3.8, 160 nodes 5.7). 2D: one tile while a workgroup holds the mesh, then tiles that
@@ -39,18 +46,18 @@ struct HostTiles {
 // lumped mass): 330 nodes, whose operator has fewer partials to add up and less to recompute (64^3
 // block: Jacobi 48.9 -> 40.2 us per iteration, the learned preconditioner's operator 32 -> 24.5, its
 // layers 11.7 -> 10.5); below 512 such tiles the CUs need the smaller ones.
-inline int default_tile_nodes(int ndim, int nnodes, bool bricks, bool j2, bool implicit_lumped) {
-    if (j2) return ndim == 3 ? 160 : 448;
-    if (ndim == 3 && bricks && implicit_lumped && nnodes >= 330 * 512) return 330;
-    if (ndim == 3) return nnodes <= 160 ? 160 : nnodes <= 12000 ? 40 : bricks ? 160 : 96;
-    if (nnodes <= 512) return 512;
-    return nnodes <= 8000 ? 64 : nnodes <= 36000 ? 128 : nnodes <= 1000000 ? 400 : 192;
-}
+int default_tile_nodes(int ndim, int nnodes, const TileTraits &q);
 
 // special[n] != 0 marks nodes that need the general update (restrained DOF, dashpot,
 // Rayleigh mass damping, point load).
 void make_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const int32_t *conn,
                 const int32_t *color, int ncolors, const uint8_t *special, int max_own, HostTiles &t);
+
+// The tiles of a model: of at most tile_nodes nodes, or of the default size (tile_nodes <= 0), which
+// must leave the corner-slot kernels possible where smaller tiles do (512 elements a tile; flat or
+// long tiles touch more).
+void plan_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const int32_t *conn, const int32_t *color,
+                int ncolors, const uint8_t *special, int tile_nodes, const TileTraits &q, HostTiles &t);
 
 // Deep-halo plan of the multi-step explicit kernel over the same tiles: every tile's nodes in
 // rings around its owned nodes (ring d: reached through d layers of elements) and its elements in

@@ -307,3 +307,13 @@ def test_caller_captured_steps_and_eager_steps():
         assert rel_l2(a, b) < 1e-12 * max(1.0, amp), f
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     dm.close()
+
+
+def test_planned_tiles_are_the_models():
+    """The host-only plan of the default tiles is the one that the model steps with."""
+    from svl_amd.integrators import plan_tiles
+    from test_tiles import stretched_layer
+    for m in (stretched_layer(), W.realization2d(61, 37, 6, nt=3)[0], W.halfspace3d(13, 11, 9, nt=3)[0]):
+        dm = DeviceModel(m)
+        assert dm.info()["ntiles"] == plan_tiles(m)["ntiles"]
+        dm.close()

@@ -66,3 +66,21 @@ def test_compact_tiles_on_structured_grid():
     avg_own = m.nnodes / st["ntiles"]
     assert avg_stage < 2.3 * avg_own
     assert st["redundancy"] < 1.6
+
+
+def stretched_layer():
+    """20 x 4000 elements, 50 times as wide as high: 400-node tiles are one or two columns of nodes and touch
+    more than 512 elements, so the default falls back to 192 nodes."""
+    m, _, _ = W.layer2d(20, 4000, nt=4)
+    m.coords = np.ascontiguousarray(m.coords * np.array([50.0, 1.0]))
+    return m
+
+
+def test_plan_default_size_of_stretched_tiles():
+    m = stretched_layer()
+    assert plan_tiles(m, 400)["max_elem"] > 512
+    st = plan_tiles(m)
+    assert st["max_elem"] <= 512 and st == plan_tiles(m, 192)
+    # Single-tile and ordinary meshes keep the default size.
+    assert plan_tiles(W.layer2d(20, 10, nt=4)[0])["ntiles"] == 1
+    assert 192 < plan_tiles(W.layer2d(400, 200, nt=4)[0])["max_own"] <= 400
