@@ -175,7 +175,7 @@ struct Model {
     DevBuf<int32_t> rec;              // recorded node-DOFs
     // Recording inside the step kernels: the history column of every node-DOF (-1: none) and
     // the tiles that own a recorded DOF.
-    DevBuf<int32_t> recmap, recdup;
+    DevBuf<int32_t> recmap;
     DevBuf<int32_t> rectile;
     std::vector<int32_t> h_f2n;       // node-DOF position of every free DOF (made on first use)
     // Multi-step plan: made by the first CentralDifference initialisation of a model that can use it.

@@ -140,15 +140,6 @@ __global__ void k_rec_map(int nrec, const int32_t *__restrict__ rec, int on, int
     if (r < nrec && rec[r] >= 0) map[rec[r]] = on ? r : -1;
 }
 
-// Columns that repeat an earlier column's DOF: dup holds (column, earlier column) pairs.
-__global__ void k_rec_dup(int ndup, const int32_t *__restrict__ dup, int nsteps, int nrec,
-                          double *__restrict__ hist) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ndup * nsteps) return;
-    double *row = hist + size_t(i / ndup) * nrec;
-    row[dup[2 * (i % ndup)]] = row[dup[2 * (i % ndup) + 1]];
-}
-
 // U, V, A of the free DOFs in free order (CentralDifference::ComputeNewStep, :141-145, with U =
 // U_{k-1}, Up = U_{k-2}, dU = U_k - U_{k-1}); null outputs are left out. Bandwidth-bound: one
 // pass over the three vectors, then one copy per field that the caller asks for. The host loop
@@ -1733,7 +1724,6 @@ int svlg_cd_steps(svlg_model *h, int32_t k0, int32_t nsteps, int32_t nrec, const
             if (m.rec.n < pos.size()) SVLG_HIP(m.rec.alloc(pos.size()));
             SVLG_HIP(hipMemcpyAsync(m.rec.p, pos.data(), sizeof(int32_t) * pos.size(), hipMemcpyHostToDevice, m.stream));
             SVLG_HIP(hipMemcpyAsync(m.rectile.p, tf.data(), sizeof(int32_t) * tf.size(), hipMemcpyHostToDevice, m.stream));
-            if (!dup.empty()) SVLG_HIP(m.recdup.upload(dup.data(), dup.size(), m.stream));
             hipLaunchKernelGGL(k_rec_map, dim3((nrec + 255) / 256), dim3(256), 0, m.stream, nrec, m.rec.p, 1,
                                m.recmap.p);
             SVLG_HIP(hipStreamSynchronize(m.stream));  // the host arrays above end with this block
@@ -1755,19 +1745,19 @@ int svlg_cd_steps(svlg_model *h, int32_t k0, int32_t nsteps, int32_t nrec, const
                                    m.U[m.ring].p, m.hist.p + size_t(s) * nrec);
         }
     }
-    if (rec.map) {
-        const int nd = int(dup.size() / 2);
-        if (nd > 0 && nsteps > 0 && rc == 0)
-            hipLaunchKernelGGL(k_rec_dup, dim3((size_t(nd) * nsteps + 255) / 256), dim3(256), 0, m.stream, nd,
-                               m.recdup.p, nsteps, nrec, m.hist.p);
+    if (rec.map)
         hipLaunchKernelGGL(k_rec_map, dim3((nrec + 255) / 256), dim3(256), 0, m.stream, nrec, m.rec.p, 0, m.recmap.p);
-    }
     if (rc) return rc;
     SVLG_HIP(hipGetLastError());
     if (nrec > 0 && nsteps > 0)
         SVLG_HIP(hipMemcpyAsync(hist, m.hist.p, sizeof(double) * size_t(nrec) * nsteps, hipMemcpyDeviceToHost,
                                 m.stream));
     SVLG_HIP(hipStreamSynchronize(m.stream));
+    // (On the host: columns times steps may pass 2^31.)
+    for (int s = 0; s < nsteps && !dup.empty(); ++s) {
+        double *row = hist + size_t(s) * nrec;
+        for (size_t i = 0; i < dup.size(); i += 2) row[dup[i]] = row[dup[i + 1]];
+    }
     return 0;
 }
 
