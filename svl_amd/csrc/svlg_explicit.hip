@@ -15,7 +15,6 @@
 #include <algorithm>
 #include <cstring>
 #include <memory>
-#include <numeric>
 
 #include "svlg_common.hpp"
 #include "svlg_drm.hpp"
@@ -135,9 +134,21 @@ __device__ __forceinline__ void record_dof(const RecRef &r, size_t g, int row, d
     if (c >= 0) r.hist[size_t(row) * r.nrec + c] = u;
 }
 
-__global__ void k_rec_map(int nrec, const int32_t *__restrict__ rec, int on, int32_t *__restrict__ map) {
+// Sets (on = 1) or clears the columns of the recorded DOFs and the flags of the tiles that own them.
+__global__ void k_rec_map(int nrec, const int32_t *__restrict__ rec, int on, int dim, int ntiles,
+                          const int32_t *__restrict__ own_ptr, int32_t *__restrict__ map,
+                          int32_t *__restrict__ tile) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nrec && rec[r] >= 0) map[rec[r]] = on ? r : -1;
+    if (r >= nrec || rec[r] < 0) return;
+    map[rec[r]] = on ? r : -1;
+    const int node = rec[r] / dim;
+    int lo = 0, hi = ntiles;  // own_ptr[lo] <= node < own_ptr[hi]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) / 2;
+        if (own_ptr[mid] <= node) lo = mid;
+        else hi = mid;
+    }
+    tile[lo] = on;
 }
 
 // U, V, A of the free DOFs in free order (CentralDifference::ComputeNewStep, :141-145, with U =
@@ -1433,6 +1444,11 @@ static int cd_one_step(Model &m, int k, const RecRef *rec = nullptr) {
     return 0;
 }
 
+static void rec_columns(Model &m, int nrec, int on) {
+    hipLaunchKernelGGL(k_rec_map, dim3((nrec + 255) / 256), dim3(256), 0, m.stream, nrec, m.rec.p, on, m.ndim,
+                       m.tiles.ntiles, m.tiles.own_ptr.p, m.recmap.p, m.rectile.p);
+}
+
 // Whether steps go through the multi-step kernel: a plan exists, and the caller has not captured steps
 // since the last initialisation. Its launches exchange buffers with the state's ring, which a
 // replay would not repeat, and a graph captured before would go on in buffers that are no longer the state:
@@ -1686,52 +1702,46 @@ int svlg_cd_steps(svlg_model *h, int32_t k0, int32_t nsteps, int32_t nrec, const
     SVLG_CHECK(m.cd_ready, "svlg_cd_init has not been called");
     SVLG_CHECK(nsteps >= 0 && nrec >= 0, "negative count");
     RecRef rec{nullptr, nullptr, nullptr, 0};
-    std::vector<int32_t> dup;
+    std::vector<int32_t> pos, dup;
     // The step kernels record, except where support motion moves DOFs after them or the
     // element-colored kernels run: there a kernel per step does.
     const bool inside = m.sm_ndofs == 0 && (m.variant == 1 || m.variant == 3);
     if (nrec > 0) {
         SVLG_CHECK(rec_dofs && hist, "recorder arrays missing");
-        std::vector<int32_t> rn;
-        if (int rc = record_positions(m, nrec, rec_dofs, rn)) return rc;
+        if (int rc = record_positions(m, nrec, rec_dofs, pos)) return rc;
         const size_t want = size_t(nrec) * std::max(nsteps, 1);
         if (m.hist.n < want) SVLG_HIP(m.hist.alloc(want));
+        if (m.rec.n < pos.size()) SVLG_HIP(m.rec.alloc(pos.size()));
         if (inside) {
-            // A DOF asked for more than once is recorded in its first column and copied.
-            std::vector<int32_t> ord(nrec);
-            std::iota(ord.begin(), ord.end(), 0);
-            std::sort(ord.begin(), ord.end(),
-                      [&](int32_t a, int32_t b) { return rn[a] < rn[b] || (rn[a] == rn[b] && a < b); });
-            std::vector<int32_t> pos = rn;
-            std::vector<int32_t> tf(m.tiles.ntiles, 0);
-            for (int i = 0, first = 0; i < nrec; ++i) {
-                if (i > 0 && rn[ord[i]] == rn[ord[first]]) {
-                    dup.push_back(ord[i]);
-                    dup.push_back(ord[first]);
-                    pos[ord[i]] = -1;
-                } else {
-                    first = i;
-                    const int node = rn[ord[i]] / m.ndim;
-                    tf[std::upper_bound(m.h_own_ptr.begin(), m.h_own_ptr.end(), node) - m.h_own_ptr.begin() - 1] = 1;
+            // A DOF asked for more than once is recorded in its first column and copied. Columns in
+            // ascending free order (a whole field, a line of nodes) hold none; otherwise one pass finds
+            // them (a sort took 68 of 70 ms of a one-step call that recorded 1.56M DOFs).
+            bool distinct = rec_dofs[0] >= 0;
+            for (int r = 1; r < nrec && distinct; ++r) distinct = rec_dofs[r] > rec_dofs[r - 1];
+            if (!distinct) {
+                std::vector<int32_t> first(m.ndofn, -1);
+                for (int r = 0; r < nrec; ++r) {
+                    int32_t &f = first[pos[r]];
+                    if (f < 0) {
+                        f = r;
+                    } else {
+                        dup.push_back(r);
+                        dup.push_back(f);
+                        pos[r] = -1;
+                    }
                 }
             }
-            if (!m.recmap.p) {
-                std::vector<int32_t> none(m.ndofn, -1);
-                SVLG_HIP(m.recmap.upload(none.data(), none.size(), m.stream));
-                SVLG_HIP(hipStreamSynchronize(m.stream));
-                SVLG_HIP(m.rectile.alloc(tf.size()));
+            if (!m.rectile.p) {
+                SVLG_HIP(m.recmap.alloc(m.ndofn));
+                SVLG_HIP(hipMemsetAsync(m.recmap.p, 0xff, sizeof(int32_t) * m.ndofn, m.stream));
+                SVLG_HIP(m.rectile.alloc(m.tiles.ntiles));
+                SVLG_HIP(hipMemsetAsync(m.rectile.p, 0, sizeof(int32_t) * m.tiles.ntiles, m.stream));
             }
-            if (m.rec.n < pos.size()) SVLG_HIP(m.rec.alloc(pos.size()));
-            SVLG_HIP(hipMemcpyAsync(m.rec.p, pos.data(), sizeof(int32_t) * pos.size(), hipMemcpyHostToDevice, m.stream));
-            SVLG_HIP(hipMemcpyAsync(m.rectile.p, tf.data(), sizeof(int32_t) * tf.size(), hipMemcpyHostToDevice, m.stream));
-            hipLaunchKernelGGL(k_rec_map, dim3((nrec + 255) / 256), dim3(256), 0, m.stream, nrec, m.rec.p, 1,
-                               m.recmap.p);
-            SVLG_HIP(hipStreamSynchronize(m.stream));  // the host arrays above end with this block
+        }
+        SVLG_HIP(hipMemcpyAsync(m.rec.p, pos.data(), sizeof(int32_t) * pos.size(), hipMemcpyHostToDevice, m.stream));
+        if (inside) {
             rec = RecRef{m.recmap.p, m.rectile.p, m.hist.p, nrec};
-        } else {
-            if (m.rec.n < rn.size()) SVLG_HIP(m.rec.alloc(rn.size()));
-            SVLG_HIP(hipMemcpyAsync(m.rec.p, rn.data(), sizeof(int32_t) * rn.size(), hipMemcpyHostToDevice, m.stream));
-            SVLG_HIP(hipStreamSynchronize(m.stream));
+            rec_columns(m, nrec, 1);
         }
     }
     int rc = 0;
@@ -1745,9 +1755,11 @@ int svlg_cd_steps(svlg_model *h, int32_t k0, int32_t nsteps, int32_t nrec, const
                                    m.U[m.ring].p, m.hist.p + size_t(s) * nrec);
         }
     }
-    if (rec.map)
-        hipLaunchKernelGGL(k_rec_map, dim3((nrec + 255) / 256), dim3(256), 0, m.stream, nrec, m.rec.p, 0, m.recmap.p);
-    if (rc) return rc;
+    if (rec.map) rec_columns(m, nrec, 0);
+    if (rc) {
+        (void)hipStreamSynchronize(m.stream);  // pos is on its way to the device
+        return rc;
+    }
     SVLG_HIP(hipGetLastError());
     if (nrec > 0 && nsteps > 0)
         SVLG_HIP(hipMemcpyAsync(hist, m.hist.p, sizeof(double) * size_t(nrec) * nsteps, hipMemcpyDeviceToHost,

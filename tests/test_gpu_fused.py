@@ -317,3 +317,34 @@ def test_planned_tiles_are_the_models():
         dm = DeviceModel(m)
         assert dm.info()["ntiles"] == plan_tiles(m)["ntiles"]
         dm.close()
+
+
+@pytest.mark.parametrize("opts", [{}, {"variant": 3, "tile_nodes": 40}, {"variant": 1, "tile_nodes": 40}])
+@pytest.mark.parametrize("kind", ["quad_one_tile", "quad_tiles", "hexa_tiles"])
+def test_recorded_columns(kind, opts):
+    """Whole fields and lists in any order, with free DOFs, total DOFs (-1 - t) of free and restrained
+    nodes and repeated columns, recorded in turn: every column of every call equals the displacement
+    that an element-coloured model (its own recorder kernel, rounding apart) has there, and columns of one DOF are
+    equal bit for bit."""
+    m, dt = _multi_model(kind)
+    rng = np.random.default_rng(11)
+    total = -1 - rng.permutation(m.nnodes * m.ndim)[:200].astype(np.int64)
+    mixed = rng.permutation(np.concatenate([np.arange(m.nfree), rng.integers(0, m.nfree, 50), total]))
+    lists = [np.arange(m.nfree), mixed[:97], mixed, np.arange(m.nfree)[::-1], [3], [3, 3]]
+    dm, ref = DeviceModel(m, **opts), DeviceModel(m, variant=2)
+    cd, cr = CentralDifference(dm, dt), CentralDifference(ref, dt)
+    cd.Initialize()
+    cr.Initialize()
+    free = m.free_dof().reshape(-1)
+    k = 1
+    for cols in lists:
+        cols = np.asarray(cols, dtype=np.int32)
+        h, r = cd.advance(k, 9, cols), cr.advance(k, 9, cols)
+        assert np.abs(h - r).max() <= 1e-11 * max(np.abs(r).max(), 1e-300)
+        dof = np.where(cols >= 0, cols, free[np.where(cols < 0, -1 - cols, 0)])  # -1: restrained
+        assert (h[:, dof < 0] == 0.0).all()
+        u = cd.GetDisplacements()
+        assert np.array_equal(h[-1, dof >= 0], u[dof[dof >= 0]])
+        k += 9
+    dm.close()
+    ref.close()
