@@ -171,6 +171,10 @@ int svlg_internal_force(svlg_model *m, const double *U /*[nfree]*/, double ftol,
 /* ---- CentralDifference (10-Integrators/02-CentralDifference/CentralDifference.cpp) */
 /* Initialize (:36-71): zero state, Keff = M/dt^2 + C/(2dt) (diagonal), ftol filter. */
 int svlg_cd_init(svlg_model *m, double dt, double ftol);
+/* The kernels of svlg_cd_steps after svlg_cd_init: plan4[0] steps per launch (1: one launch per
+ * step, also after steps captured by the caller), [1] node tiles, [2] threads per workgroup,
+ * [3] 1 for the multi-step kernel of many tiles (fewer registers, nothing kept between steps). */
+int svlg_cd_plan(svlg_model *m, int64_t *plan4);
 /* Advances nsteps steps starting at step index k0 (ComputeNewStep :124-152 via
  * Linear::ComputeNewIncrement, with DynamicAnalysis' index convention: step k uses
  * load sample k). If nrec > 0, U at the DOFs rec_dofs[] after every step is written to

@@ -156,6 +156,7 @@ SIGNATURES = {
     "svlg_damping_diagonal": (C.c_int, [C.c_void_p, f64p]),
     "svlg_internal_force": (C.c_int, [C.c_void_p, f64p, C.c_double, f64p]),
     "svlg_cd_init": (C.c_int, [C.c_void_p, C.c_double, C.c_double]),
+    "svlg_cd_plan": (C.c_int, [C.c_void_p, C.POINTER(C.c_int64)]),
     "svlg_cd_steps": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_int32, i32p, f64p]),
     "svlg_cd_steps_async": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32]),
     "svlg_cd_get_state": (C.c_int, [C.c_void_p, f64p, f64p, f64p]),

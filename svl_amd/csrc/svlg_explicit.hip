@@ -1219,14 +1219,16 @@ template <int DIM, int MAXB, int MAXE, bool WIDE>
 static const void *multi_fn_t(int path) {
     switch (path) {
         case 3: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 3, MAXB, MAXE, WIDE>);
-        case 2: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 2, MAXB, MAXE, WIDE && DIM == 2>);
+        case 2: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 2, MAXB, MAXE, WIDE>);
         case 1: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 1, MAXB, MAXE, false>);
         default: return reinterpret_cast<const void *>(&k_cd_multi<DIM, 0, MAXB, MAXE, false>);
     }
 }
 
+static bool multi_wide(const Model &m) { return m.multi.ntiles > 1024 && m.ndim == 2 && m.elem_path >= 2; }
+
 static const void *multi_fn(const Model &m) {
-    const bool wide = m.multi.ntiles > 1024;
+    const bool wide = multi_wide(m);
     if (m.ndim == 2) {
         switch (m.multi.block) {
             case 256: return wide ? multi_fn_t<2, 256, 256, true>(m.elem_path) : multi_fn_t<2, 256, 256, false>(m.elem_path);
@@ -1464,6 +1466,9 @@ static bool multi_ready(Model &m) {
     return !m.captured;
 }
 
+// Steps per launch of the multi-step kernel (one tile has no neighbours to recompute).
+static int multi_steps(const Model &m) { return m.multi.ntiles == 1 ? 2048 : m.multi.depth; }
+
 // nsteps steps from k0, recording into rec (map null: nothing).
 static int cd_advance(Model &m, int k0, int nsteps, const RecRef &rec) {
     if (!multi_ready(m)) {
@@ -1474,7 +1479,7 @@ static int cd_advance(Model &m, int k0, int nsteps, const RecRef &rec) {
         }
         return 0;
     }
-    const int most = m.multi.ntiles == 1 ? 2048 : m.multi.depth;
+    const int most = multi_steps(m);
     RecRef r = rec;
     for (int s = 0; s < nsteps;) {
         const int n = std::min(most, nsteps - s);
@@ -1613,6 +1618,18 @@ int svlg_cd_init_batch(svlg_model *h, int32_t nparts, const int32_t *part_node_p
     for (int p = 0; p < m.nnodes; ++p)
         for (int c = 0; c < m.ndim; ++c) dtd[size_t(p) * m.ndim + c] = dt_node[m.perm[p]];
     return cd_init_impl(m, dts[0], &dtd, ftol);
+}
+
+int svlg_cd_plan(svlg_model *h, int64_t *plan) {
+    SVLG_CHECK(h && plan, "null argument");
+    Model &m = h->m;
+    SVLG_CHECK(m.cd_ready, "svlg_cd_init has not been called");
+    const bool multi = m.multi.depth > 0 && !m.captured;
+    plan[0] = multi ? multi_steps(m) : 1;
+    plan[1] = m.tiles.ntiles;
+    plan[2] = multi ? m.multi.block : m.tiles.block;
+    plan[3] = multi && multi_wide(m) ? 1 : 0;
+    return 0;
 }
 
 int svlg_cd_steps_async(svlg_model *h, int32_t k0, int32_t nsteps) {

@@ -102,6 +102,14 @@ class DeviceModel:
         capi.check(capi.lib().svlg_sync(self.h), "svlg_sync")
 
 
+def cd_plan(mesh: DeviceModel) -> dict:
+    """The kernels that an initialised CentralDifference steps with: `steps` per launch (1: one launch
+    per step), `ntiles`, `block` threads per workgroup, `wide` the multi-step kernel of many tiles."""
+    a = (C.c_int64 * 4)()
+    capi.check(capi.lib().svlg_cd_plan(mesh.h, a), "svlg_cd_plan")
+    return dict(zip(["steps", "ntiles", "block", "wide"], [int(v) for v in a]))
+
+
 def plan_tiles(model: Model, tile_nodes: int = 0) -> dict:
     """Host-only tile plan of the fused explicit kernel (no GPU needed)."""
     desc, keep = capi.make_desc(model)

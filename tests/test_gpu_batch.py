@@ -12,7 +12,7 @@ import pytest
 import oracle
 from svl_amd import batch as B
 from svl_amd import workloads as W
-from svl_amd.integrators import DeviceModel
+from svl_amd.integrators import DeviceModel, cd_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -27,8 +27,8 @@ def small_batch(nt=161):
     return W.batch2d(3, nt=nt, nx_range=(8, 20), ny_range=(5, 12))
 
 
-def device(u, nptr, fptr, dts, tile_nodes=0):
-    dm = DeviceModel(u, tile_nodes=tile_nodes)
+def device(u, nptr, fptr, dts, tile_nodes=0, variant=0):
+    dm = DeviceModel(u, tile_nodes=tile_nodes, variant=variant)
     cd = B.BatchedCentralDifference(dm, dts, nptr, fptr)
     cd.Initialize()
     return dm, cd
@@ -55,16 +55,19 @@ def test_parts_match_independent_oracle_runs(tile_nodes):
     dm.close()
 
 
-def test_graph_replays_equal_eager_steps():
+@pytest.mark.parametrize("variant", [0, 1, 3])
+def test_graph_replays_equal_eager_steps(variant):
+    """Variants 1 and 3 (single-step kernels): captured graphs; 0: several steps per launch, no graph."""
     models, dts, nt = small_batch(nt=400)
     u, nptr, fptr = B.union(models)
-    dm, cd = device(u, nptr, fptr, dts)
+    dm, cd = device(u, nptr, fptr, dts, variant=variant)
+    assert (cd_plan(dm)["steps"] > 1) == (variant == 0)
     cd.advance(1, 99)
     cd.advance(100, 3)
     cd.advance(103, 198)
     Ue = cd.GetDisplacements()
     dm.close()
-    dm, cd = device(u, nptr, fptr, dts)
+    dm, cd = device(u, nptr, fptr, dts, variant=variant)
     cd.advance(1, 99, graph_steps=30)   # 3 replays + 9 eager steps
     cd.advance(100, 3)                   # eager between replays (ring slot preserved)
     cd.advance(103, 198, graph_steps=30)  # graph reused: 6 replays + 18 eager

@@ -18,7 +18,7 @@ import pytest
 
 import oracle
 from svl_amd import _capi as capi, drm
-from svl_amd.integrators import CentralDifference, DeviceModel, ExtendedNewmarkBeta
+from svl_amd.integrators import CentralDifference, DeviceModel, ExtendedNewmarkBeta, cd_plan
 from svl_amd.mesh import Model
 
 from _meshes import drm_hexa_model, drm_quad_model
@@ -119,13 +119,17 @@ def test_reactions_on_drm_layer_match_oracle():
     assert np.abs(R - want).max() <= 1e-9 * np.abs(want).max()
 
 
-def test_graph_steps_match_eager():
+@pytest.mark.parametrize("variant", [0, 3])
+def test_graph_steps_match_eager(variant):
+    """Variant 3: graphs of single steps, whose forces follow the step number on the device; 0: several
+    steps per launch, no graph."""
     m, r, box, dt, nt, rec, bg = case("quad", oracle.CENTRAL_DIFFERENCE)
     states = []
     for graph in (False, True):
-        dm = DeviceModel(r)
+        dm = DeviceModel(r, variant=variant)
         cd = CentralDifference(dm, dt)
         cd.Initialize()
+        assert (cd_plan(dm)["steps"] > 1) == (variant == 0)
         if graph:
             capi.check(capi.lib().svlg_cd_graph_steps(dm.h, 1, 12 * 6, 6), "svlg_cd_graph_steps")
         else:

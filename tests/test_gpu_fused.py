@@ -11,7 +11,7 @@ import pytest
 
 import oracle
 from svl_amd import workloads as W
-from svl_amd.integrators import CentralDifference, DeviceModel
+from svl_amd.integrators import CentralDifference, DeviceModel, cd_plan
 from svl_amd.mesh import ELEM_HEXA8, ELEM_QUAD4, Model, make_domain_area, make_domain_volume, ricker_velocity, tags_for
 
 from _meshes import block_model, graded, rotation
@@ -229,6 +229,8 @@ def test_multi_step_kernel(kind):
     dm = DeviceModel(m)
     cd = CentralDifference(dm, dt)
     cd.Initialize()
+    plan = cd_plan(dm)
+    assert plan["steps"] > 1 and plan["wide"] == 0 and (plan["steps"] == 2048) == (plan["ntiles"] == 1)
     hist = cd.advance(1, 60, rec)
     state = [cd.GetDisplacements(), cd.GetVelocities(), cd.GetAccelerations()]
     cd.Initialize()
@@ -244,6 +246,7 @@ def test_multi_step_kernel(kind):
     ref = DeviceModel(m, variant=3)
     cr = CentralDifference(ref, dt)
     cr.Initialize()
+    assert cd_plan(ref)["steps"] == 1
     href = cr.advance(1, 60, rec)
     assert rel_l2(hist, href) < 1e-12
     assert rel_l2(state[0], cr.GetDisplacements()) < 1e-12
@@ -252,6 +255,49 @@ def test_multi_step_kernel(kind):
         amp = np.linalg.norm(state[0]) / (h * np.linalg.norm(b))
         assert rel_l2(a, b) < 1e-12 * max(1.0, amp), f
     ref.close()
+
+
+@pytest.mark.parametrize("shape", ["bricks", "sheared"])
+def test_multi_step_kernel_of_many_tiles(shape):
+    """The same for the kernel of more than 1,024 tiles (nothing of a node's loads, damping or columns is
+    kept between steps): eight 400 x 200 layers with their own time steps, a domain reduction
+    layer through each, one node under two loads and repeated columns."""
+    from svl_amd import batch
+    from svl_amd.drm import attach, drm_box
+    parts = [W.realization2d(400, 200, 31 + i, nt=61, x0=408.0 * i) for i in range(8)]
+    rng = np.random.default_rng(2)
+    for i, (m, _, _) in enumerate(parts):
+        lo, hi = m.coords.min(0), m.coords.max(0)
+        elems, nodes, cond = drm_box(m, (lo + hi) / 2, 0.31 * (hi - lo))
+        attach(m, elems, nodes, cond, 1e-4 * rng.standard_normal((nodes.size, 61, 6)))
+        if shape == "sheared":
+            m.coords = np.ascontiguousarray(m.coords @ np.array([[1.0, 0.0], [0.2, 0.9]]))
+        m.add_point_load(int(m.load_node[0]), np.ones(2), 3e4 * np.sin(0.3 * np.arange(61)), 0.7)
+    m, node_ptr, free_ptr = batch.union([p[0] for p in parts])
+    dts = [0.5 * p[1] for p in parts]
+    rec = np.concatenate([np.arange(0, m.nfree, 1999), [0, 1999, 0, 0]]).astype(np.int32)
+    runs = []
+    for opts, calls in (({}, (60,)), ({}, (1, 2, 3, 4, 5, 9, 11, 1, 1, 2, 21)), ({"variant": 3}, (60,))):
+        dm = DeviceModel(m, **opts)
+        cd = batch.BatchedCentralDifference(dm, dts, node_ptr, free_ptr)
+        cd.Initialize()
+        plan = cd_plan(dm)
+        if opts:
+            assert plan["steps"] == 1
+        else:
+            assert plan["steps"] > 1 and plan["wide"] == 1
+        k, hist = 1, []
+        for c in calls:
+            hist.append(cd.advance(k, c, rec_dofs=rec))
+            k += c
+        runs.append((np.concatenate(hist), cd.GetDisplacements(), cd.GetVelocities()))
+        dm.close()
+    for a, b in zip(runs[0], runs[1]):
+        assert np.array_equal(a, b)
+    (h, u, v), (hr, ur, vr) = runs[0], runs[2]
+    assert rel_l2(h, hr) < 1e-12 and rel_l2(u, ur) < 1e-12
+    # V divides differences of U by dt.
+    assert rel_l2(v, vr) < 1e-12 * max(1.0, np.linalg.norm(ur) / (min(dts) * np.linalg.norm(vr)))
 
 
 def test_recording_after_a_refused_history():
