@@ -14,7 +14,9 @@
 // U_{k-2}) can be formed on demand with SVL's expressions.
 #include <algorithm>
 #include <cstring>
+#include <iterator>
 #include <memory>
+#include <new>
 
 #include "svlg_common.hpp"
 #include "svlg_drm.hpp"
@@ -1209,11 +1211,13 @@ static int launch_fused(Model &m, int k, const double *Ucur, const double *Uprev
 }
 
 // Block and element-plane sizes of the multi-step kernel: the plan takes the smallest class that
-// holds its tiles (0: none does).
+// holds its tiles (0: none does). Hexahedra need 142 to 194 registers, which 1,024 threads do not have: such
+// a class spilled 34 to 91 of them and took 11.0 us per step on 8,125 sheared bricks' nodes, whose
+// 40-node tiles are less compact and stage more than 512 nodes, against 6.9 for single steps.
 struct MultiClass {
     int block, elems;
 };
-static constexpr MultiClass kMulti2[] = {{256, 256}, {512, 456}, {1024, 968}}, kMulti3[] = {{256, 256}, {512, 512}, {1024, 640}};
+static constexpr MultiClass kMulti2[] = {{256, 256}, {512, 456}, {1024, 968}}, kMulti3[] = {{256, 256}, {512, 512}};
 
 template <int DIM, int MAXB, int MAXE, bool WIDE>
 static const void *multi_fn_t(int path) {
@@ -1238,8 +1242,7 @@ static const void *multi_fn(const Model &m) {
     }
     switch (m.multi.block) {
         case 256: return multi_fn_t<3, 256, 256, false>(m.elem_path);
-        case 512: return multi_fn_t<3, 512, 512, false>(m.elem_path);
-        default: return multi_fn_t<3, 1024, 640, false>(m.elem_path);
+        default: return multi_fn_t<3, 512, 512, false>(m.elem_path);
     }
 }
 
@@ -1251,14 +1254,16 @@ static const void *multi_fn(const Model &m) {
 //   Quad4, 1.77M nodes, 400-node tiles   29.4 -> 31.4 (4)            0.55M nodes, 128-node tiles  13.6 -> 19.9 (4)
 //   Hexa8, 1,183 / 8,125 nodes            5.6 -> 3.3 / 5.7 -> 3.6 (2)
 //   Hexa8, 18,513 / 60,025 nodes          5.9 -> 6.3 / 7.0 -> 17 (2)
+//   Hexa8, 288 to 384 tiles of 40 nodes   6.0 -> 6.1 (2)      flat elements (1 : 10)  6.1 -> 6.3 to 6.5 (2)
+//   sheared Hexa8, 2,890 nodes            6.2 -> 4.7 (2)      8,125 nodes, 300 tiles of 32 nodes  6.4 -> 7.1 (2)
 // Below a chip full of workgroups the launch is saved and the recomputed rings are free; above
 // it they compete with the tiles: in 2D the state's bytes still pay for them while a tile is
-// large against its rings and up to about a million nodes, in 3D never. Gauss-point hexahedra
-// (1,300 operations an element) recompute nothing.
+// large against its rings and up to about a million nodes, in 3D (one workgroup per CU) never.
+// Gauss-point hexahedra (1,300 operations an element) recompute nothing.
 static int multi_depth(const Model &m) {
     const int nt = m.tiles.ntiles, own = m.nnodes / nt;
     if (nt == 1) return 1;
-    if (m.ndim == 3) return m.elem_path >= 2 && nt <= 384 && own <= 64 ? 2 : 0;
+    if (m.ndim == 3) return m.elem_path >= 2 && nt <= 256 && own <= 64 ? 2 : 0;
     if (nt > 512) return own >= 256 && m.nnodes <= 1000000 ? 4 : 0;
     int d = 1;  // rings up to about six times the tile
     while (d < 8 && (2.0 * (d + 1)) * (2.0 * (d + 1)) <= 2.4 * own) ++d;
@@ -1279,19 +1284,22 @@ static int multi_build(Model &m) {
     gid.swap(m.h_gid);
     if (!m.auto_variant || !m.corner_unique || m.sm_ndofs > 0 || m.elem_bf16 || m.elem_fp32) return 0;
     int depth = multi_depth(m);
+    const MultiClass *classes = m.ndim == 2 ? kMulti2 : kMulti3;
+    const size_t nclasses = m.ndim == 2 ? std::size(kMulti2) : std::size(kMulti3);
+    const int least = m.tiles.ntiles == 1 ? 1 : 2;  // one step per launch is the single-step kernels'
     HostMulti h;
     MultiClass cls{0, 0};
     size_t lds = 0;
-    for (; depth >= 1; --depth) {  // the deepest that fits a class and the LDS
+    for (; depth >= least; --depth) {  // the deepest that fits a class and the LDS
         cls = MultiClass{0, 0};
         if (make_multi(m.nnodes, m.nelem, m.nen, conn.data(), special.data(), m.h_own_ptr, depth, 1024, h))
-            for (const MultiClass &c : m.ndim == 2 ? kMulti2 : kMulti3)
-                if (cls.block == 0 && h.ns <= c.block && h.ne <= c.elems) cls = c;
+            for (const MultiClass *c = classes; c != classes + nclasses && cls.block == 0; ++c)
+                if (h.ns <= c->block && h.ne <= c->elems) cls = *c;
         lds = (size_t(m.elem_path < 2 ? 2 : 1) * h.ns * m.ndim + size_t(m.nen) * m.ndim * (cls.elems + 1)) *
               sizeof(double);
         if (cls.block != 0 && lds <= 160 * 1024) break;
     }
-    if (depth < 1) return 0;
+    if (depth < least) return 0;
     // No element at a corner: the zero column of the class.
     for (uint16_t &c : h.ncor)
         if (c == h.ne) c = uint16_t(cls.elems);

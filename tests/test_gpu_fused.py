@@ -300,6 +300,31 @@ def test_multi_step_kernel_of_many_tiles(shape):
     assert rel_l2(v, vr) < 1e-12 * max(1.0, np.linalg.norm(ur) / (min(dts) * np.linalg.norm(vr)))
 
 
+@pytest.mark.parametrize("size,shape,steps", [
+    ((12, 12, 6), "bricks", 2), ((24, 24, 12), "bricks", 2), ((27, 25, 15), "bricks", 1),
+    ((12, 12, 6), "sheared", 2), ((24, 24, 12), "sheared", 1), ((27, 25, 15), "sheared", 1),
+    ((12, 12, 6), "distorted", 1)])
+def test_multi_step_rule_hexa(size, shape, steps):
+    """Where hexahedra take two steps per launch, and the result on either side against single
+    steps (1e-12, as test_multi_step_kernel)."""
+    m, dt, _ = W.halfspace3d(*size, nt=31, seed=1)
+    if shape == "sheared":
+        m.coords = np.ascontiguousarray(m.coords @ rotation().T)
+    elif shape == "distorted":
+        inner = np.all((m.coords > m.coords.min(0) + 1e-6) & (m.coords < m.coords.max(0) - 1e-6), axis=1)
+        m.coords[inner] += np.random.default_rng(3).uniform(-0.2, 0.2, (int(inner.sum()), 3))
+    out = []
+    for opts in ({}, {"variant": 3, "tile_nodes": 160}):
+        dm = DeviceModel(m, **opts)
+        cd = CentralDifference(dm, 0.5 * dt)
+        cd.Initialize()
+        assert cd_plan(dm)["steps"] == (1 if opts else steps)
+        cd.advance(1, 30)
+        out.append(cd.GetDisplacements())
+        dm.close()
+    assert np.abs(out[1]).max() > 0.0 and rel_l2(out[0], out[1]) < 1e-12
+
+
 def test_recording_after_a_refused_history():
     """A history larger than the card (400 GB; the caller's array is not reached) is refused, and the
     next recording of the model starts from an allocation of its own: the same history as a fresh model's."""
