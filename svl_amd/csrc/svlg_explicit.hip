@@ -1252,18 +1252,22 @@ static const void *multi_fn(const Model &m) {
 //   Quad4, 5,151 nodes, 64-node tiles     5.0 -> 1.37 (depth 6)      20,301 nodes, 128-node tiles  4.4 -> 1.42 (8)
 //   Quad4, 80,601 nodes, 400-node tiles   5.4 -> 2.24 (4)            0.55M nodes, 400-node tiles  13.5 -> 9.6 (4)
 //   Quad4, 1.77M nodes, 400-node tiles   29.4 -> 31.4 (4)            0.55M nodes, 128-node tiles  13.6 -> 19.9 (4)
+//   distorted Quad4, 100,651 / 114,091 nodes, 252 / 286 tiles  7.5 -> 5.9 / 9.5 -> 10.4 (4), 0.55M nodes  25 -> 31 (4)
+//   Quad4 25 times as wide as high, 400-node tiles, 210,951 / 0.55M nodes  7.4 -> 7.8 / 14.3 -> 14.9 (2)
 //   Hexa8, 1,183 / 8,125 nodes            5.6 -> 3.3 / 5.7 -> 3.6 (2)
 //   Hexa8, 18,513 / 60,025 nodes          5.9 -> 6.3 / 7.0 -> 17 (2)
 //   Hexa8, 288 to 384 tiles of 40 nodes   6.0 -> 6.1 (2)      flat elements (1 : 10)  6.1 -> 6.3 to 6.5 (2)
 //   sheared Hexa8, 2,890 nodes            6.2 -> 4.7 (2)      8,125 nodes, 300 tiles of 32 nodes  6.4 -> 7.1 (2)
 // Below a chip full of workgroups the launch is saved and the recomputed rings are free; above
 // it they compete with the tiles: in 2D the state's bytes still pay for them while a tile is
-// large against its rings and up to about a million nodes, in 3D (one workgroup per CU) never.
-// Gauss-point hexahedra (1,300 operations an element) recompute nothing.
+// large against its rings (three steps fit a launch) and up to about a million nodes, in 3D (one workgroup
+// per CU) and for Gauss-point quadrilaterals never. Gauss-point hexahedra (1,300 operations an element)
+// recompute nothing.
 static int multi_depth(const Model &m) {
     const int nt = m.tiles.ntiles, own = m.nnodes / nt;
     if (nt == 1) return 1;
     if (m.ndim == 3) return m.elem_path >= 2 && nt <= 256 && own <= 64 ? 2 : 0;
+    if (m.elem_path == 0 && nt > 256) return 0;
     if (nt > 512) return own >= 256 && m.nnodes <= 1000000 ? 4 : 0;
     int d = 1;  // rings up to about six times the tile
     while (d < 8 && (2.0 * (d + 1)) * (2.0 * (d + 1)) <= 2.4 * own) ++d;
@@ -1286,7 +1290,8 @@ static int multi_build(Model &m) {
     int depth = multi_depth(m);
     const MultiClass *classes = m.ndim == 2 ? kMulti2 : kMulti3;
     const size_t nclasses = m.ndim == 2 ? std::size(kMulti2) : std::size(kMulti3);
-    const int least = m.tiles.ntiles == 1 ? 1 : 2;  // one step per launch is the single-step kernels'
+    // One step per launch is the single-step kernels'; many tiles need three to pay for their rings.
+    const int least = m.tiles.ntiles == 1 ? 1 : m.tiles.ntiles <= 512 ? 2 : 3;
     HostMulti h;
     MultiClass cls{0, 0};
     size_t lds = 0;

@@ -325,6 +325,29 @@ def test_multi_step_rule_hexa(size, shape, steps):
     assert np.abs(out[1]).max() > 0.0 and rel_l2(out[0], out[1]) < 1e-12
 
 
+@pytest.mark.parametrize("size,shape,multi", [
+    ((400, 200), "bricks", True), ((400, 200), "distorted", True), ((450, 300), "distorted", False),
+    ((450, 300), "bricks", True), ((600, 350), "stretched", False)])
+def test_multi_step_rule_quad(size, shape, multi):
+    """The same for quadrilaterals around a chip full of tiles."""
+    m, dt, _ = W.realization2d(*size, 3, nt=31)
+    if shape == "stretched":
+        m.coords = np.ascontiguousarray(m.coords * np.array([25.0, 1.0]))
+    elif shape == "distorted":
+        inner = np.all((m.coords > m.coords.min(0) + 1e-6) & (m.coords < m.coords.max(0) - 1e-6), axis=1)
+        m.coords[inner] += np.random.default_rng(3).uniform(-0.12, 0.12, (int(inner.sum()), 2))
+    out = []
+    for opts in ({}, {"variant": 3, "tile_nodes": 192}):
+        dm = DeviceModel(m, **opts)
+        cd = CentralDifference(dm, 0.5 * dt)
+        cd.Initialize()
+        assert (cd_plan(dm)["steps"] > 1) == (multi and not opts)
+        cd.advance(1, 30)
+        out.append(cd.GetDisplacements())
+        dm.close()
+    assert np.abs(out[1]).max() > 0.0 and rel_l2(out[0], out[1]) < 1e-12
+
+
 def test_recording_after_a_refused_history():
     """A history larger than the card (400 GB; the caller's array is not reached) is refused, and the
     next recording of the model starts from an allocation of its own: the same history as a fresh model's."""
