@@ -261,6 +261,14 @@ static TileTraits tile_inputs(const svlg_mesh_desc *d, std::vector<uint8_t> &spe
             for (int a = 0; a < nen; ++a) special[d->conn[size_t(e) * nen + a]] = 1;
     }
     q.implicit_lumped = ak && d->lumped != 0;
+    // Corner-slot scatter needs every (node, corner position) pair to occur at most once.
+    std::vector<uint8_t> used(nn, 0);
+    for (int e = 0; e < ne && q.corner_unique; ++e)
+        for (int a = 0; a < nen; ++a) {
+            uint8_t &u = used[d->conn[size_t(e) * nen + a]];
+            if (u & (1u << a)) q.corner_unique = false;
+            u |= uint8_t(1u << a);
+        }
     return q;
 }
 
@@ -377,17 +385,7 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
         if (d->ray_ak) ak[e] = d->ray_ak[e];
         if (ak[e] != 0.0) m.has_ak = true;
     }
-    // Corner-slot scatter needs every (node, corner position) pair to occur at most once.
-    bool corner_unique = true;
-    {
-        std::vector<uint8_t> used(nn, 0);
-        for (int e = 0; e < ne && corner_unique; ++e)
-            for (int a = 0; a < nen; ++a) {
-                uint8_t &u = used[d->conn[size_t(e) * nen + a]];
-                if (u & (1u << a)) { corner_unique = false; break; }
-                u |= uint8_t(1u << a);
-            }
-    }
+    const bool corner_unique = traits.corner_unique;
     HostTiles ht;
     try {
         plan_tiles(ndim, nn, ne, nen, d->coords, d->conn, m.h_color.data(), m.ncolors, special.data(), tile_nodes,

@@ -161,10 +161,17 @@ void make_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const
 
 int default_tile_nodes(int ndim, int nnodes, const TileTraits &q) {
     if (q.j2) return ndim == 3 ? 160 : 448;
-    if (ndim == 3 && q.bricks && q.implicit_lumped && nnodes >= 330 * 512) return 330;
-    if (ndim == 3) return nnodes <= 160 ? 160 : nnodes <= 12000 ? 40 : q.bricks ? 160 : 96;
+    if (ndim == 3) {
+        if (nnodes <= 160) return 160;
+        if (!q.corner_unique) return nnodes <= 9000 ? 40 : !q.bricks && nnodes <= 23000 ? 96 : 160;
+        if (q.bricks && q.implicit_lumped && nnodes >= 330 * 512) return 330;
+        return nnodes <= 12000 ? 40 : q.bricks ? 160 : 96;
+    }
     if (nnodes <= 512) return 512;
-    return nnodes <= 8000 ? 64 : nnodes <= 36000 ? 128 : nnodes <= 1000000 ? 400 : 192;
+    if (nnodes <= 36000) return nnodes <= 8000 ? 64 : 128;
+    if (!q.corner_unique) return nnodes <= (q.bricks ? 1000000 : 100000) ? 400 : 448;
+    if (!q.bricks && !q.implicit_lumped && nnodes > 100000) return 192;
+    return nnodes <= 1000000 ? 400 : 192;
 }
 
 void plan_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const int32_t *conn, const int32_t *color,
@@ -173,7 +180,7 @@ void plan_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const
     if (!named) tile_nodes = default_tile_nodes(ndim, nnodes, q);
     make_tiles(ndim, nnodes, nelem, nen, X, conn, color, ncolors, special, tile_nodes, t);
     const int safe = ndim == 3 ? 160 : 192;
-    if (!named && !q.j2 && tile_nodes > safe && t.ntiles > 1 && std::max(t.max_elem, t.max_own) > 512) {
+    if (!named && !q.j2 && q.corner_unique && tile_nodes > safe && t.ntiles > 1 && std::max(t.max_elem, t.max_own) > 512) {
         t = HostTiles();
         make_tiles(ndim, nnodes, nelem, nen, X, conn, color, ncolors, special, safe, t);
     }

@@ -26,6 +26,7 @@ struct TileTraits {
     bool bricks = false;           // the elements are parallelepipeds
     bool j2 = false;               // a J2 element
     bool implicit_lumped = false;  // stiffness-proportional damping and a lumped mass: implicit integrators only
+    bool corner_unique = true;     // no node is the same corner of two elements (else: colour-phase kernel)
 };
 
 // Node-tile size when the caller names none. 3D: 160 nodes fill the chip and recompute 0.7
@@ -40,6 +41,15 @@ struct TileTraits {
 // Gauss-point hexahedra (256 registers, one wave per SIMD) take 96 nodes, whose elements are three
 // waves: 16,128 nodes 9.5 us per step against 12.9 with 160 and 12.2 with 64 nodes, 62,279 nodes 18.0
 // against 23.3 and 24.1.
+// Gauss-point quadrilaterals leave the multi-step kernel at a chip full of tiles; single steps take 192 nodes
+// from there on (208,921 nodes: 192 nodes 11.7 us per step, 400 nodes 13.2; 0.55M: 24.3 and 25.6).
+// The colour-phase kernel pays for every colour of a workgroup's elements and holds 512 threads: its
+// quads stay at 400 nodes or more (208,921 nodes: 400 nodes 8.5 us per step, 448 nodes 9.3; distorted
+// 15.5 and 12.3; 1.4M nodes, 448 nodes 38 and 192 nodes 66, distorted 58 and 86), its bricks at 160 above
+// 9,000 (11,648 nodes 15.8 against 17.0 with 40); general hexahedra, of which a CU holds one
+// workgroup, take the smallest of 40, 96 and 160 whose tiles are one round of the CUs (8,625 nodes 18.0 /
+// 18.5 / 22.0 us; 10,125 nodes 33.4 / 18.5 / 22.0; 26,381 nodes 49.7 / 34.5 / 22.0; 0.52M nodes 299 with 96, 222
+// with 160).
 // Models with J2 elements keep one size: the tiles set the order of the solver's dot products, and
 // a yielding point's elastic or plastic branch can follow their last bits.
 // Large brick models that only the implicit integrators take (stiffness-proportional damping,

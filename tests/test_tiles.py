@@ -84,3 +84,36 @@ def test_plan_default_size_of_stretched_tiles():
     # Single-tile and ordinary meshes keep the default size.
     assert plan_tiles(W.layer2d(20, 10, nt=4)[0])["ntiles"] == 1
     assert 192 < plan_tiles(W.layer2d(400, 200, nt=4)[0])["max_own"] <= 400
+
+
+def turned(m: Model, seed: int) -> Model:
+    """Every element numbered from a corner of its own: not corner-unique, as a mesh generator's."""
+    turn = np.random.default_rng(seed).integers(0, 4, m.nelem)
+    conn = m.conn.reshape(m.nelem, -1, 4).copy()
+    for k in range(1, 4):
+        conn[turn == k] = np.roll(conn[turn == k], -k, axis=2)
+    m.conn = np.ascontiguousarray(conn.reshape(m.nelem, -1))
+    return m
+
+
+def distorted(m: Model, h: float) -> Model:
+    inner = np.all((m.coords > m.coords.min(0) + 1e-6) & (m.coords < m.coords.max(0) - 1e-6), axis=1)
+    m.coords[inner] += np.random.default_rng(3).uniform(-0.12 * h, 0.12 * h, (int(inner.sum()), m.ndim))
+    return m
+
+
+def test_plan_default_size_of_the_color_phase_kernel():
+    """Sizes of meshes that are not corner-unique (the tiles hold whole elements' colours)."""
+    for n, size in (((300, 200), 400), ((1100, 1000), 448)):
+        m = turned(W.layer2d(*n, nt=4)[0], 1)
+        assert plan_tiles(m) == plan_tiles(m, size)
+    m = distorted(turned(W.layer2d(400, 300, nt=4)[0], 1), 1.0)
+    assert plan_tiles(m) == plan_tiles(m, 448)
+    for n, size in (((20, 20, 14), 40), ((28, 26, 18), 160)):
+        m = turned(W.halfspace3d(*n, nt=4)[0], 2)
+        assert plan_tiles(m) == plan_tiles(m, size)
+    for n, size in (((20, 20, 14), 40), ((28, 26, 18), 96), ((36, 30, 22), 160)):
+        m = distorted(turned(W.halfspace3d(*n, nt=4)[0], 2), 2.0)
+        assert plan_tiles(m) == plan_tiles(m, size)
+    m = distorted(W.layer2d(400, 300, nt=4)[0], 1.0)
+    assert plan_tiles(m) == plan_tiles(m, 192)
