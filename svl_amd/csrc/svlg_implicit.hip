@@ -109,8 +109,12 @@ struct OpArgs {
 // overlap: the kernel is that chain, not its bytes (2,196 Quad4 nodes 6.9 -> 6.1 us, 64^3 block with 2,188
 // tiles under the learned preconditioner 47 -> 32 us; the partials of J2 tangents as before).
 // The arithmetic and its order stay.
+// Sheared bricks (lumped, elastic): 130 registers without a bound, whose three waves per SIMD are one workgroup of
+// seven waves on a CU; held to 128 two are resident (57^3 block 64.4 -> 50.9 us per iteration).
 template <int DIM, int PATH, int MODE, bool NL, int MOC = 0, bool CM = false, bool PRE = false>
-__global__ __launch_bounds__(512) void k_nm_op(OpArgs a) {
+__global__ __launch_bounds__(512)
+__attribute__((amdgpu_waves_per_eu(DIM == 3 && PATH == 2 && MODE == OP_CG && !NL && !CM ? 4 : 2)))
+void k_nm_op(OpArgs a) {
     constexpr int NEN = Elem<DIM>::nen;
     // J2 Gauss-point loops need the coordinates, except on axis-aligned Hexa8 bricks (the
     // diagonal geometry table), where they run on the corner sums (j2_brick_force).
