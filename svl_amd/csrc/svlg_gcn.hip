@@ -120,7 +120,16 @@ __device__ __forceinline__ void gcn_elem_valu(const GcnArgs &a, int e0, int ne, 
 #pragma unroll
         for (int d = 0; d < DIM; ++d) u[c][d] = double(sXc[lc[c] * DIM + d]);
     tile_elem_force<DIM, PATH>(a.geo, a.th, lc, sCoord, lam, mu, gid, u, f);
-    if (a.cmass) tile_elem_mass<DIM, PATH>(lc, sCoord, a.cmass[e0 + tid], u, f);
+    if (a.cmass) {
+        // The operand once more from LDS: held over the element routine it took up to 48 registers (general
+        // hexahedra spilled 132; learned solve of the distorted 57 x 50 x 48 block 671 -> 378 us per iteration).
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int c = 0; c < NEN; ++c)
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) u[c][d] = double(sXc[lc[c] * DIM + d]);
+        tile_elem_mass<DIM, PATH>(lc, sCoord, a.cmass[e0 + tid], u, f);
+    }
 #pragma unroll
     for (int c = 0; c < NEN; ++c)
         if (lc[c] < nown) {
