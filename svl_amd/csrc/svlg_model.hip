@@ -260,7 +260,8 @@ static TileTraits tile_inputs(const svlg_mesh_desc *d, std::vector<uint8_t> &spe
         if (d->ray_am && d->ray_am[e] != 0.0)
             for (int a = 0; a < nen; ++a) special[d->conn[size_t(e) * nen + a]] = 1;
     }
-    q.implicit_lumped = ak && d->lumped != 0;
+    q.lumped = d->lumped != 0;
+    q.implicit = ak || !q.lumped;
     // Corner-slot scatter needs every (node, corner position) pair to occur at most once.
     std::vector<uint8_t> used(nn, 0);
     for (int e = 0; e < ne && q.corner_unique; ++e)

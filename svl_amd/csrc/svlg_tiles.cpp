@@ -164,13 +164,14 @@ int default_tile_nodes(int ndim, int nnodes, const TileTraits &q) {
     if (ndim == 3) {
         if (nnodes <= 160) return 160;
         if (!q.corner_unique) return nnodes <= 9000 ? 40 : !q.bricks && nnodes <= 23000 ? 96 : 160;
-        if (q.bricks && q.implicit_lumped && nnodes >= 330 * 512) return 330;
+        if (q.bricks && q.implicit && q.lumped && nnodes >= 330 * 512) return 330;
         return nnodes <= 12000 ? 40 : q.bricks ? 160 : 96;
     }
     if (nnodes <= 512) return 512;
     if (nnodes <= 36000) return nnodes <= 8000 ? 64 : 128;
     if (!q.corner_unique) return nnodes <= (q.bricks ? 1000000 : 100000) ? 400 : 448;
-    if (!q.bricks && !q.implicit_lumped && nnodes > 100000) return 192;
+    if (q.implicit) return q.bricks ? 448 : 400;
+    if (!q.bricks && nnodes > 100000) return 192;
     return nnodes <= 1000000 ? 400 : 192;
 }
 

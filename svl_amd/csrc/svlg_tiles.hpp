@@ -25,7 +25,8 @@ struct HostTiles {
 struct TileTraits {
     bool bricks = false;           // the elements are parallelepipeds
     bool j2 = false;               // a J2 element
-    bool implicit_lumped = false;  // stiffness-proportional damping and a lumped mass: implicit integrators only
+    bool lumped = true;            // lumped mass
+    bool implicit = false;         // only implicit integrators take it: consistent mass or stiffness-proportional damping
     bool corner_unique = true;     // no node is the same corner of two elements (else: colour-phase kernel)
 };
 
@@ -52,8 +53,11 @@ struct TileTraits {
 // with 160).
 // Models with J2 elements keep one size: the tiles set the order of the solver's dot products, and
 // a yielding point's elastic or plastic branch can follow their last bits.
-// Large brick models that only the implicit integrators take (stiffness-proportional damping,
-// lumped mass): 330 nodes, whose operator has fewer partials to add up and less to recompute (64^3
+// Models that only the implicit integrators take: quadrilateral bricks above 36,000 nodes 448, the fewest tiles
+// whose elements fit a workgroup (microseconds per iteration, 400 against 448 nodes: 60,501 nodes
+// Jacobi 12.7, 11.7; 0.56M 42.8, 40.7, learned 195, 170; 1.3M with 192 nodes 81.3, 75.3, learned 449, 402;
+// 120,701 nodes learned 76.5, 79.8); other quadrilaterals touch too many elements at 448. Large lumped
+// hexahedral bricks: 330 nodes, whose operator has fewer partials to add up and less to recompute (64^3
 // block: Jacobi 48.9 -> 40.2 us per iteration, the learned preconditioner's operator 32 -> 24.5, its
 // layers 11.7 -> 10.5); below 512 such tiles the CUs need the smaller ones.
 int default_tile_nodes(int ndim, int nnodes, const TileTraits &q);

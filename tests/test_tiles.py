@@ -117,3 +117,18 @@ def test_plan_default_size_of_the_color_phase_kernel():
         assert plan_tiles(m) == plan_tiles(m, size)
     m = distorted(W.layer2d(400, 300, nt=4)[0], 1.0)
     assert plan_tiles(m) == plan_tiles(m, 192)
+
+
+def test_plan_default_size_of_implicit_models():
+    """Consistent mass or stiffness-proportional damping: only implicit integrators take the model."""
+    for change in ("ak", "consistent"):
+        for n, shape, size in (((250, 200), "bricks", 448), ((250, 200), "distorted", 400), ((1100, 1000), "bricks", 448)):
+            m = W.layer2d(*n, nt=4)[0]
+            if shape == "distorted":
+                m = distorted(m, 1.0)
+            if change == "ak":
+                m.ray_ak = np.full(m.nelem, 1e-4)
+                m.ray_am = np.zeros(m.nelem)
+            m.massform_lumped = change != "consistent"
+            assert plan_tiles(m) == plan_tiles(m, size)
+    assert plan_tiles(stretched_layer()) == plan_tiles(stretched_layer(), 192)
