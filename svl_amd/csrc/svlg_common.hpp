@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "svlg.h"
+#include "svlg_tiles.hpp"
 
 namespace svlg {
 
@@ -89,15 +90,13 @@ struct TileSet {
     DevBuf<double> lampad, mupad;
 };
 
-// Deep-halo plan of the multi-step explicit kernel (device copy of HostMulti, svlg_tiles.hpp).
+// Deep-halo plan of the multi-step explicit kernel (device copy, see MultiArrays).
 struct MultiSet {
     int depth = 0;                           // 0: not built, one step per launch
     int ntiles = 0, ns = 0, ne = 0, nu = 0, block = 0;
     size_t lds_bytes = 0;
     DevBuf<uint8_t> slab;                    // holds the arrays below
-    const int32_t *cnt = nullptr, *node = nullptr;
-    const uint16_t *econn = nullptr, *ncor = nullptr, *egeo = nullptr;
-    const double *elam = nullptr, *emu = nullptr;
+    MultiArrays a{};
     DevBuf<double> U[2];                     // output buffers, exchanged with the state's ring
 };
 
@@ -180,15 +179,10 @@ struct Model {
     std::vector<int32_t> h_f2n;       // node-DOF position of every free DOF (made on first use)
     // Multi-step plan: made by the first CentralDifference initialisation of a model that can use it.
     MultiSet multi;
+    MultiInput multi_in;              // kept from the creation until then where a plan may come, else empty
     bool auto_variant = false;        // the kernels were chosen by the library, not by the caller
-    bool multi_tried = false;
     bool captured = false;            // the caller has captured explicit steps since svlg_cd_init
     bool corner_unique = false;       // every (node, corner position) pair belongs to at most one element
-    std::vector<int32_t> h_conn;      // [nelem*nen] connectivity in device numbering
-    std::vector<int32_t> h_own_ptr;   // [ntiles+1]
-    std::vector<uint8_t> h_special;   // [nnodes] device order: nodes that take the general update
-    std::vector<double> h_lam, h_mu;  // [nelem] Lame constants
-    std::vector<uint16_t> h_gid;      // [nelem] geometry-table entry
     // Independent meshes advanced together (one model whose parts share no node): each part
     // keeps its own time step.
     std::vector<double> h_dt_dof;     // [ndofn] time step of every DOF (empty: m.dt everywhere)

@@ -1274,19 +1274,21 @@ static int multi_depth(const Model &m) {
     return d;
 }
 
-// The multi-step plan of a model that steps one tile per workgroup with kernels of the library's choice.
+// Whether the first CentralDifference initialisation looks for a plan: the library chose the kernels, and
+// they are the FP64 step of a corner-unique mesh that this integrator takes.
+bool multi_wanted(const Model &m) {
+    return m.auto_variant && m.corner_unique && m.lumped && !m.has_ak && !m.has_j2 && m.sm_ndofs == 0 &&
+           !m.elem_bf16 && !m.elem_fp32 && multi_depth(m) > 0;
+}
+
+// The plan is set-up: Initialize takes 1.3 ms with it on 20,301 Quad4 nodes (0.2 without), 11.6 ms on 0.55M (0.4), 1.2
+// ms on 8,125 Hexa8 nodes (0.15), the gain of 300, 1,100 and 500 steps. Rings and arrays are made by a
+// few threads, straight into the block that is copied to the device.
 static int multi_build(Model &m) {
     MultiSet &t = m.multi;
-    std::vector<int32_t> conn, own;
-    std::vector<uint8_t> special;
-    std::vector<double> lam, mu;
-    std::vector<uint16_t> gid;
-    conn.swap(m.h_conn);  // used once
-    special.swap(m.h_special);
-    lam.swap(m.h_lam);
-    mu.swap(m.h_mu);
-    gid.swap(m.h_gid);
-    if (!m.auto_variant || !m.corner_unique || m.sm_ndofs > 0 || m.elem_bf16 || m.elem_fp32) return 0;
+    MultiInput in;
+    std::swap(in, m.multi_in);  // used once
+    if (in.conn.empty()) return 0;
     int depth = multi_depth(m);
     const MultiClass *classes = m.ndim == 2 ? kMulti2 : kMulti3;
     const size_t nclasses = m.ndim == 2 ? std::size(kMulti2) : std::size(kMulti3);
@@ -1297,7 +1299,7 @@ static int multi_build(Model &m) {
     size_t lds = 0;
     for (; depth >= least; --depth) {  // the deepest that fits a class and the LDS
         cls = MultiClass{0, 0};
-        if (make_multi(m.nnodes, m.nelem, m.nen, conn.data(), special.data(), m.h_own_ptr, depth, 1024, h))
+        if (make_multi(in, m.nen, depth, 1024, h))
             for (const MultiClass *c = classes; c != classes + nclasses && cls.block == 0; ++c)
                 if (h.ns <= c->block && h.ne <= c->elems) cls = *c;
         lds = (size_t(m.elem_path < 2 ? 2 : 1) * h.ns * m.ndim + size_t(m.nen) * m.ndim * (cls.elems + 1)) *
@@ -1305,9 +1307,6 @@ static int multi_build(Model &m) {
         if (cls.block != 0 && lds <= 160 * 1024) break;
     }
     if (depth < least) return 0;
-    // No element at a corner: the zero column of the class.
-    for (uint16_t &c : h.ncor)
-        if (c == h.ne) c = uint16_t(cls.elems);
     hipStream_t s = m.stream;
     // One allocation and one copy for all of it (each costs tens of microseconds of set-up).
     size_t total = 0;
@@ -1316,23 +1315,17 @@ static int multi_build(Model &m) {
         total += (bytes + 15) / 16 * 16;
         return at;
     };
-    const size_t ne = h.elem.size(), o_cnt = room(h.cnt.size() * 4), o_node = room(h.node.size() * 4),
-                 o_econn = room(h.econn.size() * 2), o_ncor = room(h.ncor.size() * 2), o_egeo = room(ne * 2),
-                 o_lam = room(ne * 8), o_mu = room(ne * 8);
+    const size_t nt = h.tiles.size(), ne = nt * h.ne, o_cnt = room(nt * 2 * (depth + 1) * 4),
+                 o_node = room(nt * h.ns * 4), o_econn = room(ne * m.nen * 2), o_ncor = room(nt * h.nu * m.nen * 2),
+                 o_egeo = room(ne * 2), o_lam = room(ne * 8), o_mu = room(ne * 8);
     std::unique_ptr<uint8_t[]> slab(new uint8_t[total]);
-    std::memcpy(slab.get() + o_cnt, h.cnt.data(), h.cnt.size() * 4);
-    std::memcpy(slab.get() + o_node, h.node.data(), h.node.size() * 4);
-    std::memcpy(slab.get() + o_econn, h.econn.data(), h.econn.size() * 2);
-    std::memcpy(slab.get() + o_ncor, h.ncor.data(), h.ncor.size() * 2);
-    uint16_t *eg = reinterpret_cast<uint16_t *>(slab.get() + o_egeo);
-    double *el = reinterpret_cast<double *>(slab.get() + o_lam), *em = reinterpret_cast<double *>(slab.get() + o_mu);
-    for (size_t i = 0; i < ne; ++i) {
-        const int e = h.elem[i];
-        const double sc = e >= 0 && m.elem_path >= 2 ? m.h_escale[e] : 1.0;
-        el[i] = e >= 0 ? lam[e] * sc : 0.0;
-        em[i] = e >= 0 ? mu[e] * sc : 0.0;
-        eg[i] = e >= 0 && m.elem_path >= 2 ? gid[e] : uint16_t(0);
-    }
+    auto at = [&](uint8_t *base) {
+        return MultiArrays{reinterpret_cast<int32_t *>(base + o_cnt), reinterpret_cast<int32_t *>(base + o_node),
+                           reinterpret_cast<uint16_t *>(base + o_econn), reinterpret_cast<uint16_t *>(base + o_ncor),
+                           reinterpret_cast<uint16_t *>(base + o_egeo), reinterpret_cast<double *>(base + o_lam),
+                           reinterpret_cast<double *>(base + o_mu)};
+    };
+    fill_multi(h, in, cls.elems, at(slab.get()));  // (no element at a corner: the zero column of the class)
     if (t.slab.alloc(total) != hipSuccess || t.U[0].alloc(m.ndofn) != hipSuccess ||
         t.U[1].alloc(m.ndofn) != hipSuccess) {
         t.slab.release();
@@ -1342,14 +1335,8 @@ static int multi_build(Model &m) {
     }
     SVLG_HIP(hipMemcpyAsync(t.slab.p, slab.get(), total, hipMemcpyHostToDevice, s));
     SVLG_HIP(hipStreamSynchronize(s));
-    t.cnt = reinterpret_cast<const int32_t *>(t.slab.p + o_cnt);
-    t.node = reinterpret_cast<const int32_t *>(t.slab.p + o_node);
-    t.econn = reinterpret_cast<const uint16_t *>(t.slab.p + o_econn);
-    t.ncor = reinterpret_cast<const uint16_t *>(t.slab.p + o_ncor);
-    t.egeo = reinterpret_cast<const uint16_t *>(t.slab.p + o_egeo);
-    t.elam = reinterpret_cast<const double *>(t.slab.p + o_lam);
-    t.emu = reinterpret_cast<const double *>(t.slab.p + o_mu);
-    t.ntiles = h.ntiles;
+    t.a = at(t.slab.p);
+    t.ntiles = int(nt);
     t.ns = h.ns;
     t.ne = h.ne;
     t.nu = h.nu;
@@ -1363,8 +1350,6 @@ static int multi_build(Model &m) {
 
 // The plan saves time only: where host or device memory does not hold it, the model steps singly.
 static int multi_setup(Model &m) {
-    if (m.multi_tried) return 0;
-    m.multi_tried = true;
     try {
         return multi_build(m);
     } catch (const std::bad_alloc &) {
@@ -1379,13 +1364,13 @@ static int multi_launch(Model &m, int k, int n, bool last, const RecRef &rec) {
     MultiSet &t = m.multi;
     double *&cur = m.U[m.ring].p, *&prev = m.U[(m.ring + 2) % 3].p, *&old = m.U[(m.ring + 1) % 3].p;
     MultiArgs a;
-    a.cnt = t.cnt;
-    a.node = t.node;
-    a.econn = t.econn;
-    a.ncor = t.ncor;
-    a.egeo = t.egeo;
-    a.elam = t.elam;
-    a.emu = t.emu;
+    a.cnt = t.a.cnt;
+    a.node = t.a.node;
+    a.econn = t.a.econn;
+    a.ncor = t.a.ncor;
+    a.egeo = t.a.egeo;
+    a.elam = t.a.elam;
+    a.emu = t.a.emu;
     a.geo = m.geo.p;
     a.X = m.X.p;
     a.Ucur = cur;

@@ -26,6 +26,7 @@ static thread_local std::string g_error;
 void set_error(const std::string &msg) { g_error = msg; }
 
 int prepare_fused(Model &m);                           // svlg_explicit.hip
+bool multi_wanted(const Model &m);                     // svlg_explicit.hip
 int build_hexa_kmat(Model &m, DevBuf<float> &kmat);    // svlg_gcn.hip
 
 // ---------------------------------------------------------------- kernels
@@ -536,15 +537,6 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     m.h_escale = escale;
     m.auto_variant = req_variant == 0;
     m.corner_unique = corner_unique;
-    m.h_own_ptr = ht.own_ptr;
-    if (m.auto_variant && corner_unique) {
-        m.h_conn = connp;
-        m.h_special.resize(nn);
-        for (int p = 0; p < nn; ++p) m.h_special[p] = special[m.perm[p]];
-        m.h_lam = lam;
-        m.h_mu = mu;
-        m.h_gid = gid;
-    }
     // Tiles.
     {
         TileSet &t = m.tiles;
@@ -764,6 +756,24 @@ static int create_impl(const svlg_mesh_desc *d, const svlg_exec_opts *o, svlg_mo
     if (int rc = drm_setup(m, d)) return fail(rc);
     if (int rc = sm_setup(m, d)) return fail(rc);
     if (int rc = prepare_fused(m)) return fail(rc);
+    if (multi_wanted(m)) {
+        MultiInput &in = m.multi_in;
+        in.special.resize(nn);
+        for (int p = 0; p < nn; ++p) in.special[p] = special[m.perm[p]];
+        if (m.elem_path >= 2) {
+            for (int e = 0; e < ne; ++e) {
+                lam[e] *= escale[e];
+                mu[e] *= escale[e];
+            }
+            in.gid = std::move(gid);
+        }
+        in.lam = std::move(lam);
+        in.mu = std::move(mu);
+        in.conn = std::move(connp);
+        in.n2e_ptr = std::move(n2e_ptr);
+        in.n2e = std::move(n2e);
+        in.own_ptr = std::move(ht.own_ptr);
+    }
     *out = h;
     return 0;
 }

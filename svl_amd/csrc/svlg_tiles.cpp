@@ -187,51 +187,45 @@ void plan_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const
     }
 }
 
-bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8_t *special,
-                const std::vector<int32_t> &own_ptr, int depth, int max_threads, HostMulti &t) {
-    const int nt = int(own_ptr.size()) - 1;
-    std::vector<int32_t> n2e_ptr(nnodes + 1, 0), n2e(size_t(nelem) * nen);
-    for (size_t i = 0; i < size_t(nelem) * nen; ++i) n2e_ptr[conn[i] + 1]++;
-    for (int n = 0; n < nnodes; ++n) n2e_ptr[n + 1] += n2e_ptr[n];
-    {
-        std::vector<int32_t> p(n2e_ptr.begin(), n2e_ptr.end() - 1);
-        for (int e = 0; e < nelem; ++e)
-            for (int a = 0; a < nen; ++a) n2e[p[conn[size_t(e) * nen + a]]++] = e;
-    }
-    struct Tile {
-        std::vector<int32_t> node, elem, ncnt, ecnt;
-        std::vector<uint16_t> conn;
-    };
-    std::vector<Tile> tiles(nt);
-    // Tiles are independent: a few host threads take them in turn (the result does not depend on
-    // which thread built a tile). Threads that the system refuses are done without; an allocation
-    // refused inside a worker ends the plan, not the process.
+// fn(take) on a few host threads, where take() hands out the tiles 0..nt-1 in turn (nt and above: none left): tiles
+// are independent, so the result does not depend on which thread takes one. Threads that the system
+// refuses are done without; a worker that runs out of memory makes the answer false, and the
+// others stop.
+template <class F>
+static bool over_tiles(int nt, F &&fn) {
     const int nthr = std::max(1, std::min({12, int(std::thread::hardware_concurrency()), nt / 16}));
     std::atomic<int> next{0};
-    std::atomic<bool> fits{true};
-    auto run = [&](auto &&fn) {
-        next = 0;
-        auto work = [&] {
-            try {
-                fn();
-            } catch (const std::bad_alloc &) {
-                fits = false;
-            }
-        };
-        std::vector<std::thread> th;
+    std::atomic<bool> ok{true};
+    auto work = [&] {
         try {
-            th.reserve(nthr);
-            for (int i = 1; i < nthr; ++i) th.emplace_back(work);
-        } catch (const std::exception &) {
+            fn([&] { return ok ? next++ : nt; });
+        } catch (const std::bad_alloc &) {
+            ok = false;
         }
-        work();
-        for (auto &x : th) x.join();
     };
-    run([&] {
+    std::vector<std::thread> th;
+    try {
+        th.reserve(nthr);
+        for (int i = 1; i < nthr; ++i) th.emplace_back(work);
+    } catch (const std::exception &) {
+    }
+    work();
+    for (auto &x : th) x.join();
+    return ok;
+}
+
+bool make_multi(const MultiInput &in, int nen, int depth, int max_threads, HostMulti &t) {
+    const int nt = int(in.own_ptr.size()) - 1, nnodes = int(in.special.size()), nelem = int(in.conn.size()) / nen;
+    const int32_t *conn = in.conn.data();
+    t.depth = depth;
+    t.nen = nen;
+    t.tiles.assign(nt, HostMulti::Tile());
+    std::atomic<bool> fits{true};
+    const bool made = over_tiles(nt, [&](auto &&take) {
         std::vector<int32_t> slot(nnodes, -1), seen(nelem, -1);
-        for (int ti; fits && (ti = next++) < nt;) {
-            Tile &q = tiles[ti];
-            for (int32_t n = own_ptr[ti]; n < own_ptr[ti + 1]; ++n) {
+        for (int ti; fits && (ti = take()) < nt;) {
+            HostMulti::Tile &q = t.tiles[ti];
+            for (int32_t n = in.own_ptr[ti]; n < in.own_ptr[ti + 1]; ++n) {
                 slot[n] = int32_t(q.node.size());
                 q.node.push_back(n);
             }
@@ -242,11 +236,13 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
                 // neighbouring LDS words.
                 const size_t end = q.node.size(), e0 = q.elem.size();
                 for (size_t i = from; i < end; ++i)
-                    for (int k = n2e_ptr[q.node[i]]; k < n2e_ptr[q.node[i] + 1]; ++k)
-                        if (seen[n2e[k]] != ti) {
-                            seen[n2e[k]] = ti;
-                            q.elem.push_back(n2e[k]);
+                    for (int k = in.n2e_ptr[q.node[i]]; k < in.n2e_ptr[q.node[i] + 1]; ++k) {
+                        const int e = in.n2e[k] / nen;
+                        if (seen[e] != ti) {
+                            seen[e] = ti;
+                            q.elem.push_back(e);
                         }
+                    }
                 for (size_t i = e0; i < q.elem.size(); ++i)
                     for (int a = 0; a < nen; ++a) {
                         const int32_t n = conn[size_t(q.elem[i]) * nen + a];
@@ -272,38 +268,44 @@ bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8
             for (int32_t n : q.node) slot[n] = -1;
         }
     });
-    if (!fits) return false;
-    t.depth = depth;
-    t.ntiles = nt;
+    if (!made || !fits) return false;
     t.ns = t.ne = t.nu = 1;
-    for (const Tile &q : tiles) {
+    for (const HostMulti::Tile &q : t.tiles) {
         t.ns = std::max(t.ns, q.ncnt[depth]);
         t.ne = std::max(t.ne, q.ecnt[depth - 1]);
         t.nu = std::max(t.nu, q.ncnt[depth - 1]);
     }
-    const int nc = 2 * (depth + 1);
-    t.cnt.assign(size_t(nt) * nc, 0);
-    t.node.assign(size_t(nt) * t.ns, 0);
-    t.elem.assign(size_t(nt) * t.ne, -1);
-    t.econn.assign(size_t(nt) * t.ne * nen, 0);
-    t.ncor.assign(size_t(nt) * t.nu * nen, uint16_t(t.ne));
-    run([&] {
-        for (int ti; fits && (ti = next++) < nt;) {
-            const Tile &q = tiles[ti];
-            for (size_t i = 0; i < q.node.size(); ++i)
-                t.node[size_t(ti) * t.ns + i] = q.node[i] | (special[q.node[i]] ? INT32_MIN : 0);
-            for (int d = 0; d <= depth; ++d) t.cnt[size_t(ti) * nc + d] = q.ncnt[d];
-            for (int d = 0; d < depth; ++d) t.cnt[size_t(ti) * nc + depth + 1 + d] = q.ecnt[d];
-            std::copy(q.elem.begin(), q.elem.end(), t.elem.begin() + size_t(ti) * t.ne);
-            std::copy(q.conn.begin(), q.conn.end(), t.econn.begin() + size_t(ti) * t.ne * nen);
-            for (size_t i = 0; i < q.elem.size(); ++i)
+    return true;
+}
+
+void fill_multi(const HostMulti &t, const MultiInput &in, int none, const MultiArrays &o) {
+    const int nt = int(t.tiles.size()), nc = 2 * (t.depth + 1), nen = t.nen;
+    over_tiles(nt, [&](auto &&take) {
+        for (int ti; (ti = take()) < nt;) {
+            const HostMulti::Tile &q = t.tiles[ti];
+            const size_t nn = q.node.size(), ne = q.elem.size(), n0 = size_t(ti) * t.ns, e0 = size_t(ti) * t.ne;
+            for (int d = 0; d <= t.depth; ++d) o.cnt[size_t(ti) * nc + d] = q.ncnt[d];
+            for (int d = 0; d <= t.depth; ++d)
+                o.cnt[size_t(ti) * nc + t.depth + 1 + d] = d < t.depth ? q.ecnt[d] : 0;
+            for (size_t i = 0; i < nn; ++i) o.node[n0 + i] = q.node[i] | (in.special[q.node[i]] ? INT32_MIN : 0);
+            std::fill(o.node + n0 + nn, o.node + n0 + t.ns, 0);
+            std::copy(q.conn.begin(), q.conn.end(), o.econn + e0 * nen);
+            std::fill(o.econn + (e0 + ne) * nen, o.econn + (e0 + t.ne) * nen, uint16_t(0));
+            for (int i = 0; i < t.ne; ++i) {
+                const int e = i < int(ne) ? q.elem[i] : -1;
+                o.egeo[e0 + i] = e >= 0 && !in.gid.empty() ? in.gid[e] : uint16_t(0);
+                o.elam[e0 + i] = e >= 0 ? in.lam[e] : 0.0;
+                o.emu[e0 + i] = e >= 0 ? in.mu[e] : 0.0;
+            }
+            uint16_t *nc0 = o.ncor + size_t(ti) * t.nu * nen;
+            std::fill(nc0, nc0 + size_t(t.nu) * nen, uint16_t(none));
+            for (size_t i = 0; i < ne; ++i)
                 for (int a = 0; a < nen; ++a) {
                     const int sl = q.conn[i * nen + a];
-                    if (sl < q.ncnt[depth - 1]) t.ncor[(size_t(ti) * t.nu + sl) * nen + a] = uint16_t(i);
+                    if (sl < q.ncnt[t.depth - 1]) nc0[size_t(sl) * nen + a] = uint16_t(i);
                 }
         }
     });
-    return fits;
 }
 
 }  // namespace svlg

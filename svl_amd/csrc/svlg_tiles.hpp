@@ -73,23 +73,44 @@ void make_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const
 void plan_tiles(int ndim, int nnodes, int nelem, int nen, const double *X, const int32_t *conn, const int32_t *color,
                 int ncolors, const uint8_t *special, int tile_nodes, const TileTraits &q, HostTiles &t);
 
+// What the multi-step plan is made from, in device numbering (empty: the model has no plan).
+struct MultiInput {
+    std::vector<int32_t> conn;         // [nelem*nen]
+    std::vector<int32_t> n2e_ptr, n2e; // [nnodes+1], node -> element * nen + corner in ascending element order
+    std::vector<int32_t> own_ptr;      // [ntiles+1]
+    std::vector<uint8_t> special;      // [nnodes] nodes that take the general update
+    std::vector<double> lam, mu;       // [nelem] Lame constants, times the volume scale on the table paths
+    std::vector<uint16_t> gid;         // [nelem] geometry-table entry (empty: none)
+};
+
 // Deep-halo plan of the multi-step explicit kernel over the same tiles: every tile's nodes in
 // rings around its owned nodes (ring d: reached through d layers of elements) and its elements in
 // layers (layer d: touching a node of ring d or nearer), so that a workgroup can advance its owned
-// nodes by up to `depth` steps from one staging. All arrays have fixed strides per tile.
+// nodes by up to `depth` steps from one staging.
 struct HostMulti {
-    int depth = 0, ntiles = 0;
-    int ns = 0, ne = 0, nu = 0;      // strides: staged nodes, elements, updated nodes (rings < depth)
-    std::vector<int32_t> cnt;        // [ntiles][2 (depth + 1)]: nodes up to ring 0..depth, elements up to layer 0..depth-1, 0
-    std::vector<int32_t> node;       // [ntiles][ns] device node, the sign bit set on special nodes
-    std::vector<int32_t> elem;       // [ntiles][ne] element (tag order), -1 padding
-    std::vector<uint16_t> econn;     // [ntiles][ne][nen] staged slot of each corner
-    std::vector<uint16_t> ncor;      // [ntiles][nu][nen] tile element whose corner a the node is; ne: none
+    struct Tile {
+        std::vector<int32_t> node, elem;  // device nodes by ring, elements (tag order) by layer
+        std::vector<int32_t> ncnt, ecnt;  // nodes up to ring 0..depth, elements up to layer 0..depth-1
+        std::vector<uint16_t> conn;       // [elements * nen] staged slot of each corner
+    };
+    int depth = 0, nen = 0;
+    int ns = 0, ne = 0, nu = 0;  // strides: staged nodes, elements, updated nodes (rings < depth)
+    std::vector<Tile> tiles;
 };
 
-// own_ptr, conn and special in device numbering; false if a tile needs more than max_threads
-// staged nodes or elements, or if memory ran out in a worker (in the caller's thread: std::bad_alloc).
-bool make_multi(int nnodes, int nelem, int nen, const int32_t *conn, const uint8_t *special,
-                const std::vector<int32_t> &own_ptr, int depth, int max_threads, HostMulti &t);
+// False if a tile needs more than max_threads staged nodes or elements, or if memory ran out in a
+// worker (in the caller's thread: std::bad_alloc).
+bool make_multi(const MultiInput &in, int nen, int depth, int max_threads, HostMulti &t);
+
+// The plan's arrays as the kernel reads them, all of fixed strides per tile.
+struct MultiArrays {
+    int32_t *cnt;            // [ntiles][2 (depth + 1)]: ncnt, ecnt, 0
+    int32_t *node;           // [ntiles][ns] device node, the sign bit set on special nodes
+    uint16_t *econn;         // [ntiles][ne][nen] staged slot of each corner
+    uint16_t *ncor;          // [ntiles][nu][nen] tile element whose corner a the node is, or none
+    uint16_t *egeo;          // [ntiles][ne]
+    double *elam, *emu;      // [ntiles][ne], 0 on the padding
+};
+void fill_multi(const HostMulti &t, const MultiInput &in, int none, const MultiArrays &o);
 
 }  // namespace svlg
