@@ -222,13 +222,14 @@ int svlg_reactions(svlg_model *m, int32_t n, const int32_t *nodes, int32_t k, do
  * process) --------------------------------------------------------------------------
  * A model whose description is the disjoint union of nparts meshes (node ranges
  * part_node_ptr[p]..part_node_ptr[p+1] in description order, sharing no element) is stepped
- * by one fused launch per step over all of them; each part keeps its own dt (CentralDifference
+ * by launches over all of them, of one step or several (svlg_cd_plan); each part keeps its own dt (CentralDifference
  * coefficients per DOF, CentralDifference.cpp:64-70) and reads sample k of its own load series. */
 int svlg_cd_init_batch(svlg_model *m, int32_t nparts, const int32_t *part_node_ptr /*[nparts+1]*/,
                        const double *dts /*[nparts]*/, double ftol);
-/* Advances nsteps steps from step index k0 by replaying a captured hipGraph of graph_steps
- * fused launches (a multiple of 3; captured on first use, reused while the size and the U ring
- * slot match), the remainder eagerly. Asynchronous like svlg_cd_steps_async. */
+/* Advances nsteps steps from step index k0. Models whose launches cover several steps (svlg_cd_plan)
+ * step as svlg_cd_steps_async does; others replay a captured hipGraph of graph_steps fused launches
+ * (a multiple of 3; captured on first use, reused while the size and the U ring slot match), the
+ * remainder eagerly. Asynchronous like svlg_cd_steps_async. */
 int svlg_cd_graph_steps(svlg_model *m, int32_t k0, int32_t nsteps, int32_t graph_steps);
 /* Autotuner of the node-tile size: builds the model once per candidate tile_nodes (other
  * options from base, may be NULL), times `steps` CentralDifference steps with HIP events and

@@ -239,5 +239,15 @@ def iptr(a: np.ndarray):
     return a.ctypes.data_as(i32p)
 
 
+def state_field(name: str, handle, n: int, i: int) -> np.ndarray:
+    """Field i of (U, V, A) through the state getter `name` (it leaves out the fields whose pointer is
+    null)."""
+    out = np.zeros(n)
+    p = [None, None, None]
+    p[i] = fptr(out)
+    check(getattr(lib(), name)(handle, *p), name)
+    return out
+
+
 def device_count() -> int:
     return int(lib().svlg_device_count())

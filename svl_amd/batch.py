@@ -114,9 +114,10 @@ class BatchedCentralDifference:
                                                  capi.fptr(self.dts), self.ftol), "svlg_cd_init_batch")
 
     def advance(self, k0: int, nsteps: int, graph_steps: int = 0, rec_dofs=None):
-        """nsteps steps from step index k0: replayed hipGraphs of graph_steps launches (0: one
-        eager launch per step; recording forces eager steps). Returns the history of the
-        recorded union free DOFs when rec_dofs is given."""
+        """nsteps steps from step index k0. Models that take several steps per launch (cd_plan) do so in any
+        case; others replay hipGraphs of graph_steps single steps (0: eager single steps, as
+        recording forces). Returns the history of the recorded union free DOFs when rec_dofs is
+        given."""
         if rec_dofs is not None and len(rec_dofs):
             rec = np.ascontiguousarray(rec_dofs, dtype=np.int32)
             hist = np.zeros((nsteps, rec.size))
@@ -139,11 +140,8 @@ class BatchedCentralDifference:
         return U, V, A
 
     def _field(self, i: int, part: int | None) -> np.ndarray:
-        """One of U, V, A (the library leaves out the fields whose pointer is null)."""
-        out = np.zeros(self.mesh.nfree)
-        p = [None, None, None]
-        p[i] = capi.fptr(out)
-        capi.check(capi.lib().svlg_cd_get_state(self.mesh.h, *p), "svlg_cd_get_state")
+        """One of U, V, A of the union, or of one part."""
+        out = capi.state_field("svlg_cd_get_state", self.mesh.h, self.mesh.nfree, i)
         return out if part is None else out[self.free_ptr[part]:self.free_ptr[part + 1]]
 
     def GetDisplacements(self, part: int | None = None) -> np.ndarray:

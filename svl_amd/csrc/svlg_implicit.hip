@@ -60,7 +60,7 @@ struct OpArgs {
     CgParts cg;
     int reduce;           // OP_CG: 1 = iteration `iter` of a solve (beta, stopping test, p.q partials)
     int reset;            // OP_CG, reduce 0: 1 = first launch of a solve, set the solver's scalars
-    double tol2, maxit;   // their values
+    double tol2;          // their tolerance, squared
     int iter;
     // OP_RHS
     const double *U, *V, *A, *mdiag, *cdiag;
@@ -190,7 +190,7 @@ void k_nm_op(OpArgs a) {
     double beta = 0.0;
     if constexpr (!RHS) {
         if (a.reset && blockIdx.x == 0 && tid < SC_COUNT)
-            a.scal[tid] = tid == SC_TOL2 ? a.tol2 : tid == SC_MAXIT ? a.maxit : 0.0;
+            a.scal[tid] = tid == SC_TOL2 ? a.tol2 : 0.0;
         if (a.reduce) {
             if (flag != 0.0) return;
             const int j = a.iter;
@@ -585,11 +585,10 @@ __global__ __launch_bounds__(512) void k_cg_one(OpArgs a, OneArgs o) {
     }
 }
 
-__global__ void k_solver_reset(double *scal, double tol2, double maxit) {
+__global__ void k_solver_reset(double *scal, double tol2) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         for (int i = 0; i < SC_COUNT; ++i) scal[i] = 0.0;
         scal[SC_TOL2] = tol2;
-        scal[SC_MAXIT] = maxit;
     }
 }
 
@@ -1013,7 +1012,7 @@ static int launch_op(Model &m, int mode, const OpArgs &a0) {
 
 // y = Keff x (node-DOF layout) through the CG operator with beta = 0.
 int keff_apply_node(Model &m, const double *x, double *y) {
-    hipLaunchKernelGGL(k_solver_reset, dim3(1), dim3(64), 0, m.stream, m.scal.p, 0.0, 0.0);
+    hipLaunchKernelGGL(k_solver_reset, dim3(1), dim3(64), 0, m.stream, m.scal.p, 0.0);
     OpArgs a = op_args(m);
     a.coef = m.coef_keff.p;
     a.z = x;
@@ -1050,11 +1049,6 @@ static CgParts cg_parts(Model &m, int flexible) {
 
 static size_t cg_parts_size(const Model &m) { return 8 * size_t(m.tiles.ntiles) + 7 * size_t(kVecGrid); }
 
-// Solves Keff x = b (node-DOF layout; x holds the initial guess on entry) by CG with the
-// Jacobi preconditioner (precond = SVLG_PRECOND_JACOBI) or by flexible CG with the learned
-// preconditioner (SVLG_PRECOND_LEARNED; beta = -z.q / p.q, Notay's FCG(1)). Per iteration:
-// one operator launch, one vector launch (plus the preconditioner's); the host polls the
-// done flag every 16 iterations.
 // Launches of CG iteration j, of which the kernels use the parity (so a captured run of iterations
 // that starts at an even one is replayed for any). p ping-pongs: even iterations stage
 // p = z + beta cg_p[1] into cg_p[0], odd ones the reverse.
@@ -1123,6 +1117,11 @@ static int cg_poll(Model &m) {
     return 0;
 }
 
+// Solves Keff x = b (node-DOF layout; x holds the initial guess on entry) by CG with the
+// Jacobi preconditioner (precond = SVLG_PRECOND_JACOBI) or by flexible CG with the learned
+// preconditioner (SVLG_PRECOND_LEARNED; beta = -z.q / p.q, Notay's FCG(1)). Per iteration:
+// one operator launch, one vector launch (plus the preconditioner's), or one launch for both
+// (use_one); the host polls the done flag where the last solve ended and every 16 iterations.
 int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int precond, int *iters, double *relres,
              bool graph) {
     hipStream_t s = m.stream;
@@ -1140,7 +1139,6 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
     a.reduce = 0;
     a.reset = 1;
     a.tol2 = rtol * rtol;
-    a.maxit = double(maxit);
     if (int rc = launch_op(m, OP_CG, a)) return rc;
     a.reset = 0;
     hipLaunchKernelGGL(k_cg_init, dim3(kVecGrid), dim3(kVecBlock), 0, s, n, c, b, m.cg_q.p, m.jac.p, m.cg_r.p,
@@ -1156,7 +1154,7 @@ int cg_solve(Model &m, const double *b, double *x, double rtol, int maxit, int p
     hipGraphExec_t pair = graph && maxit >= 2 ? cg_run_graph(m, c, a, x, 2) : nullptr;
     hipGraphExec_t run8 = pair && maxit >= 8 ? cg_run_graph(m, c, a, x, 8) : nullptr;
     hipGraphExec_t one = pair ? cg_run_graph(m, c, a, x, 1) : nullptr;
-    // The polls copy the scalars into pinned host memory (a direct copy, no staging).
+    // The polls write the scalars into pinned host memory (k_cg_poll).
     if (!m.scal_host && hipHostMalloc((void **)&m.scal_host, sizeof(double) * SC_COUNT) != hipSuccess) {
         m.scal_host = nullptr;
         set_error("hipHostMalloc failed");

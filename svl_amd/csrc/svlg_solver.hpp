@@ -19,7 +19,6 @@ enum {
     SC_DONE,     // 1 once converged
     SC_ITERS,
     SC_TOL2,     // rtol^2
-    SC_MAXIT,
     SC_CNT,      // operator launches of the solve so far: the iteration index (kernels know its parity)
     SC_SEQ,      // host copy only: the poll's number
     SC_ONE,      // one-kernel iterations: r.z and alpha of the even and of the odd iteration before
@@ -145,9 +144,6 @@ __device__ __forceinline__ bool cg_stop_test(const CgParts &c, int j, double *sc
         scal[SC_DONE] = 1.0;
     }
     return done;
-}
-__device__ __forceinline__ double cg_pq(const CgParts &c, int j, double *buf) {
-    return sum_partials(c.pq + size_t(j & 1) * c.ntiles, c.ntiles, 1, buf);
 }
 // (z.r, z.q) of iteration j from the preconditioner partials.
 __device__ __forceinline__ void cg_pre(const CgParts &c, int j, double *buf, double (&o)[2]) {

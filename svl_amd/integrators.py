@@ -212,22 +212,14 @@ class CentralDifference:
                    "svlg_cd_get_state")
         return U, V, A
 
-    def _field(self, i: int) -> np.ndarray:
-        """One of U, V, A (the library leaves out the fields whose pointer is null)."""
-        out = np.zeros(self.mesh.nfree)
-        p = [None, None, None]
-        p[i] = capi.fptr(out)
-        capi.check(capi.lib().svlg_cd_get_state(self.mesh.h, *p), "svlg_cd_get_state")
-        return out
-
     def GetDisplacements(self) -> np.ndarray:
-        return self._field(0)
+        return capi.state_field("svlg_cd_get_state", self.mesh.h, self.mesh.nfree, 0)
 
     def GetVelocities(self) -> np.ndarray:
-        return self._field(1)
+        return capi.state_field("svlg_cd_get_state", self.mesh.h, self.mesh.nfree, 1)
 
     def GetAccelerations(self) -> np.ndarray:
-        return self._field(2)
+        return capi.state_field("svlg_cd_get_state", self.mesh.h, self.mesh.nfree, 2)
 
 
 PRECOND_JACOBI = 0
@@ -305,22 +297,14 @@ class ExtendedNewmarkBeta:
                    "svlg_nm_get_state")
         return U, V, A
 
-    def _field(self, i: int) -> np.ndarray:
-        """One of U, V, A (the library leaves out the fields whose pointer is null)."""
-        out = np.zeros(self.mesh.nfree)
-        p = [None, None, None]
-        p[i] = capi.fptr(out)
-        capi.check(capi.lib().svlg_nm_get_state(self.mesh.h, *p), "svlg_nm_get_state")
-        return out
-
     def GetDisplacements(self) -> np.ndarray:
-        return self._field(0)
+        return capi.state_field("svlg_nm_get_state", self.mesh.h, self.mesh.nfree, 0)
 
     def GetVelocities(self) -> np.ndarray:
-        return self._field(1)
+        return capi.state_field("svlg_nm_get_state", self.mesh.h, self.mesh.nfree, 1)
 
     def GetAccelerations(self) -> np.ndarray:
-        return self._field(2)
+        return capi.state_field("svlg_nm_get_state", self.mesh.h, self.mesh.nfree, 2)
 
 
 class NewmarkBeta(ExtendedNewmarkBeta):

@@ -172,16 +172,8 @@ class PmlNewmark:
                    "svlg_pml_get_state")
         return U, V, A
 
-    def _field(self, i: int):
-        """One of U, V, A (the library leaves out the fields whose pointer is null)."""
-        out = np.zeros(self.nfree)
-        p = [None, None, None]
-        p[i] = capi.fptr(out)
-        capi.check(capi.lib().svlg_pml_get_state(self.h, *p), "svlg_pml_get_state")
-        return out
-
     def GetDisplacements(self):
-        return self._field(0)
+        return capi.state_field("svlg_pml_get_state", self.h, self.nfree, 0)
 
     def set_graph(self, on: bool):
         """Replay the MINRES iterations from a captured hipGraph (default) or launch them eagerly."""
@@ -194,10 +186,10 @@ class PmlNewmark:
         return out
 
     def GetVelocities(self):
-        return self._field(1)
+        return capi.state_field("svlg_pml_get_state", self.h, self.nfree, 1)
 
     def GetAccelerations(self):
-        return self._field(2)
+        return capi.state_field("svlg_pml_get_state", self.h, self.nfree, 2)
 
 
 def soil_column(n_reg: int, n_pml: int, load_series, E=5e7, nu=0.25, rho=2000.0, m=2.0, L=None, R=1e-5,
