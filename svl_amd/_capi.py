@@ -240,9 +240,9 @@ def iptr(a: np.ndarray):
 
 
 def state_field(name: str, handle, n: int, i: int) -> np.ndarray:
-    """Field i of (U, V, A) through the state getter `name` (it leaves out the fields whose pointer is
-    null)."""
-    out = np.zeros(n)
+    """Field i of (U, V, A) through the state getter `name`, which writes every entry (and leaves out the
+    fields whose pointer is null)."""
+    out = np.empty(n)
     p = [None, None, None]
     p[i] = fptr(out)
     check(getattr(lib(), name)(handle, *p), name)
