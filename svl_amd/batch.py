@@ -1,6 +1,6 @@
 """Independent meshes advanced together on one GPU (no SVL counterpart: SVL runs one model per
 process). The meshes are concatenated into one model whose parts share no node; the device
-steps all parts with one fused launch per step (replayed from a captured hipGraph), each
+steps all parts together, several steps per launch or single steps replayed from a captured hipGraph, each
 part with its own time step and load series, and an autotuner picks the node-tile size.
 """
 from __future__ import annotations

@@ -1249,8 +1249,8 @@ static const void *multi_fn(const Model &m) {
 // Steps per launch of the multi-step kernel for this model's tiles (0: single-step kernels).
 // Measured, microseconds per step, single-step kernel against the multi-step kernel:
 //   one tile (231 Quad4 nodes)            4.3 -> 0.80
-//   Quad4, 5,151 nodes, 64-node tiles     5.0 -> 1.37 (depth 6)      20,301 nodes, 128-node tiles  4.4 -> 1.42 (8)
-//   Quad4, 80,601 nodes, 400-node tiles   5.4 -> 2.24 (4)            0.55M nodes, 400-node tiles  13.5 -> 9.6 (4)
+//   Quad4, 5,151 nodes, 64-node tiles     5.0 -> 1.37 (depth 5)      20,301 nodes, 128-node tiles  4.4 -> 1.42 (7)
+//   Quad4, 80,601 nodes, 400-node tiles   5.4 -> 2.24 (5)            0.55M nodes, 400-node tiles  13.5 -> 9.6 (4)
 //   Quad4, 1.77M nodes, 400-node tiles   29.4 -> 31.4 (4)            0.55M nodes, 128-node tiles  13.6 -> 19.9 (4)
 //   distorted Quad4, 100,651 / 114,091 nodes, 252 / 286 tiles  7.5 -> 5.9 / 9.5 -> 10.4 (4), 0.55M nodes  25 -> 31 (4)
 //   Quad4 25 times as wide as high, 400-node tiles, 210,951 / 0.55M nodes  7.4 -> 7.8 / 14.3 -> 14.9 (2)
@@ -1282,7 +1282,7 @@ bool multi_wanted(const Model &m) {
 }
 
 // The plan is set-up: Initialize takes 1.3 ms with it on 20,301 Quad4 nodes (0.2 without), 11.6 ms on 0.55M (0.4), 1.2
-// ms on 8,125 Hexa8 nodes (0.15), the gain of 300, 1,100 and 500 steps. Rings and arrays are made by a
+// ms on 8,125 Hexa8 nodes (0.15), the gain of 300, 2,500 and 500 steps over single steps. Rings and arrays are made by a
 // few threads, straight into the block that is copied to the device.
 static int multi_build(Model &m) {
     MultiSet &t = m.multi;
