@@ -976,10 +976,23 @@ static const void *one_fn(const Model &m) {
 }
 
 // Whether Jacobi solves of the model take the one-kernel iteration. Every tile adds up every tile's
-// three partials, so the line is at the tiles where that costs what the second launch does
-// (microseconds per iteration, two kernels against one: 43 tiles 12.5 -> 8.2, 384 tiles 16.8 ->
-// 13.8, 1,021 tiles 40.2 both, 2,188 tiles 48.9 -> 69.8).
-static bool use_one(const Model &m) { return !m.has_j2 && m.tiles.one_pass && m.tiles.ntiles <= 768; }
+// three partials and forms its halo's z itself, so the line is at the tiles where that costs what the second
+// launch does (microseconds per iteration, two kernels against one):
+//   Hexa8 bricks      384 tiles 17.4 -> 14.5, 488 18.0 -> 15.2, 532 19.4 -> 21.3, 2,188 48.9 -> 69.8
+//   sheared, graded   340 19.9 -> 17.7, 532 27.5 -> 25.5, 587 28.0 -> 26.8; bricks with consistent mass 588 30.1 -> 29.4
+//   general Hexa8     300 19.5 -> 16.1, 725 31.1 -> 29.1, 808 35.5 both; with consistent mass (84 registers spill)
+//                     302 tiles of 40 nodes 28.2 -> 27.1, of 96 nodes 215 24.4 -> 24.6, 522 47.0 -> 53.0
+//   Quad4             490 20.2 -> 16.3, 585 23.8 -> 23.3, 618 24.5 -> 25.3
+//   general Quad4     206 17.0 -> 13.8, 287 21.2 -> 23.3, 703 33.1 -> 37.9; with consistent mass 703 42.8 -> 41.4
+static int one_tiles(const Model &m) {
+    if (m.elem_path == 0) {
+        if (m.ndim == 2) return m.lumped ? 256 : 768;
+        return m.lumped ? 768 : m.tiles.max_own <= 64 ? 512 : 0;
+    }
+    if (m.ndim == 2) return 600;
+    return m.elem_path == 3 && m.lumped ? 512 : 768;
+}
+static bool use_one(const Model &m) { return !m.has_j2 && m.tiles.one_pass && m.tiles.ntiles <= one_tiles(m); }
 
 // One-kernel iteration j (start: the product and sums of z_0 alone, into the halves that iteration 0
 // reads). r, w, s: buffers 0 to 1 on even iterations and back on odd ones.

@@ -168,18 +168,24 @@ def test_newmark_rejects_unsupported_models():
 
 @pytest.mark.parametrize("kind,tile_nodes", [("quad", 448), ("quad", 16), ("quad_consistent", 40), ("hexa", 0),
                                              ("hexa", 16), ("hexa_consistent", 0), ("distorted", 40),
-                                             ("many_tiles", 16), ("many_tiles", 24)])
+                                             ("distorted_consistent", 40), ("distorted_consistent", 100),
+                                             ("quad_distorted", 40), ("quad_distorted", 16),
+                                             ("many_tiles", 16), ("many_tiles", 24), ("many_tiles", 40)])
 def test_cg_iteration_kernels(kind, tile_nodes):
-    """Jacobi solves of the one-kernel iteration (up to 768 tiles) and of the two-kernel one (`many_tiles`
-    with 16 nodes: above): the true residual, recomputed by Keff apply, meets the tolerance up to the
+    """Jacobi solves of the one-kernel iteration and of the two-kernel one (bricks above 512 tiles,
+    quadrilaterals of `quad_distorted` above 256, distorted hexahedra with consistent mass in tiles
+    above 64 nodes): the true residual, recomputed by Keff apply, meets the tolerance up to the
     recurrence's round-off (iterations x eps x the norms' ratio, far below 1e-12 here), a zero right-hand
     side gives zero, and a second solve is bitwise the first."""
     from svl_amd.integrators import LinearSystem
     if kind.startswith("quad"):
-        m, dt, nt = W.realization2d(33, 19, 4, nt=11)
+        m, dt, nt = W.realization2d(*((33, 19) if kind != "quad_distorted" else (80, 60)), 4, nt=11)
+        if kind == "quad_distorted":
+            inner = np.all((m.coords > m.coords.min(0) + 1e-6) & (m.coords < m.coords.max(0) - 1e-6), axis=1)
+            m.coords[inner] += np.random.default_rng(3).uniform(-0.12, 0.12, (int(inner.sum()), 2))
         am, ak = W.rayleigh(0.05, 1.0, 10.0)
         m.ray_am, m.ray_ak = np.full(m.nelem, am), np.full(m.nelem, ak)
-    elif kind == "distorted":
+    elif kind.startswith("distorted"):
         from _meshes import block_model
         m = block_model(9, 8, 7, distort=0.15, seed=2)[0]
     elif kind == "many_tiles":
@@ -188,8 +194,11 @@ def test_cg_iteration_kernels(kind, tile_nodes):
         m, dt, nt = W.block3d_implicit(9, 7, 8, nt=11)
     m.massform_lumped = not kind.endswith("consistent")
     dm = DeviceModel(m, tile_nodes=tile_nodes)
+    ntiles = dm.info()["ntiles"]
     if kind == "many_tiles":
-        assert (dm.info()["ntiles"] > 768) == (tile_nodes == 16)
+        assert (ntiles > 512) == (tile_nodes < 40)
+    if kind == "quad_distorted":
+        assert (ntiles > 256) == (tile_nodes == 16)
     nm = ExtendedNewmarkBeta(dm, 2e-3, rtol=1e-11, maxit=2000)
     nm.Initialize()
     ls = LinearSystem(nm)
